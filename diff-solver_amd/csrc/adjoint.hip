@@ -48,18 +48,20 @@ __device__ __forceinline__ void trace_reverse(const Geo& g, const VBound& b, con
     scatter_face_to<2>(sink, sx, sy, sz, s * mz, g, b);
 }
 
+constexpr int kVjpThreads = 512;   // of both advection reverses
+
 // advect_scalar_vjp_kernel (operators.cu:537-561) for NF fields that share one trace: the
 // velocity adjoint of both fields is summed before it is scattered (the map is linear). A block
 // owns a kSvBX x kSvBY x kSvBZ brick of cells and privatises its scatters as the velocity reverse
 // does: the NF fields' and the three velocity components' adds that land in a window around the
 // brick (halo kSvHalo) are LDS atomics, the rest (long traces, periodic wraps) global atomics; the
-// windows are flushed once.
+// windows are flushed once. The windows hold FP64: see kVjpThreads.
 constexpr int kSvBX = 32, kSvBY = 8, kSvBZ = 2, kSvHalo = 1;
 constexpr int kSwX = kSvBX + 2 * kSvHalo + 1, kSwY = kSvBY + 2 * kSvHalo + 1, kSwZ = kSvBZ + 2 * kSvHalo + 1;
 constexpr int kSw = kSwX * kSwY * kSwZ;   // per target array: velocity components 0-2, fields 3-4
 
 struct ScalarBrickSink {
-    float* win;        // LDS, 5 * kSw
+    double* win;       // LDS, 5 * kSw
     int ox, oy, oz;    // coordinates of window element (0, 0, 0)
     F3 va;
     float* s0;
@@ -68,23 +70,23 @@ struct ScalarBrickSink {
     __device__ __forceinline__ void add(int x, int y, int z, uint32_t i, float value) const {
         const unsigned lx = (unsigned)(x - ox), ly = (unsigned)(y - oy), lz = (unsigned)(z - oz);
         if (lx < (unsigned)kSwX && ly < (unsigned)kSwY && lz < (unsigned)kSwZ)
-            __hip_atomic_fetch_add(win + W * kSw + ((int)lz * kSwY + (int)ly) * kSwX + (int)lx, value, __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(win + W * kSw + ((int)lz * kSwY + (int)ly) * kSwX + (int)lx, (double)value, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         else
             atomicAdd((W < 3 ? va.p[W < 3 ? W : 0] : W == 3 ? s0 : s1) + i, value);
     }
 };
 
-// 4 waves per SIMD (registers capped at 128, the rest spilled), the most its 38.5 KB of LDS allows:
-// the dependent gathers of the trace want waves more than registers.
+// One cell per thread; 4 waves per SIMD (registers capped at 128, the rest spilled), the most two
+// blocks' 77 KB of LDS allow: the dependent gathers of the trace want waves more than registers.
 template <int NF, bool HasSolids>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void advect_scalar_vjp_kernel(Geo g, const VBound* __restrict__ vbp, const SBound* __restrict__ sb0p,
+__global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))) void advect_scalar_vjp_kernel(Geo g, const VBound* __restrict__ vbp, const SBound* __restrict__ sb0p,
                                                                 const SBound* __restrict__ sb1p, const uint8_t* __restrict__ mask,
                                                                 const float* __restrict__ src0, const float* __restrict__ src1, Vel3 u,
                                                                 const float* __restrict__ oa0, const float* __restrict__ oa1,
                                                                 float* src_adj0, float* src_adj1, F3 va) {
-    static_assert(kSvBX * kSvBY == 256, "one plane of the brick per pass of the block");
-    __shared__ float win[5 * kSw];
+    static_assert(kSvBX * kSvBY * kSvBZ == kVjpThreads, "one cell of the brick per thread");
+    __shared__ double win[5 * kSw];
     const VBound& vb = *vbp;
     const SBound& sb0 = *sb0p;
     const SBound& sb1 = *sb1p;
@@ -93,18 +95,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void a
     const uint32_t lb = xcd_block();
     if (lb >= bricks) return;   // padding blocks of the XCD-rounded grid (whole block)
     const int x0 = (int)(lb % nbx) * kSvBX, y0 = (int)((lb / nbx) % nby) * kSvBY, z0 = (int)(lb / (nbx * nby)) * kSvBZ;
-    for (int k = threadIdx.x; k < 5 * kSw; k += blockDim.x) win[k] = 0.0f;
+    for (int k = threadIdx.x; k < 5 * kSw; k += blockDim.x) win[k] = 0.0;
     __syncthreads();
     const ScalarBrickSink sink{win, x0 - kSvHalo, y0 - kSvHalo, z0 - kSvHalo, va, src_adj0, NF == 2 ? src_adj1 : src_adj0};
-    const int x = x0 + (int)(threadIdx.x % kSvBX), y = y0 + (int)(threadIdx.x / kSvBX);
-    for (int f = 0; f < kSvBZ; ++f) {
-        const int z = z0 + f;
-        if (x >= g.nx || y >= g.ny || z >= g.nz) continue;
+    const int x = x0 + (int)(threadIdx.x % kSvBX), y = y0 + (int)(threadIdx.x / kSvBX) % kSvBY,
+              z = z0 + (int)threadIdx.x / (kSvBX * kSvBY);
+    auto cell = [&] {
+        if (x >= g.nx || y >= g.ny || z >= g.nz) return;
         const uint32_t i = cidx(g, x, y, z);
-        if (HasSolids && mask[i] != 0) continue;
+        if (HasSolids && mask[i] != 0) return;
         const float a0 = oa0[i];
         const float a1 = NF == 2 ? oa1[i] : 0.0f;
-        if (a0 == 0.0f && a1 == 0.0f) continue;
+        if (a0 == 0.0f && a1 == 0.0f) return;
         const float sx = (x + 0.5f) * g.h, sy = (y + 0.5f) * g.h, sz = (z + 0.5f) * g.h;
         Sample mid[3];
         const TraceOut t = trace_rk2<HasSolids, true>(sx, sy, sz, u, mask, g, vb, mid);
@@ -120,10 +122,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void a
         }
         const float v1x = -(t.dx * g.dt) * gx, v1y = -(t.dy * g.dt) * gy, v1z = -(t.dz * g.dt) * gz;
         trace_reverse(g, vb, sink, sx, sy, sz, t, mid, v1x, v1y, v1z);
-    }
+    };
+    cell();
     __syncthreads();
     for (int k = threadIdx.x; k < 5 * kSw; k += blockDim.x) {
-        const float v = win[k];
+        const float v = (float)win[k];
         if (v == 0.0f) continue;
         const int W = k / kSw, r = k - W * kSw;
         const int wx = x0 - kSvHalo + r % kSwX, wy = y0 - kSvHalo + (r / kSwX) % kSwY, wz = z0 - kSvHalo + r / (kSwX * kSwY);
@@ -144,12 +147,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void a
 // move a few cells at most, so their 56 scatters per face land in a small box around the brick.
 // Scatters inside the box (brick plus a halo of kVjpHalo faces, each component) are LDS atomics;
 // those outside it (long traces, periodic wraps) stay global atomics. The box is flushed once.
+//
+// The windows hold FP64. An LDS FP32 add serialises its lanes (193 cycles per wave and CU, measured
+// with conflict-free addresses; the integer add takes 5.5, the FP64 add 9.3), and these scatters
+// bound both reverse kernels: with FP64 windows the velocity reverse of one axis went from 455 to
+// 230-310 us and the scalar reverse from 685 to 448 us at 128^3, with sums that no longer round
+// per add. The windows are twice as large, so blocks of 512 threads (not 256) share one: two blocks
+// and 4 waves per SIMD per CU, as with FP32.
 constexpr int kVjpBX = 32, kVjpBY = 8, kVjpBZ = 4, kVjpHalo = 1;
+constexpr int kVjpPlanes = kVjpThreads / (kVjpBX * kVjpBY);   // brick planes handled at once
 constexpr int kWinX = kVjpBX + 2 * kVjpHalo + 1, kWinY = kVjpBY + 2 * kVjpHalo + 1, kWinZ = kVjpBZ + 2 * kVjpHalo + 1;
 constexpr int kWin = kWinX * kWinY * kWinZ;   // per component
 
 struct WindowSink {
-    float* win;        // LDS, 3 * kWin
+    double* win;       // LDS, 3 * kWin
     int ox, oy, oz;    // face coordinates of window element (0, 0, 0)
     F3 va;
     template <int B>
@@ -158,7 +169,7 @@ struct WindowSink {
         // workgroup scope for the LDS add: it keeps the two atomics distinct (merged into one
         // atomic on a selected pointer they would both become flat atomics)
         if (lx < (unsigned)kWinX && ly < (unsigned)kWinY && lz < (unsigned)kWinZ)
-            __hip_atomic_fetch_add(win + B * kWin + ((int)lz * kWinY + (int)ly) * kWinX + (int)lx, value, __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(win + B * kWin + ((int)lz * kWinY + (int)ly) * kWinX + (int)lx, (double)value, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         else
             atomicAdd(va.p[B] + i, value);
@@ -188,11 +199,11 @@ __device__ __forceinline__ bool start_gatherable(const Geo& g, uint32_t per, int
     return ok;
 }
 
-// 4 waves per SIMD (registers capped at 128, the rest spilled), the most its 32 KB window allows.
+// 4 waves per SIMD (registers capped at 128, the rest spilled), the most two blocks' 65 KB windows allow.
 template <int A, bool HasSolids, bool GatherStart>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void advect_velocity_vjp_kernel(Geo g, const VBound* __restrict__ bp, const uint8_t* __restrict__ mask,
+__global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))) void advect_velocity_vjp_kernel(Geo g, const VBound* __restrict__ bp, const uint8_t* __restrict__ mask,
                                                                   Vel3 u, const float* __restrict__ oa, F3 va, F3 start, uint32_t per) {
-    __shared__ float win[3 * kWin];
+    __shared__ double win[3 * kWin];
     const VBound& b = *bp;
     int nbx, nby;
     const uint32_t bricks = vjp_bricks(g, A, nbx, nby);
@@ -201,12 +212,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void a
     const int x0 = (int)(lb % (uint32_t)nbx) * kVjpBX;
     const int y0 = (int)((lb / (uint32_t)nbx) % (uint32_t)nby) * kVjpBY;
     const int z0 = (int)(lb / ((uint32_t)nbx * nby)) * kVjpBZ;
-    for (int i = threadIdx.x; i < 3 * kWin; i += blockDim.x) win[i] = 0.0f;
+    for (int i = threadIdx.x; i < 3 * kWin; i += blockDim.x) win[i] = 0.0;
     __syncthreads();
     const WindowSink sink{win, x0 - kVjpHalo, y0 - kVjpHalo, z0 - kVjpHalo, va};
     const int ex = ext(g, A, 0), ey = ext(g, A, 1), ez = ext(g, A, 2);
-    const int x = x0 + (int)(threadIdx.x % kVjpBX), y = y0 + (int)(threadIdx.x / kVjpBX);
-    for (int f = 0; f < kVjpBZ; ++f) {
+    const int x = x0 + (int)(threadIdx.x % kVjpBX), y = y0 + (int)(threadIdx.x / kVjpBX) % kVjpBY;
+    for (int f = (int)threadIdx.x / (kVjpBX * kVjpBY); f < kVjpBZ; f += kVjpPlanes) {
         const int z = z0 + f;
         if (x >= ex || y >= ey || z >= ez) continue;
         const uint32_t fi = fidx(g, A, x, y, z);
@@ -246,7 +257,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void a
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 3 * kWin; i += blockDim.x) {
-        const float v = win[i];
+        const float v = (float)win[i];
         if (v == 0.0f) continue;
         const int B = i / kWin, r = i - B * kWin;
         const int wx = x0 - kVjpHalo + r % kWinX, wy = y0 - kVjpHalo + (r / kWinX) % kWinY, wz = z0 - kVjpHalo + r / (kWinX * kWinY);
@@ -568,18 +579,18 @@ void launch_advect_scalar_vjp(ds_context* c, int nf, int first_field, const floa
     const uint32_t G = (uint32_t)((bricks + 7) & ~7ull);
     if (nf == 2) {
         if (c->has_solids)
-            advect_scalar_vjp_kernel<2, true><<<G, kBlock, 0, c->stream>>>(c->geo, c->d_vb, c->d_db, c->d_tb, c->mask, src0, src1, v, oa0, oa1, sa0,
+            advect_scalar_vjp_kernel<2, true><<<G, kVjpThreads, 0, c->stream>>>(c->geo, c->d_vb, c->d_db, c->d_tb, c->mask, src0, src1, v, oa0, oa1, sa0,
                                                                           sa1, va);
         else
-            advect_scalar_vjp_kernel<2, false><<<G, kBlock, 0, c->stream>>>(c->geo, c->d_vb, c->d_db, c->d_tb, c->mask, src0, src1, v, oa0, oa1,
+            advect_scalar_vjp_kernel<2, false><<<G, kVjpThreads, 0, c->stream>>>(c->geo, c->d_vb, c->d_db, c->d_tb, c->mask, src0, src1, v, oa0, oa1,
                                                                            sa0, sa1, va);
     } else {
         const SBound* b0 = first_field == 0 ? c->d_db : c->d_tb;
         if (c->has_solids)
-            advect_scalar_vjp_kernel<1, true><<<G, kBlock, 0, c->stream>>>(c->geo, c->d_vb, b0, b0, c->mask, src0, src0, v, oa0, oa0, sa0, sa0,
+            advect_scalar_vjp_kernel<1, true><<<G, kVjpThreads, 0, c->stream>>>(c->geo, c->d_vb, b0, b0, c->mask, src0, src0, v, oa0, oa0, sa0, sa0,
                                                                           va);
         else
-            advect_scalar_vjp_kernel<1, false><<<G, kBlock, 0, c->stream>>>(c->geo, c->d_vb, b0, b0, c->mask, src0, src0, v, oa0, oa0, sa0,
+            advect_scalar_vjp_kernel<1, false><<<G, kVjpThreads, 0, c->stream>>>(c->geo, c->d_vb, b0, b0, c->mask, src0, src0, v, oa0, oa0, sa0,
                                                                            sa0, va);
     }
     check_launch("advect_scalar_vjp_kernel");
@@ -605,14 +616,14 @@ void launch_advect_velocity_vjp(ds_context* c, CF3 u, CF3 oa, F3 va) {
         const F3 st{{c->vjp_start[A][0], c->vjp_start[A][1], c->vjp_start[A][2]}};
         if (gather) {
             if (c->has_solids)
-                advect_velocity_vjp_kernel<A, true, true><<<G, kBlock, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
+                advect_velocity_vjp_kernel<A, true, true><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
             else
-                advect_velocity_vjp_kernel<A, false, true><<<G, kBlock, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
+                advect_velocity_vjp_kernel<A, false, true><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
         } else {
             if (c->has_solids)
-                advect_velocity_vjp_kernel<A, true, false><<<G, kBlock, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
+                advect_velocity_vjp_kernel<A, true, false><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
             else
-                advect_velocity_vjp_kernel<A, false, false><<<G, kBlock, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
+                advect_velocity_vjp_kernel<A, false, false><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
         }
         if (e0 && e1) {
             DS_HIP(hipEventRecord(e1, c->stream));
