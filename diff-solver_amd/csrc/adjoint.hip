@@ -19,20 +19,26 @@ namespace ds {
 
 namespace {
 
-// Sink of the three velocity-adjoint components: plain global atomics.
-struct VelSink {
-    F3 va;
-    template <int B>
-    __device__ __forceinline__ void add(int, int, int, uint32_t i, float value) const { atomicAdd(va.p[B] + i, value); }
-};
+// Adds of a whole interior stencil into an LDS window of X x Y x Z doubles when its 8 points lie in
+// it, its lower corner at window coordinates (lx, ly, lz): one address, constant offsets.
+template <int X, int Y, int Z>
+__device__ __forceinline__ bool window_add8(double* win, int lx, int ly, int lz, float adj, const float (&a)[8]) {
+    if ((unsigned)lx >= (unsigned)(X - 1) || (unsigned)ly >= (unsigned)(Y - 1) || (unsigned)lz >= (unsigned)(Z - 1)) return false;
+    double* p = win + (lz * Y + ly) * X + lx;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        __hip_atomic_fetch_add(p + ((k >> 2) * Y + ((k >> 1) & 1)) * X + (k & 1), (double)(adj * a[k]), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    return true;
+}
 
-// Reverse of trace_rk2 + final sample (operators.cu:422-438 / 544-560): given the adjoint of the
-// trace end point (pbx, pby, pbz) = -deriv * dt * grad(sample) * out_adj, scatter through the
-// midpoint and start samples of the velocity; mid: the velocity samples at the midpoint with their
-// gradients (from trace_rk2<.., true>).
-template <typename Sink>
-__device__ __forceinline__ void trace_reverse(const Geo& g, const VBound& b, const Sink& sink, float sx, float sy, float sz,
-                                              const TraceOut& t, const Sample (&mid)[3], float v1x, float v1y, float v1z) {
+// Reverse of trace_rk2 + final sample (operators.cu:422-438 / 544-560) from lattice point (x, y, z)
+// of L: given the adjoint of the trace end point (v1x, v1y, v1z) = -deriv * dt * grad(sample) *
+// out_adj, scatter through the midpoint and start samples of the velocity; mid: the velocity samples
+// at the midpoint with their gradients (from trace_rk2<.., true>).
+template <int L, typename Sink>
+__device__ __forceinline__ void trace_reverse(const Geo& g, const VBound& b, const Sink& sink, int x, int y, int z, const TraceOut& t,
+                                              const Sample (&mid)[3], float v1x, float v1y, float v1z) {
     const Sample& m0 = mid[0];
     const Sample& m1 = mid[1];
     const Sample& m2 = mid[2];
@@ -43,9 +49,9 @@ __device__ __forceinline__ void trace_reverse(const Geo& g, const VBound& b, con
     const float my = m0.gy * v1x + m1.gy * v1y + m2.gy * v1z;
     const float mz = m0.gz * v1x + m1.gz * v1y + m2.gz * v1z;
     const float s = -0.5f * g.dt;
-    scatter_face_to<0>(sink, sx, sy, sz, s * mx, g, b);
-    scatter_face_to<1>(sink, sx, sy, sz, s * my, g, b);
-    scatter_face_to<2>(sink, sx, sy, sz, s * mz, g, b);
+    scatter_start<L, 0>(sink, x, y, z, s * mx, g, b);
+    scatter_start<L, 1>(sink, x, y, z, s * my, g, b);
+    scatter_start<L, 2>(sink, x, y, z, s * mz, g, b);
 }
 
 constexpr int kVjpThreads = 512;   // of both advection reverses
@@ -74,6 +80,10 @@ struct ScalarBrickSink {
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         else
             atomicAdd((W < 3 ? va.p[W < 3 ? W : 0] : W == 3 ? s0 : s1) + i, value);
+    }
+    template <int W>
+    __device__ __forceinline__ bool window8(int x, int y, int z, float adj, const float (&a)[8]) const {
+        return window_add8<kSwX, kSwY, kSwZ>(win + W * kSw, x - ox, y - oy, z - oz, adj, a);
     }
 };
 
@@ -107,9 +117,8 @@ __global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))
         const float a0 = oa0[i];
         const float a1 = NF == 2 ? oa1[i] : 0.0f;
         if (a0 == 0.0f && a1 == 0.0f) return;
-        const float sx = (x + 0.5f) * g.h, sy = (y + 0.5f) * g.h, sz = (z + 0.5f) * g.h;
         Sample mid[3];
-        const TraceOut t = trace_rk2<HasSolids, true>(sx, sy, sz, u, mask, g, vb, mid);
+        const TraceOut t = trace_rk2<3, HasSolids, true>(x, y, z, u, mask, g, vb, mid);
         const Sample s0 = sample_scalar<true>(src0, t.px, t.py, t.pz, g, sb0);
         scatter_scalar_to<3>(sink, t.px, t.py, t.pz, a0, g, sb0);
         float gx = s0.gx * a0, gy = s0.gy * a0, gz = s0.gz * a0;
@@ -121,7 +130,7 @@ __global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))
             gz += s1.gz * a1;
         }
         const float v1x = -(t.dx * g.dt) * gx, v1y = -(t.dy * g.dt) * gy, v1z = -(t.dz * g.dt) * gz;
-        trace_reverse(g, vb, sink, sx, sy, sz, t, mid, v1x, v1y, v1z);
+        trace_reverse<3>(g, vb, sink, x, y, z, t, mid, v1x, v1y, v1z);
     };
     cell();
     __syncthreads();
@@ -174,6 +183,10 @@ struct WindowSink {
         else
             atomicAdd(va.p[B] + i, value);
     }
+    template <int B>
+    __device__ __forceinline__ bool window8(int x, int y, int z, float adj, const float (&a)[8]) const {
+        return window_add8<kWinX, kWinY, kWinZ>(win + B * kWin, x - ox, y - oy, z - oz, adj, a);
+    }
 };
 
 __device__ __forceinline__ uint32_t vjp_bricks(const Geo& g, int A, int& nbx, int& nby) {
@@ -182,27 +195,10 @@ __device__ __forceinline__ uint32_t vjp_bricks(const Geo& g, int A, int& nbx, in
     return (uint32_t)nbx * nby * ((ext(g, A, 2) + kVjpBZ - 1) / kVjpBZ);
 }
 
-// The start point of a face's trace is the face itself, so the trace reverse's last three scatters
-// (the start sample's adjoint, trace_reverse) have a fixed stencil: with a power-of-two cell size
-// the component A corner is the face (weight 1) and a component B != A has the four B-faces
-// {a - 1, a} x {b, b + 1} x {c} (along A, B and the third axis; weight 1/4 each). A face whose
-// stencil needs no boundary value and no periodic mapping (start_gatherable) leaves those values in
-// `start` instead of scattering them, and start_gather_kernel (after the three axes) adds them to
-// each target face as a gather: 9 of the about 41 LDS atomics per face, which bound the kernel.
-template <int A>
-__device__ __forceinline__ bool start_gatherable(const Geo& g, uint32_t per, int x, int y, int z) {
-    const int c[3]{x, y, z}, n[3]{g.nx, g.ny, g.nz};
-    bool ok = c[A] >= 1 && c[A] <= n[A] - 1;
-#pragma unroll
-    for (int B = 0; B < 3; ++B)
-        if (B != A && (per & (1u << B))) ok = ok && c[B] + 1 < n[B];
-    return ok;
-}
-
 // 4 waves per SIMD (registers capped at 128, the rest spilled), the most two blocks' 65 KB windows allow.
-template <int A, bool HasSolids, bool GatherStart>
+template <int A, bool HasSolids>
 __global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))) void advect_velocity_vjp_kernel(Geo g, const VBound* __restrict__ bp, const uint8_t* __restrict__ mask,
-                                                                  Vel3 u, const float* __restrict__ oa, F3 va, F3 start, uint32_t per) {
+                                                                  Vel3 u, const float* __restrict__ oa, F3 va) {
     __shared__ double win[3 * kWin];
     const VBound& b = *bp;
     int nbx, nby;
@@ -222,38 +218,12 @@ __global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))
         if (x >= ex || y >= ey || z >= ez) continue;
         const uint32_t fi = fidx(g, A, x, y, z);
         const float a = oa[fi];
-        const bool gather = GatherStart && start_gatherable<A>(g, per, x, y, z);
-        float st[3]{0.0f, 0.0f, 0.0f};   // the start point's adjoints, gathered later
-        if (a != 0.0f) {
-            const float sx = (x + (A == 0 ? 0.0f : 0.5f)) * g.h;
-            const float sy = (y + (A == 1 ? 0.0f : 0.5f)) * g.h;
-            const float sz = (z + (A == 2 ? 0.0f : 0.5f)) * g.h;
-            Sample mid[3];
-            const TraceOut t = trace_rk2<HasSolids, true>(sx, sy, sz, u, mask, g, b, mid);
-            const Sample s = sample_face<A, true>(u.u[A], t.px, t.py, t.pz, g, b);
-            scatter_face_to<A>(sink, t.px, t.py, t.pz, a, g, b);
-            const float v1x = -(t.dx * g.dt) * (s.gx * a), v1y = -(t.dy * g.dt) * (s.gy * a), v1z = -(t.dz * g.dt) * (s.gz * a);
-            // trace_reverse, with the start point's three adjoints either kept for the gather or
-            // scattered here
-            scatter_face_to<0>(sink, t.mx, t.my, t.mz, v1x, g, b);
-            scatter_face_to<1>(sink, t.mx, t.my, t.mz, v1y, g, b);
-            scatter_face_to<2>(sink, t.mx, t.my, t.mz, v1z, g, b);
-            const float sc = -0.5f * g.dt;
-            st[0] = sc * (mid[0].gx * v1x + mid[1].gx * v1y + mid[2].gx * v1z);
-            st[1] = sc * (mid[0].gy * v1x + mid[1].gy * v1y + mid[2].gy * v1z);
-            st[2] = sc * (mid[0].gz * v1x + mid[1].gz * v1y + mid[2].gz * v1z);
-            if (!gather) {
-                scatter_face_to<0>(sink, sx, sy, sz, st[0], g, b);
-                scatter_face_to<1>(sink, sx, sy, sz, st[1], g, b);
-                scatter_face_to<2>(sink, sx, sy, sz, st[2], g, b);
-                st[0] = st[1] = st[2] = 0.0f;
-            }
-        }
-        if (GatherStart) {
-            start.p[0][fi] = st[0];
-            start.p[1][fi] = st[1];
-            start.p[2][fi] = st[2];
-        }
+        if (a == 0.0f) continue;
+        Sample mid[3];
+        const TraceOut t = trace_rk2<A, HasSolids, true>(x, y, z, u, mask, g, b, mid);
+        const Sample s = sample_face<A, true>(u.u[A], t.px, t.py, t.pz, g, b);
+        scatter_face_to<A>(sink, t.px, t.py, t.pz, a, g, b);
+        trace_reverse<A>(g, b, sink, x, y, z, t, mid, -(t.dx * g.dt) * (s.gx * a), -(t.dy * g.dt) * (s.gy * a), -(t.dz * g.dt) * (s.gz * a));
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 3 * kWin; i += blockDim.x) {
@@ -266,45 +236,6 @@ __global__ __launch_bounds__(kVjpThreads) __attribute__((amdgpu_waves_per_eu(4))
         float* dst = B == 0 ? va.p[0] : B == 1 ? va.p[1] : va.p[2];
         atomicAdd(dst + fidx(g, B, wx, wy, wz), v);
     }
-}
-
-// The transpose of the start stencils of the three axes' faces, for every face of component B (one
-// thread per face of the three components, concatenated), after the three axes' reverse kernels:
-// adds the gathered start adjoints. start[A][B]: component B's start adjoints of axis A's faces.
-struct StartAdj {
-    const float* p[3][3];
-};
-__global__ __launch_bounds__(256) void start_gather_kernel(Geo g, uint32_t per, StartAdj start, F3 va) {
-    const uint32_t f = xcd_block() * blockDim.x + threadIdx.x;
-    if (f >= g.foff[3]) return;
-    for_face(g, f, [&]<int B>(uint32_t local) {
-        int t[3];
-        decode_face_axis<B>(g, local, t[0], t[1], t[2]);
-        const int n[3]{g.nx, g.ny, g.nz};
-        float s = 0.0f;
-        auto from_axis = [&]<int A>() {
-            if (A == B) {
-                if (start_gatherable<A>(g, per, t[0], t[1], t[2])) s += start.p[A][A][local];
-            } else {
-#pragma unroll
-                for (int da = 0; da < 2; ++da)
-#pragma unroll
-                    for (int db = -1; db <= 0; ++db) {
-                        int q[3]{t[0], t[1], t[2]};
-                        q[A] += da;
-                        q[B] += db;
-                        // an axis-A face: its own axis has n + 1 faces, the others n
-                        if (q[A] < 0 || q[A] > n[A] || q[B] < 0 || q[B] >= n[B]) continue;
-                        if (!start_gatherable<A>(g, per, q[0], q[1], q[2])) continue;
-                        s += 0.25f * start.p[A][B][fidx(g, A, q[0], q[1], q[2])];
-                    }
-            }
-        };
-        from_axis.template operator()<0>();
-        from_axis.template operator()<1>();
-        from_axis.template operator()<2>();
-        if (s != 0.0f) va.p[B][local] += s;
-    });
 }
 
 // constrained_boundary, operators.cu:452-458
@@ -599,11 +530,6 @@ void launch_advect_scalar_vjp(ds_context* c, int nf, int first_field, const floa
 void launch_advect_velocity_vjp(ds_context* c, CF3 u, CF3 oa, F3 va) {
     const Vel3 v{{u.p[0], u.p[1], u.p[2]}};
     const Geo& g = c->geo;
-    uint32_t per = 0;   // bit d: axis d of the velocity boundary is periodic (vperiodic)
-    for (int d = 0; d < 3; ++d)
-        if (c->vb.modes[2 * d] == 3u && c->vb.modes[2 * d + 1] == 3u) per |= 1u << d;
-    // the start stencils are gathered when the context holds the buffers and the fractions are exact
-    const bool gather = c->vjp_start[0][0] != nullptr && g.h_pow2;
     // profiling: every sample_every-th call has each axis launch bracketed by HIP events
     Profiler& prof = c->profiler;
     const bool sample = prof.every && (prof.launches[6] / 3) % prof.every == 0 && prof.used + 6 <= 6000;
@@ -613,18 +539,8 @@ void launch_advect_velocity_vjp(ds_context* c, CF3 u, CF3 oa, F3 va) {
         const uint32_t G = (uint32_t)((bricks + 7) & ~7ull);
         hipEvent_t e0 = sample ? prof.take() : nullptr, e1 = sample ? prof.take() : nullptr;
         if (e0) DS_HIP(hipEventRecord(e0, c->stream));
-        const F3 st{{c->vjp_start[A][0], c->vjp_start[A][1], c->vjp_start[A][2]}};
-        if (gather) {
-            if (c->has_solids)
-                advect_velocity_vjp_kernel<A, true, true><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
-            else
-                advect_velocity_vjp_kernel<A, false, true><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
-        } else {
-            if (c->has_solids)
-                advect_velocity_vjp_kernel<A, true, false><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
-            else
-                advect_velocity_vjp_kernel<A, false, false><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va, st, per);
-        }
+        if (c->has_solids) advect_velocity_vjp_kernel<A, true><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va);
+        else advect_velocity_vjp_kernel<A, false><<<G, kVjpThreads, 0, c->stream>>>(g, c->d_vb, c->mask, v, oa.p[A], va);
         if (e0 && e1) {
             DS_HIP(hipEventRecord(e1, c->stream));
             prof.recs.push_back({6, e0, e1});
@@ -634,12 +550,6 @@ void launch_advect_velocity_vjp(ds_context* c, CF3 u, CF3 oa, F3 va) {
     launch.template operator()<0>();
     launch.template operator()<1>();
     launch.template operator()<2>();
-    if (gather) {
-        StartAdj sa;
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b) sa.p[a][b] = c->vjp_start[a][b];
-        start_gather_kernel<<<xcd_blocks_for(g.foff[3]), kBlock, 0, c->stream>>>(g, per, sa, va);
-    }
     check_launch("advect_velocity_vjp_kernel");
 }
 

@@ -105,56 +105,64 @@ __device__ __forceinline__ uint32_t xcd_block() {
 
 __device__ __forceinline__ bool vperiodic(const VBound& b, int d) { return b.modes[2 * d] == 3u && b.modes[2 * d + 1] == 3u; }
 __device__ __forceinline__ bool speriodic(const SBound& b, int d) { return b.modes[2 * d] == 2u && b.modes[2 * d + 1] == 2u; }
+// v modulo p for a coordinate that is at most one period outside [0, p) in almost every case.
 __device__ __forceinline__ int wrapi(int v, int p) {
-    const int r = v % p;
-    return r < 0 ? r + p : r;
-}
-__device__ __forceinline__ int mapc(int v, int size, bool per, int period) {
-    return per ? wrapi(v, period) : max(0, min(size - 1, v));
+    int r = v < 0 ? v + p : v >= p ? v - p : v;
+    if ((unsigned)r >= (unsigned)p) {
+        r = v % p;
+        r = r < 0 ? r + p : r;
+    }
+    return r;
 }
 
-// load_scalar constant test (operators.cu:115-121 / scatter skip at :212).
-__device__ __forceinline__ bool scalar_const(const Geo& g, int x, int y, int z, const SBound& b, float& value) {
-    if (x < 0 && b.modes[0] == 0u) { value = b.values[0]; return true; }
-    if (x >= g.nx && b.modes[1] == 0u) { value = b.values[1]; return true; }
-    if (y < 0 && b.modes[2] == 0u) { value = b.values[2]; return true; }
-    if (y >= g.ny && b.modes[3] == 0u) { value = b.values[3]; return true; }
-    if (z < 0 && b.modes[4] == 0u) { value = b.values[4]; return true; }
-    if (z >= g.nz && b.modes[5] == 0u) { value = b.values[5]; return true; }
-    return false;
-}
-__device__ __forceinline__ uint32_t scalar_mapped(const Geo& g, int x, int y, int z, const SBound& b) {
-    x = mapc(x, g.nx, speriodic(b, 0), g.nx);
-    y = mapc(y, g.ny, speriodic(b, 1), g.ny);
-    z = mapc(z, g.nz, speriodic(b, 2), g.nz);
-    return cidx(g, x, y, z);
-}
-// load_face constant test (operators.cu:125-132 / scatter skip at :230-237). The axis is a
-// template parameter so that every boundary-array index is a compile-time constant (a runtime
-// index into a by-value kernel argument would move it to scratch memory).
-template <int A>
-__device__ __forceinline__ bool face_const(const Geo& g, int x, int y, int z, const VBound& b, float& value) {
-    const int c[3]{x, y, z};
+// One axis of a trilinear stencil whose lower corner is at coordinate c0, on a lattice of `size`
+// points: the stored coordinates of its two corners (periodic: modulo `period`, the cell count;
+// else clamped), and whether each corner lies beyond a face whose value is fixed, with the value.
+// The bounds are tested per axis, not per corner, and without divisions: a wave that holds one
+// domain-edge cell runs this for all its lanes (the rows of a grid end in every second wave at 128^3),
+// so the boundary path's instructions bound the trace kernels. With this form, the fixed stencils of
+// the start point (start_velocity) and paired loads: velocity / scalar reverse 277 / 448 -> 159 / 207
+// us (per axis at 128^3), velocity / scalar tangent 608 / 258 -> 180 / 79 us (96^3), forward velocity
+// 133 -> 53 us (90 x 70 x 110, solids) and 1241 -> 756 us (256^3).
+struct AxisStencil {
+    int i[2];
+    bool fixed[2];
+    float value[2];
+};
+__device__ __forceinline__ AxisStencil axis_stencil(int c0, int size, bool periodic, int period, bool fix_lo, bool fix_hi, float lo,
+                                                    float hi) {
+    AxisStencil s;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const int size = ext(g, A, d);
-        if (c[d] < 0) {
-            const uint32_t m = b.modes[2 * d];
-            if (m == 0u || (m == 2u && A == d)) { value = b.values[3 * (2 * d) + A]; return true; }
-        } else if (c[d] >= size) {
-            const uint32_t m = b.modes[2 * d + 1];
-            if (m == 0u || (m == 2u && A == d)) { value = b.values[3 * (2 * d + 1) + A]; return true; }
-        }
+    for (int k = 0; k < 2; ++k) {
+        const int c = c0 + k;
+        const bool below = c < 0, above = c >= size;
+        s.fixed[k] = (below && fix_lo) || (above && fix_hi);
+        s.value[k] = below ? lo : hi;
+        s.i[k] = periodic ? wrapi(c, period) : min(max(c, 0), size - 1);
     }
-    return false;
+    return s;
 }
-// mapped_face_index, operators.cu:105-113 (period = cell count of the dimension).
-template <int A>
-__device__ __forceinline__ uint32_t face_mapped(const Geo& g, int x, int y, int z, const VBound& b) {
-    x = mapc(x, ext(g, A, 0), vperiodic(b, 0), g.nx);
-    y = mapc(y, ext(g, A, 1), vperiodic(b, 1), g.ny);
-    z = mapc(z, ext(g, A, 2), vperiodic(b, 2), g.nz);
-    return fidx(g, A, x, y, z);
+
+// load_scalar's rule for axis d (operators.cu:115-121, scatter skip at :212).
+template <int D>
+__device__ __forceinline__ AxisStencil scalar_axis(const Geo& g, int c0, const SBound& b) {
+    const int n = dim_size(g, D);
+    return axis_stencil(c0, n, speriodic(b, D), n, b.modes[2 * D] == 0u, b.modes[2 * D + 1] == 0u, b.values[2 * D], b.values[2 * D + 1]);
+}
+// load_face's rule for the faces of axis A along axis D (operators.cu:105-113,125-132, scatter skip
+// at :230-237). The axes are template parameters so that every boundary-array index is a
+// compile-time constant (a runtime index into a by-value kernel argument would move it to scratch).
+template <int A, int D>
+__device__ __forceinline__ AxisStencil face_axis(const Geo& g, int c0, const VBound& b) {
+    const uint32_t ml = b.modes[2 * D], mh = b.modes[2 * D + 1];
+    return axis_stencil(c0, ext(g, A, D), vperiodic(b, D), dim_size(g, D), ml == 0u || (ml == 2u && A == D), mh == 0u || (mh == 2u && A == D),
+                        b.values[3 * (2 * D) + A], b.values[3 * (2 * D + 1) + A]);
+}
+
+// Index x + ex (y + ey z) of a lattice whose extents are at most 1025: the partial products fit the
+// 24-bit multiply, which runs at the full rate (the 32-bit one at a quarter of it).
+__device__ __forceinline__ uint32_t lattice_index(int x, int y, int z, int ex, int ey) {
+    return (uint32_t)x + __umul24((uint32_t)ex, (uint32_t)y + __umul24((uint32_t)ey, (uint32_t)z));
 }
 
 struct Corner8 {   // the 2x2x2 trilinear stencil: base cell and fractional offsets
@@ -178,9 +186,9 @@ __device__ __forceinline__ Corner8 corners(const Geo& g, float px, float py, flo
     // stays representable) and takes the boundary-mapped loads; finite positions within 2^24
     // cells of the domain are unchanged.
     constexpr float kFar = 16777216.0f;
-    c.x0 = (int)fminf(fmaxf(fx, -kFar), kFar);
-    c.y0 = (int)fminf(fmaxf(fy, -kFar), kFar);
-    c.z0 = (int)fminf(fmaxf(fz, -kFar), kFar);
+    c.x0 = (int)__builtin_amdgcn_fmed3f(fx, -kFar, kFar);
+    c.y0 = (int)__builtin_amdgcn_fmed3f(fy, -kFar, kFar);
+    c.z0 = (int)__builtin_amdgcn_fmed3f(fz, -kFar, kFar);
     c.tx = gx - fx;
     c.ty = gy - fy;
     c.tz = gz - fz;
@@ -220,6 +228,36 @@ __device__ __forceinline__ bool face_interior(const Geo& g, const Corner8& c, co
     return c.x0 >= 0 && c.x0 + 1 < lx && c.y0 >= 0 && c.y0 + 1 < ly && c.z0 >= 0 && c.z0 + 1 < lz;
 }
 
+// The 8 corner values of an interior stencil: four loads of two neighbours along x (4-byte aligned)
+// from one address per row pair.
+struct __attribute__((packed, aligned(4))) Pair {
+    float a, b;
+};
+__device__ __forceinline__ void load8(const float* __restrict__ v, uint32_t base, uint32_t sy, uint32_t sz, float vals[8]) {
+    const float* p = v + base;
+    const Pair q0 = *reinterpret_cast<const Pair*>(p), q1 = *reinterpret_cast<const Pair*>(p + sy);
+    const Pair q2 = *reinterpret_cast<const Pair*>(p + sz), q3 = *reinterpret_cast<const Pair*>(p + (size_t)(sz + sy));
+    vals[0] = q0.a;
+    vals[1] = q0.b;
+    vals[2] = q1.a;
+    vals[3] = q1.b;
+    vals[4] = q2.a;
+    vals[5] = q2.b;
+    vals[6] = q3.a;
+    vals[7] = q3.b;
+}
+// The 8 corner values of a stencil that touches a boundary; x decides a corner's fixed value before
+// y, y before z.
+__device__ __forceinline__ void load8_boundary(const float* __restrict__ v, const AxisStencil& ax, const AxisStencil& ay,
+                                               const AxisStencil& az, int ex, int ey, float vals[8]) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
+        const float l = v[lattice_index(ax.i[dx], ay.i[dy], az.i[dz], ex, ey)];
+        vals[k] = ax.fixed[dx] ? ax.value[dx] : ay.fixed[dy] ? ay.value[dy] : az.fixed[dz] ? az.value[dz] : l;
+    }
+}
+
 // sample_face (operators.cu:166-194) with an interior fast path.
 template <int A, bool Grad>
 __device__ __forceinline__ Sample sample_face(const float* __restrict__ v, float px, float py, float pz, const Geo& g,
@@ -227,25 +265,10 @@ __device__ __forceinline__ Sample sample_face(const float* __restrict__ v, float
     const Corner8 c = corners(g, px, py, pz, A == 0 ? 0.0f : 0.5f, A == 1 ? 0.0f : 0.5f, A == 2 ? 0.0f : 0.5f);
     const int ex = ext(g, A, 0), ey = ext(g, A, 1);
     float vals[8];
-    if (face_interior<A>(g, c, b)) {
-        const uint32_t base = (uint32_t)c.x0 + (uint32_t)ex * ((uint32_t)c.y0 + (uint32_t)ey * (uint32_t)c.z0);
-        const uint32_t sy = (uint32_t)ex, sz = (uint32_t)ex * (uint32_t)ey;
-        vals[0] = v[base];
-        vals[1] = v[base + 1];
-        vals[2] = v[base + sy];
-        vals[3] = v[base + sy + 1];
-        vals[4] = v[base + sz];
-        vals[5] = v[base + sz + 1];
-        vals[6] = v[base + sz + sy];
-        vals[7] = v[base + sz + sy + 1];
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int x = c.x0 + (k & 1), y = c.y0 + ((k >> 1) & 1), z = c.z0 + (k >> 2);
-            float cv;
-            vals[k] = face_const<A>(g, x, y, z, b, cv) ? cv : v[face_mapped<A>(g, x, y, z, b)];
-        }
-    }
+    if (face_interior<A>(g, c, b))
+        load8(v, lattice_index(c.x0, c.y0, c.z0, ex, ey), (uint32_t)ex, (uint32_t)ex * (uint32_t)ey, vals);
+    else
+        load8_boundary(v, face_axis<A, 0>(g, c.x0, b), face_axis<A, 1>(g, c.y0, b), face_axis<A, 2>(g, c.z0, b), ex, ey, vals);
     return trilerp<Grad>(vals, c, g.inv_h);
 }
 
@@ -255,112 +278,61 @@ __device__ __forceinline__ Sample sample_scalar(const float* __restrict__ v, flo
                                                 const SBound& b) {
     const Corner8 c = corners(g, px, py, pz, 0.5f, 0.5f, 0.5f);
     float vals[8];
-    if (c.x0 >= 0 && c.x0 + 1 < g.nx && c.y0 >= 0 && c.y0 + 1 < g.ny && c.z0 >= 0 && c.z0 + 1 < g.nz) {
-        const uint32_t base = cidx(g, c.x0, c.y0, c.z0);
-        const uint32_t sy = (uint32_t)g.nx, sz = (uint32_t)g.nx * (uint32_t)g.ny;
-        vals[0] = v[base];
-        vals[1] = v[base + 1];
-        vals[2] = v[base + sy];
-        vals[3] = v[base + sy + 1];
-        vals[4] = v[base + sz];
-        vals[5] = v[base + sz + 1];
-        vals[6] = v[base + sz + sy];
-        vals[7] = v[base + sz + sy + 1];
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int x = c.x0 + (k & 1), y = c.y0 + ((k >> 1) & 1), z = c.z0 + (k >> 2);
-            float cv;
-            vals[k] = scalar_const(g, x, y, z, b, cv) ? cv : v[scalar_mapped(g, x, y, z, b)];
-        }
-    }
+    if (c.x0 >= 0 && c.x0 + 1 < g.nx && c.y0 >= 0 && c.y0 + 1 < g.ny && c.z0 >= 0 && c.z0 + 1 < g.nz)
+        load8(v, lattice_index(c.x0, c.y0, c.z0, g.nx, g.ny), (uint32_t)g.nx, (uint32_t)g.nx * (uint32_t)g.ny, vals);
+    else
+        load8_boundary(v, scalar_axis<0>(g, c.x0, b), scalar_axis<1>(g, c.y0, b), scalar_axis<2>(g, c.z0, b), g.nx, g.ny, vals);
     return trilerp<Grad>(vals, c, g.inv_h);
 }
 
-// Sink of a scatter: adds value to face (x, y, z) of axis A (flat index i). The default adds to
-// the global array with an FP32 atomic.
-struct GlobalSink {
-    float* v;
-    template <int A>
-    __device__ __forceinline__ void add(int, int, int, uint32_t i, float value) const { atomicAdd(v + i, value); }
-};
+// The adds of one trilinear stencil's transpose (operators.cu:196-240) into array W of a sink: the
+// corners' weights times adj, on a lattice of extents ex, ey. `interior`: every corner is a stored
+// point (at c.x0 .. c.x0 + 1 and so on); else the axes' stencils give the points and the skipped
+// corners. A sink may take a whole interior stencil at once (Sink::window8: true when all eight
+// points lie in its window); it is not offered non-finite adjoints, whose product with a zero weight
+// would not be 0.
+template <int W, typename Sink, typename Axes>
+__device__ __forceinline__ void scatter8(const Sink& sink, const Corner8& c, float adj, int ex, int ey, bool interior, Axes&& axes) {
+    const float w[2][3] = {{1.0f - c.tx, 1.0f - c.ty, 1.0f - c.tz}, {c.tx, c.ty, c.tz}};
+    float a[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] = w[k & 1][0] * w[(k >> 1) & 1][1] * w[k >> 2][2];
+    if (interior && fabsf(adj) < __builtin_inff() && sink.template window8<W>(c.x0, c.y0, c.z0, adj, a)) return;
+    AxisStencil ax, ay, az;
+    axes(ax, ay, az);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
+        if (ax.fixed[dx] || ay.fixed[dy] || az.fixed[dz] || a[k] == 0.0f) continue;
+        const int x = ax.i[dx], y = ay.i[dy], z = az.i[dz];
+        sink.template add<W>(x, y, z, lattice_index(x, y, z, ex, ey), adj * a[k]);
+    }
+}
 
 // scatter_face (operators.cu:217-240): transpose of sample_face's value.
 template <int A, typename Sink>
 __device__ __forceinline__ void scatter_face_to(const Sink& sink, float px, float py, float pz, float adj, const Geo& g, const VBound& b) {
     if (adj == 0.0f) return;
     const Corner8 c = corners(g, px, py, pz, A == 0 ? 0.0f : 0.5f, A == 1 ? 0.0f : 0.5f, A == 2 ? 0.0f : 0.5f);
-    const int ex = ext(g, A, 0), ey = ext(g, A, 1);
-    const float w[2][3] = {{1.0f - c.tx, 1.0f - c.ty, 1.0f - c.tz}, {c.tx, c.ty, c.tz}};
-    if (face_interior<A>(g, c, b)) {
-        const uint32_t base = (uint32_t)c.x0 + (uint32_t)ex * ((uint32_t)c.y0 + (uint32_t)ey * (uint32_t)c.z0);
-        const uint32_t sy = (uint32_t)ex, sz = (uint32_t)ex * (uint32_t)ey;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-            const float wk = w[dx][0] * w[dy][1] * w[dz][2];
-            if (wk != 0.0f) sink.template add<A>(c.x0 + dx, c.y0 + dy, c.z0 + dz, base + dx + dy * sy + dz * sz, adj * wk);
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-            int x = c.x0 + dx, y = c.y0 + dy, z = c.z0 + dz;
-            float cv;
-            if (face_const<A>(g, x, y, z, b, cv)) continue;
-            const float wk = w[dx][0] * w[dy][1] * w[dz][2];
-            if (wk == 0.0f) continue;
-            x = mapc(x, ext(g, A, 0), vperiodic(b, 0), g.nx);
-            y = mapc(y, ext(g, A, 1), vperiodic(b, 1), g.ny);
-            z = mapc(z, ext(g, A, 2), vperiodic(b, 2), g.nz);
-            sink.template add<A>(x, y, z, fidx(g, A, x, y, z), adj * wk);
-        }
-    }
+    scatter8<A>(sink, c, adj, ext(g, A, 0), ext(g, A, 1), face_interior<A>(g, c, b), [&](AxisStencil& ax, AxisStencil& ay, AxisStencil& az) {
+        ax = face_axis<A, 0>(g, c.x0, b);
+        ay = face_axis<A, 1>(g, c.y0, b);
+        az = face_axis<A, 2>(g, c.z0, b);
+    });
 }
 
-template <int A>
-__device__ __forceinline__ void scatter_face(float* v, float px, float py, float pz, float adj, const Geo& g, const VBound& b) {
-    scatter_face_to<A>(GlobalSink{v}, px, py, pz, adj, g, b);
-}
-
-// scatter_scalar with a sink: the same weights and skips, the adds go to sink.add<W>(x, y, z, i, value)
-// with (x, y, z) the mapped cell and i its index (W names the sink's target array).
+// scatter_scalar (operators.cu:196-215): transpose of sample_scalar's value, into the sink's array W.
 template <int W, typename Sink>
 __device__ __forceinline__ void scatter_scalar_to(const Sink& sink, float px, float py, float pz, float adj, const Geo& g,
                                                   const SBound& b) {
     if (adj == 0.0f) return;
     const Corner8 c = corners(g, px, py, pz, 0.5f, 0.5f, 0.5f);
-    const float w[2][3] = {{1.0f - c.tx, 1.0f - c.ty, 1.0f - c.tz}, {c.tx, c.ty, c.tz}};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-        int x = c.x0 + dx, y = c.y0 + dy, z = c.z0 + dz;
-        float cv;
-        if (scalar_const(g, x, y, z, b, cv)) continue;
-        const float wk = w[dx][0] * w[dy][1] * w[dz][2];
-        if (wk == 0.0f) continue;
-        x = mapc(x, g.nx, speriodic(b, 0), g.nx);
-        y = mapc(y, g.ny, speriodic(b, 1), g.ny);
-        z = mapc(z, g.nz, speriodic(b, 2), g.nz);
-        sink.template add<W>(x, y, z, cidx(g, x, y, z), adj * wk);
-    }
-}
-
-// scatter_scalar (operators.cu:196-215).
-__device__ __forceinline__ void scatter_scalar(float* v, float px, float py, float pz, float adj, const Geo& g,
-                                               const SBound& b) {
-    if (adj == 0.0f) return;
-    const Corner8 c = corners(g, px, py, pz, 0.5f, 0.5f, 0.5f);
-    const float w[2][3] = {{1.0f - c.tx, 1.0f - c.ty, 1.0f - c.tz}, {c.tx, c.ty, c.tz}};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-        const int x = c.x0 + dx, y = c.y0 + dy, z = c.z0 + dz;
-        float cv;
-        if (scalar_const(g, x, y, z, b, cv)) continue;
-        const float wk = w[dx][0] * w[dy][1] * w[dz][2];
-        if (wk != 0.0f) atomicAdd(v + scalar_mapped(g, x, y, z, b), adj * wk);
-    }
+    const bool interior = c.x0 >= 0 && c.x0 + 1 < g.nx && c.y0 >= 0 && c.y0 + 1 < g.ny && c.z0 >= 0 && c.z0 + 1 < g.nz;
+    scatter8<W>(sink, c, adj, g.nx, g.ny, interior, [&](AxisStencil& ax, AxisStencil& ay, AxisStencil& az) {
+        ax = scalar_axis<0>(g, c.x0, b);
+        ay = scalar_axis<1>(g, c.y0, b);
+        az = scalar_axis<2>(g, c.z0, b);
+    });
 }
 
 struct Vel3 {
@@ -386,16 +358,85 @@ struct TraceOut {
     float mx, my, mz;   // midpoint
 };
 
-// trace_rk2, operators.cu:256-276. has_solids = false skips the mask lookup (no colliders).
+// Component B of the velocity at a lattice point: face (x, y, z) of axis L, or the centre of cell
+// (x, y, z) for L = 3. The trilinear stencil is fixed there: along an axis where the two lattices
+// agree one point (weight 1), else the two around it (1/2 each); so 1, 2 or 4 loads instead of 8.
+// Order of the sums: x inside y inside z, as trilerp.
+template <int L, int B>
+struct StartStencil {
+    // axis d of B's stencil has two points when exactly one of L and B is staggered along d
+    static constexpr bool two(int d) { return (L == d) != (B == d); }
+    // lower point's offset: a face of axis L sits between cells c - 1 and c, a cell between faces c and c + 1
+    static constexpr int lower(int d) { return L == d && B != d ? -1 : 0; }
+};
+template <int L, int B, int D>
+__device__ __forceinline__ AxisStencil start_axis(const Geo& g, int c, const VBound& b) {
+    return face_axis<B, D>(g, c + StartStencil<L, B>::lower(D), b);
+}
+template <int L, int B>
+__device__ __forceinline__ float start_velocity(const float* __restrict__ v, int x, int y, int z, const Geo& g, const VBound& b) {
+    using S = StartStencil<L, B>;
+    const AxisStencil ax = start_axis<L, B, 0>(g, x, b), ay = start_axis<L, B, 1>(g, y, b), az = start_axis<L, B, 2>(g, z, b);
+    const int ex = ext(g, B, 0), ey = ext(g, B, 1);
+    float sz[2];
+#pragma unroll
+    for (int dz = 0; dz <= (S::two(2) ? 1 : 0); ++dz) {
+        float sy[2];
+#pragma unroll
+        for (int dy = 0; dy <= (S::two(1) ? 1 : 0); ++dy) {
+            float sx[2];
+#pragma unroll
+            for (int dx = 0; dx <= (S::two(0) ? 1 : 0); ++dx) {
+                const float l = v[lattice_index(ax.i[dx], ay.i[dy], az.i[dz], ex, ey)];
+                sx[dx] = ax.fixed[dx] ? ax.value[dx] : ay.fixed[dy] ? ay.value[dy] : az.fixed[dz] ? az.value[dz] : l;
+            }
+            sy[dy] = S::two(0) ? 0.5f * sx[0] + 0.5f * sx[1] : sx[0];
+        }
+        sz[dz] = S::two(1) ? 0.5f * sy[0] + 0.5f * sy[1] : sy[0];
+    }
+    return S::two(2) ? 0.5f * sz[0] + 0.5f * sz[1] : sz[0];
+}
+// Transpose of start_velocity into array B of a sink.
+template <int L, int B, typename Sink>
+__device__ __forceinline__ void scatter_start(const Sink& sink, int x, int y, int z, float adj, const Geo& g, const VBound& b) {
+    if (adj == 0.0f) return;
+    using S = StartStencil<L, B>;
+    const AxisStencil ax = start_axis<L, B, 0>(g, x, b), ay = start_axis<L, B, 1>(g, y, b), az = start_axis<L, B, 2>(g, z, b);
+    const float a = adj * ((S::two(0) ? 0.5f : 1.0f) * (S::two(1) ? 0.5f : 1.0f) * (S::two(2) ? 0.5f : 1.0f));
+#pragma unroll
+    for (int dz = 0; dz <= (S::two(2) ? 1 : 0); ++dz)
+#pragma unroll
+        for (int dy = 0; dy <= (S::two(1) ? 1 : 0); ++dy)
+#pragma unroll
+            for (int dx = 0; dx <= (S::two(0) ? 1 : 0); ++dx) {
+                if (ax.fixed[dx] || ay.fixed[dy] || az.fixed[dz]) continue;
+                const int px = ax.i[dx], py = ay.i[dy], pz = az.i[dz];
+                sink.template add<B>(px, py, pz, lattice_index(px, py, pz, ext(g, B, 0), ext(g, B, 1)), a);
+            }
+}
+
+// Position of a lattice point (a face of axis L, or a cell centre for L = 3).
+struct Pos {
+    float x, y, z;
+};
+template <int L>
+__device__ __forceinline__ Pos start_position(const Geo& g, int x, int y, int z) {
+    return Pos{(x + (L == 0 ? 0.0f : 0.5f)) * g.h, (y + (L == 1 ? 0.0f : 0.5f)) * g.h, (z + (L == 2 ? 0.0f : 0.5f)) * g.h};
+}
+
+// trace_rk2, operators.cu:256-276, from face (x, y, z) of axis L (a cell centre for L = 3).
+// has_solids = false skips the mask lookup (no colliders).
 // MidGrad: also return the three velocity samples at the midpoint with their gradients in mid
 // (the reverse and tangent sweeps need them; the values are the ones the trace uses).
-template <bool HasSolids, bool MidGrad = false>
-__device__ __forceinline__ TraceOut trace_rk2(float sx, float sy, float sz, const Vel3& u, const uint8_t* __restrict__ mask,
+template <int L, bool HasSolids, bool MidGrad = false>
+__device__ __forceinline__ TraceOut trace_rk2(int x, int y, int z, const Vel3& u, const uint8_t* __restrict__ mask,
                                               const Geo& g, const VBound& b, Sample* mid = nullptr) {
     TraceOut t;
-    const float v0x = sample_face<0, false>(u.u[0], sx, sy, sz, g, b).value;
-    const float v0y = sample_face<1, false>(u.u[1], sx, sy, sz, g, b).value;
-    const float v0z = sample_face<2, false>(u.u[2], sx, sy, sz, g, b).value;
+    const Pos start = start_position<L>(g, x, y, z);
+    const float sx = start.x, sy = start.y, sz = start.z;
+    const float v0x = start_velocity<L, 0>(u.u[0], x, y, z, g, b);
+    const float v0y = start_velocity<L, 1>(u.u[1], x, y, z, g, b);
+    const float v0z = start_velocity<L, 2>(u.u[2], x, y, z, g, b);
     t.mx = sx - 0.5f * g.dt * v0x;
     t.my = sy - 0.5f * g.dt * v0y;
     t.mz = sz - 0.5f * g.dt * v0z;

@@ -118,10 +118,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void a
                 if (A == 2) z = 0;
             }
         }
-        const float sx = (x + (A == 0 ? 0.0f : 0.5f)) * g.h;
-        const float sy = (y + (A == 1 ? 0.0f : 0.5f)) * g.h;
-        const float sz = (z + (A == 2 ? 0.0f : 0.5f)) * g.h;
-        const TraceOut t = trace_rk2<HasSolids>(sx, sy, sz, u, mask, g, b);
+        const TraceOut t = trace_rk2<A, HasSolids>(x, y, z, u, mask, g, b);
         out.p[A][local] = sample_face<A, false>(u.u[A], t.px, t.py, t.pz, g, b).value;
     });
 }
@@ -193,7 +190,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void a
     }
     int x, y, z;
     decode_cell(g, i, x, y, z);
-    const TraceOut t = trace_rk2<HasSolids>((x + 0.5f) * g.h, (y + 0.5f) * g.h, (z + 0.5f) * g.h, u, mask, g, vb);
+    const TraceOut t = trace_rk2<3, HasSolids>(x, y, z, u, mask, g, vb);
     out0[i] = sample_scalar<false>(src0, t.px, t.py, t.pz, g, sb0).value;
     if (NF == 2) out1[i] = sample_scalar<false>(src1, t.px, t.py, t.pz, g, sb1).value;
 }

@@ -124,17 +124,17 @@ __global__ __launch_bounds__(256) void buoyancy_jvp_kernel(Geo g, const uint8_t*
 }
 
 // The shared part of advect_velocity_jvp_kernel and advect_scalar_jvp_kernel (operators.cu:390-412,
-// 509-533): the trace from s, and the tangent of its end point.
-template <bool HasSolids>
-__device__ __forceinline__ TraceOut trace_tangent(float sx, float sy, float sz, const Vel3& u, const Vel3& ut,
+// 509-533): the trace from a lattice point (trace_rk2), and the tangent of its end point.
+template <int L, bool HasSolids>
+__device__ __forceinline__ TraceOut trace_tangent(int x, int y, int z, const Vel3& u, const Vel3& ut,
                                                   const uint8_t* __restrict__ mask, const Geo& g, const VBound& b, const VBound& bz,
                                                   float pos_t[3]) {
     Sample mid[3];
-    const TraceOut t = trace_rk2<HasSolids, true>(sx, sy, sz, u, mask, g, b, mid);
+    const TraceOut t = trace_rk2<L, HasSolids, true>(x, y, z, u, mask, g, b, mid);
     const float hdt = -0.5f * g.dt;
-    const float mtx = hdt * sample_face<0, false>(ut.u[0], sx, sy, sz, g, bz).value;
-    const float mty = hdt * sample_face<1, false>(ut.u[1], sx, sy, sz, g, bz).value;
-    const float mtz = hdt * sample_face<2, false>(ut.u[2], sx, sy, sz, g, bz).value;
+    const float mtx = hdt * start_velocity<L, 0>(ut.u[0], x, y, z, g, bz);
+    const float mty = hdt * start_velocity<L, 1>(ut.u[1], x, y, z, g, bz);
+    const float mtz = hdt * start_velocity<L, 2>(ut.u[2], x, y, z, g, bz);
     const Sample& s0 = mid[0];
     const Sample& s1 = mid[1];
     const Sample& s2 = mid[2];
@@ -172,11 +172,8 @@ __global__ __launch_bounds__(256) void advect_velocity_jvp_kernel(Geo g, const V
                 if (A == 2) z = 0;
             }
         }
-        const float sx = (x + (A == 0 ? 0.0f : 0.5f)) * g.h;
-        const float sy = (y + (A == 1 ? 0.0f : 0.5f)) * g.h;
-        const float sz = (z + (A == 2 ? 0.0f : 0.5f)) * g.h;
         float pt[3];
-        const TraceOut t = trace_tangent<HasSolids>(sx, sy, sz, u, ut, mask, g, b, bz, pt);
+        const TraceOut t = trace_tangent<A, HasSolids>(x, y, z, u, ut, mask, g, b, bz, pt);
         const Sample src = sample_face<A, true>(u.u[A], t.px, t.py, t.pz, g, b);
         out.p[A][local] = sample_face<A, false>(ut.u[A], t.px, t.py, t.pz, g, bz).value + src.gx * pt[0] + src.gy * pt[1] + src.gz * pt[2];
     });
@@ -201,7 +198,7 @@ __global__ __launch_bounds__(256) void advect_scalar_jvp_kernel(Geo g, const VBo
     int x, y, z;
     decode_cell(g, i, x, y, z);
     float pt[3];
-    const TraceOut t = trace_tangent<HasSolids>((x + 0.5f) * g.h, (y + 0.5f) * g.h, (z + 0.5f) * g.h, u, ut, mask, g, *vbp, *vbzp, pt);
+    const TraceOut t = trace_tangent<3, HasSolids>(x, y, z, u, ut, mask, g, *vbp, *vbzp, pt);
     const Sample s0 = sample_scalar<true>(src0, t.px, t.py, t.pz, g, *sb0p);
     out0[i] = sample_scalar<false>(src0_t, t.px, t.py, t.pz, g, *sbz0p).value + s0.gx * pt[0] + s0.gy * pt[1] + s0.gz * pt[2];
     if (NF == 2) {
