@@ -43,20 +43,22 @@ BYTES_OTHER["pcg_resident_kernel"] = BYTES_OTHER["pcg_fused_kernel"]
 # pcg_s2_kernel (s-step form, two iterations per launch): every cell reads the code, the five
 # basis vectors and the solution increment and writes the new basis and the increment
 BYTES_UNKNOWN["pcg_s2_kernel"] = BYTES_OTHER["pcg_s2_kernel"] = 1 + 5 * 4 + 4 + 5 * 4 + 4
-# pcg_mg_iteration (multigrid-preconditioned form; the timed unit is one iteration, thirteen
-# kernels: the V-cycle, the direction and the update). Level 0 per unknown: pre-smoothing reads
-# code and r and writes x (9), restriction reads code, r, x and writes an eighth of a coarse value
-# (9.5), the first post sweep reads code, r, x, an eighth of the coarse result and writes y (13.5),
-# the second reads code, r, y and writes z (13), the direction reads code, z, p_old and writes p
-# (13), the update reads code, p, r and the solution pair and writes r and the pair (29); other
-# cells read the code and write the zeros of x, y, z, p (22.5 with the restriction's share). Each
-# cell of a coarser level but the last: diagonal, its reciprocal, three couplings and the
-# right-hand side read by the down and the up kernel, an eighth of a value written down, an eighth
-# read and the result written up (53); the coarsest level's FP64 inverse is read once (mg_bytes).
-BYTES_UNKNOWN["pcg_mg_iteration"] = 9 + 9.5 + 13.5 + 13 + 13 + 29
-BYTES_OTHER["pcg_mg_iteration"] = 5 + 1.5 + 5 + 5 + 5 + 1
-MG_COARSE_BYTES_PER_CELL = 53
-MG_COARSEST = 512
+# pcg_mg_iteration (multigrid-preconditioned form; the timed unit is one iteration: direction, down
+# and post kernels of level 0, two kernels per coarser level of more than MG_BOTTOM cells, one for
+# the levels below). Level 0 per unknown: the direction reads code, z, p_old and writes p (13); the
+# down kernel reads code, p, r and the solution pair and writes r, the pair, the smoothed iterate and
+# an eighth of a coarse value (33.5); the post kernel reads code, x, r, an eighth of the coarse result
+# and writes z (13.5); other cells read the code and write the zeros of r, x, z, p (17.5 with the
+# restriction's share). Each cell of a coarser level but the last: diagonal, its reciprocal, three
+# couplings and the right-hand side read by the down and the up kernel, the iterate written and read,
+# an eighth of a value each way and the result written up (61); the coarsest level's FP64 inverse is
+# read once (mg_bytes).
+BYTES_UNKNOWN["pcg_mg_iteration"] = 13 + 33.5 + 13.5
+BYTES_OTHER["pcg_mg_iteration"] = 5 + 9.5 + 5
+MG_COARSE_BYTES_PER_CELL = 61
+MG_DIRECT = 512    # a grid of at most this many cells is solved directly
+MG_COARSEST = 64   # else the coarsest level has at most this many
+MG_BOTTOM = 4096
 # advect_velocity_vjp_kernel, one launch per face axis: 75 B per face of the axis (the reference's
 # decomposition: the face's output adjoint, the three velocity components of its trace and the
 # three adjoint components it scatters into, each array streamed once)
@@ -65,15 +67,28 @@ FACE_BYTES = {"advect_velocity_vjp_kernel": 75}
 COMPOSITE = {"pcg_mg_iteration"}
 
 
-def mg_bytes(res):
-    """Bytes of the coarser levels and the coarsest inverse per multigrid iteration: 2 x 2 x 2
-    aggregation (extents halved, rounded up) until at most MG_COARSEST cells."""
-    dims, coarse = list(res), 0
+def mg_levels(res):
+    """Cells of the coarser levels of the multigrid hierarchy: 2 x 2 x 2 aggregation (extents halved,
+    rounded up) until at most MG_COARSEST cells."""
+    dims, cells = list(res), []
+    if dims[0] * dims[1] * dims[2] <= MG_DIRECT:
+        return cells
     while dims[0] * dims[1] * dims[2] > MG_COARSEST:
         dims = [(d + 1) // 2 for d in dims]
-        coarse += dims[0] * dims[1] * dims[2]
-    last = dims[0] * dims[1] * dims[2]
-    return MG_COARSE_BYTES_PER_CELL * (coarse - (last if coarse else 0)) + 4 * last * 2 + 8 * last * last
+        cells.append(dims[0] * dims[1] * dims[2])
+    return cells
+
+
+def mg_bytes(res):
+    """Bytes of the coarser levels and the coarsest inverse per multigrid iteration."""
+    cells = mg_levels(res)
+    last = cells[-1] if cells else res[0] * res[1] * res[2]
+    return MG_COARSE_BYTES_PER_CELL * sum(cells[:-1]) + 4 * last * 2 + 8 * last * last
+
+
+def mg_kernels(res):
+    """Kernels per multigrid iteration."""
+    return 4 + 2 * sum(c > MG_BOTTOM for c in mg_levels(res)) if mg_levels(res) else 5
 
 
 def host_threads():
@@ -385,7 +400,7 @@ def main():
         "loss": r["loss"],
         "cnn_vs_plain": cnn_vs_plain,
         "roofline": roofline,
-        "solver_iteration": next(({"unit": k, "kernels_per_iteration": 13, "avg_us": round(kern[k]["avg_us"], 2),
+        "solver_iteration": next(({"unit": k, "kernels_per_iteration": mg_kernels(sc.resolution), "avg_us": round(kern[k]["avg_us"], 2),
                                    "algorithmic_bytes": kern[k]["algorithmic_bytes"], "achieved": round(kern[k]["gbs"], 1),
                                    "peak": HBM_PEAK_GBS, "unit_bw": "GB/s", "frac": round(kern[k]["gbs"] / HBM_PEAK_GBS, 4)}
                                   for k in COMPOSITE if k in kern and kern[k]["gbs"]), None),

@@ -107,8 +107,9 @@ struct PcgStatus {
     uint32_t aborted;       // 1 when a resident launch's grid barrier exceeded its bound
     double bb;              // ||b||^2
     double rr;              // last reduced ||r||^2 (recursive or true)
-    uint32_t k;             // DS_CG_MULTIGRID: the iteration whose V-cycle ran last (advanced on the device)
+    uint32_t k;             // DS_CG_MULTIGRID: updates applied so far (advanced on the device)
     uint32_t unused;
+    double rr0;             // DS_CG_MULTIGRID: ||r||^2 of the initial guess
 };
 
 // HIP-event timing of sampled PCG kernel launches (kernel 0 = direction, 1 = update, 2 = the
@@ -169,7 +170,7 @@ struct PcgWork {
     float* p[2]{};               // search directions, ping-pong between iterations
     uint32_t blocks = 8;         // blocks of the PCG kernels
     uint32_t variant = DS_CG_SINGLE_REDUCTION;
-    // single-reduction form: r (sets r, r_alt), w = A D^-1 r and s = A p double-buffered; p = p[0]
+    // multigrid form: r (sets r, r_alt); single-reduction form: r (sets r, r_alt), w = A D^-1 r and s = A p double-buffered; p = p[0]
     float* r_alt = nullptr;
     float* wv[2]{};
     float* sv[2]{};
@@ -187,7 +188,9 @@ struct PcgWork {
     // vectors on chip (pcg_resident.hpp; DS_CG_SINGLE_REDUCTION_RESIDENT), when the grid allows it
     bool resident = false;
     uint32_t* resident_sync = nullptr;   // ResidentSync (2 words)
-    uint32_t mg_expect = 0;      // DS_CG_MULTIGRID: iterations of the last converged solve
+    // DS_CG_MULTIGRID: iterations of the last solve of each sequence: the right-hand-side kinds, and
+    // [4] the forward solves replayed from their stored solution
+    uint32_t mg_expect[5]{6, 6, 6, 6, 0};
 };
 
 // DS_CG_MULTIGRID (pcg_mg.hip): one level of the aggregation hierarchy. Level 0 is the pressure
@@ -204,15 +207,29 @@ struct MgLevel {
     const float* wp[3];
 };
 constexpr int kMgMaxLevels = 32;
-constexpr uint32_t kMgCoarsest = 512;   // at most this many cells on the level solved directly
+constexpr uint32_t kMgCoarsest = 512;   // a grid of at most this many cells is solved directly
+constexpr uint32_t kMgDense = 64;       // else at most this many cells on the level solved directly
+constexpr uint32_t kMgBottomCells = 4096;   // levels of at most this many cells share one workgroup
+// Over all grids of extents up to 1024 these levels number at most 5, with at most 5720 cells
+// together, 1140 on the second and 342 on the third.
+constexpr uint32_t kMgBottomLds = 6144;
+constexpr int kMgBottomLevels = 5;
+struct MgBottom {
+    uint32_t count;
+    uint32_t off[kMgBottomLevels];  // first element of each level's vectors
+    uint32_t n[kMgBottomLevels], nx[kMgBottomLevels], nxy[kMgBottomLevels];
+    const uint32_t* words[kMgBottomLevels];   // rows and neighbours (pcg_mg.hip), none for the last level
+    const double* dense;
+};
 struct MgWork {
     int levels = 0;
     MgLevel lv[kMgMaxLevels]{};
-    // per level: right-hand side (levels > 0), pre-smoothed iterate (level 0), iterate after the
-    // first post sweep (level 0), result (levels > 0)
-    float* vec[kMgMaxLevels][4]{};
+    // per level: right-hand side (levels > 0), pre-smoothed iterate, result (levels > 0)
+    float* vec[kMgMaxLevels][3]{};
     double* dense = nullptr;        // inverse of the coarsest operator, n x n (symmetric)
-    float* z = nullptr;             // the preconditioned residual (n + 1, zero pad)
+    float* z = nullptr;             // the preconditioned residual
+    int bottom_first = 1;           // first level of the single-workgroup kernel
+    MgBottom bottom{};
     // one iteration (V-cycle, direction, update) captured as a HIP graph per solution pair and
     // tolerance: a kernel launch costs the host about as long as the kernels of a coarse level
     // take on the device, a graph launch replays all thirteen for about the cost of one
@@ -342,9 +359,11 @@ ds_solve_info pcg_solve(ds_context* c, float* x_hi, float* x_lo, const float* x0
 // Solves A x = b with b built from `u` (kind 1: forward divergence of the advected velocity;
 // kind 2: adjoint, u = projected-velocity adjoint plus `extra`; kind 3: tangent, the forward
 // divergence without the fixed-face term) or given in c->pcg.b (kind 0).
-// correct: under DS_WARM_START_CNN the network corrects the given guess (x0h, x0l).
+// correct: under DS_WARM_START_CNN the network corrects the given guess (x0h, x0l). replay: the guess
+// is this very solve's stored solution.
 ds_solve_info pcg_solve_kind(ds_context* c, int kind, const float* const u[3], const float* const extra[3], float* xh,
-                             float* xl, const float* x0h, const float* x0l, double tol, uint32_t max_it, bool correct = false);
+                             float* xl, const float* x0h, const float* x0l, double tol, uint32_t max_it, bool correct = false,
+                             bool replay = false);
 uint32_t pcg_periodic_bits(const ds_context* c);
 // DS_WARM_START_PROJECTION (window.hip): the window of a right-hand-side kind (null when the mode
 // is off or the kind has none), the guess for right-hand side b (null while the window is empty),
@@ -357,19 +376,19 @@ void window_allocate(ds_context* c, SolveWindow& w);
 // Decides whether the single-reduction solve runs resident (full 64 x kTY tiles, at most 8 planes
 // per block, cooperative launch possible with every block co-resident) and allocates its state.
 void pcg_resident_prepare(ds_context* c);
-// DS_CG_MULTIGRID (pcg_mg.hip): builds the hierarchy from the host copy of the code; then per
-// iteration z = M^-1 r (the V-cycle, <r, z> partials into pcg.partials), the direction kernel
-// (convergence test, p = z + beta p_old, <p, A p> partials) and the update kernel (solution pair
-// x = (xh, xl), residual, ||r||^2 partials).
-// The kernels take the iteration index from the status (PcgStatus::k, advanced by the V-cycle's
-// first kernel), so one captured iteration replays for every k: mg_set_iteration sets it (the
-// V-cycle of iteration k runs after k - 1), mg_iteration launches the captured iteration (captured
-// on first use for the pair and tolerance), mg_release destroys the captured graphs.
+// DS_CG_MULTIGRID (pcg_mg.hip): builds the hierarchy from the host copy of the code. A solve is
+// mg_start (stopping test and V-cycle of the residual as it stands; first: take ||b||^2 and the
+// initial residual; reject: 1 a guess with a residual above ||b||, 2 only a non-finite one), then one
+// mg_iteration per iteration: direction, update of the solution pair (xh, xl) and the residual,
+// stopping test, V-cycle. The kernels take the iteration index k from the status (set-up and
+// mg_set_iteration set it, the stopping test of an iteration advances it), so one captured iteration
+// (per pair and tolerance) replays for every k; the residual of index k is mg_residual(k).
+// mg_blocks: blocks of the level-0 kernels, one partial each; mg_release destroys the graphs.
 void mg_prepare(ds_context* c, const std::vector<uint8_t>& code);
-void mg_precondition(ds_context* c, const float* r, float* z);
-void mg_direction(ds_context* c, const float* z, double tol2, bool check_only);
-void mg_update(ds_context* c, float* xh, float* xl);
-void mg_set_iteration(ds_context* c, uint32_t k_before);
+uint32_t mg_blocks(const ds_context* c);
+void mg_start(ds_context* c, double tol2, uint32_t first, uint32_t reject);
+void mg_set_iteration(ds_context* c, uint32_t k);
+float* mg_residual(const ds_context* c, uint32_t k);
 void mg_iteration(ds_context* c, float* xh, float* xl, double tol2);
 void mg_release(ds_context* c);
 // DS_PROJECTION_RBGS (rbgs.hip): the diagonal table, then the solve of a right-hand-side kind

@@ -166,7 +166,7 @@ ds_solve_info forward_step(ds_context* c, const ds_state* s, const ds_control* k
     }
     const float* uac[3]{ua.p[0], ua.p[1], ua.p[2]};
     const ds_solve_info si = pcg_solve_kind(c, 1, uac, nullptr, c->pressure_hi, c->pressure_lo, x0h, x0l, c->tolerance, c->max_iterations,
-                                            c->config.warm_start == DS_WARM_START_CNN && !cache->pressure_guess);
+                                            c->config.warm_start == DS_WARM_START_CNN && !cache->pressure_guess, cache->pressure_guess != nullptr);
     c->pressure_valid = true;
     launch_project(c, CF3{{ua.p[0], ua.p[1], ua.p[2]}}, c->pressure_hi, c->pressure_lo, F3{{next->velocity[0], next->velocity[1], next->velocity[2]}});
     launch_advect_scalars(c, 2, 0, cache->sourced_density, cache->sourced_temperature,

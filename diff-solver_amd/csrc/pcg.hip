@@ -142,21 +142,24 @@ __global__ __launch_bounds__(kPcgThreads) void pcg_setup_kernel(Geo g, uint32_t 
             status->iterations = 0u;
             status->rejected = 0u;
             status->aborted = 0u;
+            status->k = 0u;
         }
     }
 }
 
-// True residual r = b - A (x_hi + x_lo) in FP64; replaces the recursive residual.
+// True residual r = b - A (x_hi + x_lo) in FP64; replaces the recursive residual (r_odd, when given,
+// is the residual of odd iteration counts: DS_CG_MULTIGRID). stop_mode 1: not once the solve has
+// stopped; 2: only then.
 __global__ __launch_bounds__(kPcgThreads) void pcg_true_residual_kernel(Geo g, uint32_t per, const uint8_t* __restrict__ code,
                                                                 const float* __restrict__ b, const float* __restrict__ xh,
-                                                                const float* __restrict__ xl, float* __restrict__ r,
+                                                                const float* __restrict__ xl, float* __restrict__ r_even,
                                                                 double* __restrict__ partials, PcgStatus* status,
-                                                                uint32_t respect_stop) {
+                                                                uint32_t stop_mode, float* __restrict__ r_odd = nullptr) {
     __shared__ double lds[3 * kMaxWaves];
-    if (respect_stop && status->stop) return;
+    if (stop_mode && (status->stop != 0u) == (stop_mode == 1u)) return;
+    float* __restrict__ r = r_odd && (status->k & 1u) ? r_odd : r_even;
     uint32_t lb, start, end;
     block_range(g.n, lb, start, end);
-    const uint32_t G = gridDim.x;
     double rr = 0.0, rz = 0.0;
     for (uint32_t i = start + threadIdx.x; i < end; i += blockDim.x) {
         const uint32_t d = code[i];
@@ -314,10 +317,12 @@ __global__ __launch_bounds__(kPcgThreads) void pcg_s2_gram_kernel(Geo g, uint32_
     s2_block_partials(acc, lds, out_parts + 16u * lb);
 }
 
-// One block: reduce the ||b||^2 (optional) and ||r||^2 partials into the status.
+// One block: reduce the ||b||^2 (optional) and ||r||^2 partials into the status (if_stopped: only
+// once the solve has stopped).
 __global__ __launch_bounds__(256) void pcg_finalize_kernel(const double* __restrict__ partials, uint32_t G,
-                                                           PcgStatus* status, uint32_t with_bb) {
+                                                           PcgStatus* status, uint32_t with_bb, uint32_t if_stopped = 0u) {
     __shared__ double lds[3 * kMaxWaves];
+    if (if_stopped && !status->stop) return;
     const double* parts[2]{partials + kPartBB * kPcgMaxBlocks, partials + kPartRR * kPcgMaxBlocks};
     double red[2];
     reduce_partials<2>(parts, G, red, lds);
@@ -724,41 +729,39 @@ ds_solve_info pcg_iterate_s2(ds_context* c, float* xh, float* xl, double tol, ui
     return info;
 }
 
-// Multigrid-preconditioned iteration (DS_CG_MULTIGRID, pcg_mg.hip) from the state left by
-// launch_setup (r; BB, RR partials) until the true residual meets tol or max_it. Iteration k: the
-// V-cycle z = M^-1 r, the direction kernel (stopping test, p, <p, A p>), the update kernel (which
-// adds to the solution pair directly); the true residual is recomputed every replacement interval.
-ds_solve_info pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, uint32_t max_it, bool warm, bool rejected) {
+// Multigrid-preconditioned iteration (DS_CG_MULTIGRID, pcg_mg.hip) from the state left by launch_setup
+// (r; BB, RR partials) until the true residual meets tol or max_it; the true residual is recomputed
+// every replacement interval. reject (mg_start): the guess is dropped on the device and the caller
+// runs the solve again without it (returns true then, with nothing else decided).
+// The host waits once per solve in the usual case: it queues as many iterations as the previous solve
+// of the same sequence took (a V-cycle's rate hardly changes along a trajectory), the final residual
+// behind them (both kernels return at once unless the solve has stopped), and reads the status.
+bool pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, uint32_t max_it, int sequence, uint32_t reject, ds_solve_info& info,
+                    double& rr0) {
     PcgWork& w = c->pcg;
     const uint32_t per = periodic_bits(c);
     const double tol2 = tol * tol;
     const uint32_t R = c->replacement_interval;
-    float* z = c->mg.z;
-    auto true_residual = [&](uint32_t respect_stop) {
+    auto true_residual = [&](uint32_t stop_mode) {
         pcg_true_residual_kernel<<<w.blocks, kPcgThreads, 0, c->stream>>>(c->geo, per, c->code, w.b, xh, xl, w.r, w.partials, w.status,
-                                                                          respect_stop);
+                                                                          stop_mode, w.r_alt);
     };
-    ds_solve_info info{};
-    info.warm_started = warm ? 1u : 0u;
-    info.guess_rejected = rejected ? 1u : 0u;
-    // ||b||^2 (and ||r0||^2) from the set-up's partials into the status; iteration 0 next
-    pcg_finalize_kernel<<<1, kBlock, 0, c->stream>>>(w.partials, w.blocks, w.status, 1u);
-    mg_set_iteration(c, ~0u);
+    auto finish = [&](uint32_t stop_mode) {
+        true_residual(stop_mode);
+        pcg_finalize_kernel<<<1, kBlock, 0, c->stream>>>(w.partials, w.blocks, w.status, 0u, stop_mode);
+        check_launch("pcg_true_residual_kernel");
+        return read_status(c);
+    };
+    mg_start(c, tol2, 1u, reject);
     uint32_t k = 0;
     uint32_t restarts = 0;
     Profiler& prof = c->profiler;
     while (true) {
-        // Batches are queued one ahead of the status the host reads, and the iterations queued
-        // behind the stop cost their launches: the first batch runs to a little before the
-        // previous solve's count (a V-cycle's convergence rate hardly changes between the solves
-        // of a trajectory), the later ones two iterations at a time.
-        uint32_t batch = w.mg_expect > 4u ? w.mg_expect - 3u : 2u;
-        int slot = 0, pending = -1;
-        bool stop_seen = false;
+        uint32_t batch = restarts ? 1u : w.mg_expect[sequence];
         PcgStatus st{};
-        while (k < max_it && !stop_seen) {
+        while (true) {
             const uint32_t nb = std::min(batch, max_it - k);
-            for (uint32_t j = 0; j < nb; ++j, ++k) {
+            for (uint32_t j = 0; j < nb; ++j) {
                 hipEvent_t e0 = nullptr, e1 = nullptr;
                 if (prof.every && k % prof.every == 0 && prof.used + 2 <= 6000) {
                     e0 = prof.take();
@@ -771,55 +774,37 @@ ds_solve_info pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, ui
                     prof.recs.push_back({5, e0, e1});
                 }
                 if (prof.every) prof.launches[5]++;
-                if ((k + 1u) % R == 0u && k + 1u < max_it) true_residual(1u);
-            }
-            check_launch("pcg multigrid iteration");
-            DS_HIP(hipMemcpyAsync(&w.host_status[slot], w.status, sizeof(PcgStatus), hipMemcpyDeviceToHost, c->stream));
-            DS_HIP(hipEventRecord(w.batch_event[slot], c->stream));
-            if (pending >= 0) {
-                DS_HIP(hipEventSynchronize(w.batch_event[pending]));
-                if (w.host_status[pending].stop) {
-                    stop_seen = true;
-                    st = w.host_status[pending];
+                ++k;
+                if (k % R == 0u && k < max_it) {   // residual replacement, and its V-cycle
+                    true_residual(1u);
+                    mg_start(c, tol2, 0u, 0u);
                 }
             }
-            pending = slot;
-            slot ^= 1;
-            batch = 2u;
+            st = finish(2u);
+            if (st.stop || k >= max_it) break;
+            batch = 1u;
         }
-        // the stopping launch's status when the host saw it, else the last batch's
-        if (!stop_seen) st = read_status(c);
-        if (!st.stop && k >= max_it) {
-            // one more stopping test on the last update's residual (its V-cycle gives the RZ
-            // partials the test reads but does not use)
-            mg_precondition(c, w.r, z);
-            mg_direction(c, z, tol2, true);
-            check_launch("mg_direction_kernel");
-            st = read_status(c);
-        }
+        if (st.rejected) return true;
+        rr0 = st.rr0;
         const uint32_t done = st.stop ? st.iterations : max_it;
         k = done;
-        true_residual(0u);
-        pcg_finalize_kernel<<<1, kBlock, 0, c->stream>>>(w.partials, w.blocks, w.status, 0u);
-        check_launch("pcg_true_residual_kernel");
-        const PcgStatus fin = read_status(c);
-        if (st.stop) w.mg_expect = done;
+        if (st.stop) w.mg_expect[sequence] = done;
+        else st = finish(0u);
         info.iterations = done;
-        info.rhs_norm = std::sqrt(fin.bb);
-        info.final_residual = std::sqrt(std::max(0.0, fin.rr));
-        const bool finite = std::isfinite(fin.rr);
-        const bool ok = finite && fin.rr <= tol2 * fin.bb;
+        info.rhs_norm = std::sqrt(st.bb);
+        info.final_residual = std::sqrt(std::max(0.0, st.rr));
+        const bool finite = std::isfinite(st.rr);
+        const bool ok = finite && st.rr <= tol2 * st.bb;
         info.converged = ok ? 1u : 0u;
-        if (!finite) info.final_residual = fin.rr;
+        if (!finite) info.final_residual = st.rr;
         if (ok || !finite || !st.stop || done >= max_it || ++restarts > 8) break;
         // the recursive residual met the tolerance but the true one (now in r) does not: continue
         // from it with the previous direction discarded
         fill_zero(c, w.p[(k + 1u) & 1u], c->geo.n);
-        mg_set_iteration(c, k - 1u);
-        pcg_clear_stop_kernel<<<1, 64, 0, c->stream>>>(w.status);
-        check_launch("pcg_clear_stop_kernel");
+        mg_set_iteration(c, k);
+        mg_start(c, tol2, 0u, 0u);
     }
-    return info;
+    return false;
 }
 
 // Iterates from the state left by launch_setup until the true residual meets tol or max_it.
@@ -933,13 +918,14 @@ void pcg_resident_prepare(ds_context* c) {
 
 // Solves A x = b for the given right-hand-side kind. Returns the solve info; x = (xh, xl).
 ds_solve_info pcg_solve_kind(ds_context* c, int kind, const float* const u[3], const float* const extra[3], float* xh,
-                             float* xl, const float* x0h, const float* x0l, double tol, uint32_t max_it, bool correct) {
+                             float* xl, const float* x0h, const float* x0l, double tol, uint32_t max_it, bool correct, bool replay) {
     if (c->config.projection_solver == DS_PROJECTION_RBGS && kind != kRhsGiven) return rbgs_solve_kind(c, kind, u, extra, xh, xl);
     RhsIn in{};
     for (int a = 0; a < 3; ++a) {
         in.u[a] = u ? u[a] : nullptr;
         in.extra[a] = extra ? extra[a] : nullptr;
     }
+    const int sequence = replay ? 4 : kind;
     max_it = std::min(max_it, c->max_iterations);   // the per-iteration history is sized for this cap
     bool network_guess = false;
     // a solve with a given guess (the recompute pass's taped pressure) is not part of the sequence
@@ -973,7 +959,21 @@ ds_solve_info pcg_solve_kind(ds_context* c, int kind, const float* const u[3], c
     const bool warm = x0h != nullptr;
     bool rejected = false;
     launch_setup(c, kind, in, x0h, x0l, x0h == xh, xh, xl);
-    double rr0 = 0.0, bb = 0.0;
+    double rr0 = 0.0;
+    if (c->pcg.variant == DS_CG_MULTIGRID) {
+        // the guess is judged on the device by the rules below
+        ds_solve_info info{};
+        rejected = pcg_iterate_mg(c, xh, xl, tol, max_it, sequence, !warm ? 0u : network_guess ? 2u : 1u, info, rr0);
+        if (rejected) {
+            launch_setup(c, kRhsGiven, in, nullptr, nullptr, false, xh, xl);
+            (void)pcg_iterate_mg(c, xh, xl, tol, max_it, sequence, 0u, info, rr0);
+        }
+        info.warm_started = warm ? 1u : 0u;
+        info.guess_rejected = rejected ? 1u : 0u;
+        info.initial_residual = warm && !rejected ? std::sqrt(std::max(0.0, rr0)) : info.rhs_norm;
+        if (win && info.converged) window_add(c, *win, xh, xl);
+        return info;
+    }
     if (warm) {
         // Reject a non-finite guess, and a given guess whose residual exceeds ||b|| (worse than
         // x0 = 0). The network's guess is scaled to its A-norm-optimal multiple, which never has
@@ -982,7 +982,6 @@ ds_solve_info pcg_solve_kind(ds_context* c, int kind, const float* const u[3], c
         check_launch("pcg_finalize_kernel");
         const PcgStatus s = read_status(c);
         rr0 = s.rr;
-        bb = s.bb;
         if (!std::isfinite(s.rr) || (!network_guess && !(s.rr <= s.bb))) {
             rejected = true;
             launch_setup(c, kRhsGiven, in, nullptr, nullptr, false, xh, xl);
@@ -990,10 +989,8 @@ ds_solve_info pcg_solve_kind(ds_context* c, int kind, const float* const u[3], c
     }
     ds_solve_info info = c->pcg.variant == DS_CG_SINGLE_REDUCTION ? pcg_iterate_fused(c, xh, xl, tol, max_it, warm, rejected)
                          : c->pcg.variant == DS_CG_S_STEP        ? pcg_iterate_s2(c, xh, xl, tol, max_it, warm, rejected)
-                         : c->pcg.variant == DS_CG_MULTIGRID     ? pcg_iterate_mg(c, xh, xl, tol, max_it, warm, rejected)
                                                                  : pcg_iterate(c, xh, xl, tol, max_it, warm, rejected);
     info.initial_residual = warm && !rejected ? std::sqrt(std::max(0.0, rr0)) : info.rhs_norm;
-    (void)bb;
     if (win && info.converged) window_add(c, *win, xh, xl);
     return info;
 }

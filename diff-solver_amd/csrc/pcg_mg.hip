@@ -1,35 +1,47 @@
 // pcg_mg.hip — conjugate gradients preconditioned by an aggregation multigrid V-cycle
 // (DS_CG_MULTIGRID): the same pressure system as the Jacobi forms (the reference solves it with
 // Jacobi-preconditioned CG, solvers/smoke/operators.cu), to the same FP64 stopping test on the true
-// residual, in a few tens of iterations instead of about a thousand at 128^3.
+// residual, in about ten iterations instead of about a thousand at 128^3.
 //
 // Hierarchy: each coarser level aggregates 2 x 2 x 2 cells of the finer one (an odd extent leaves
 // a last aggregate one cell wide; an extent of 1 stays 1). The prolongation P copies a coarse value
 // to the aggregate's cells and the restriction is its transpose (the cells' sum), so the coarse
 // operator A_c = P^T A P sums the fine couplings over the aggregates: a 7-point operator again, held
 // as its diagonal and the per-axis couplings to the + neighbour, built once per context on the host
-// from the connectivity code (periodic wraps included). The coarsest level (at most kMgCoarsest
-// cells) is solved exactly with its inverse (FP64 Cholesky on the host, applied in FP64).
+// from the connectivity code (periodic wraps included). The coarsest level (at most kMgDense cells)
+// is solved exactly with its inverse (FP64 Cholesky on the host, applied in FP64); a grid of at most
+// kMgCoarsest cells is its own coarsest level.
 //
-// V-cycle (symmetric, so a valid CG preconditioner): damped Jacobi sweeps from zero (two on level 0,
-// one on the coarser levels), the residual restricted, the coarse correction scaled up (piecewise-
-// constant aggregation under-corrects smooth errors; scaling it is the usual remedy), then as many
-// damped Jacobi sweeps again. Values a sweep needs at the neighbours are formed on the fly: level 0
-// costs four launches (pre-smoothing, restriction, two post sweeps), a coarser level two (down: the
-// restriction of the residual after its pre-smoothing; up: prolongation plus its post sweep).
-// Without the over-correction an FP64 CPU model of the 128^3 plume needs about twice the CG
-// iterations (25 against 13 on V(2,2)); Jacobi-PCG needs 1015.
+// V-cycle (symmetric, so a valid CG preconditioner): on every level two Jacobi sweeps from zero
+// weighted as the second Chebyshev polynomial on [0.45, 2] (D^-1 A has its spectrum in [0, 2]; the
+// lower end is where the smoother hands over to the coarse level), the residual restricted, the
+// coarse correction scaled by 1.9 (piecewise-constant aggregation under-corrects smooth errors:
+// its coarse operator is about twice too stiff), the two sweeps again in the reverse order. An FP64
+// CPU model (random and smooth right-hand sides, 64^3 to 128^3, with and without solids) needs 7 to
+// 10 iterations to 1e-6 this way; with the equal weights of 0.9, one sweep on the coarser levels and
+// corrections of 1.8 and 1.5 that this file used before, 11 to 17; Jacobi-PCG 1015 at 128^3.
 //
-// The outer loop is textbook PCG with two reductions per iteration: the direction kernel forms
-// p = z + beta p_old and <p, A p>; the update kernel adds alpha p to the solution increment, updates
-// the residual and forms ||r||^2; the V-cycle's last kernel forms <r, z>. Every scalar comes from
-// FP64 per-block partials that each consumer block reduces in the same order. Every kernel returns at
-// once after the stopping test has fired, so the iterations queued behind it cost only launches.
+// The outer loop is textbook PCG with two reductions per iteration. Level 0 costs three kernels per
+// iteration, each staging its brick of cells and the halo that its chain of stencils needs in LDS:
+//   direction   p = z + beta p_old, <p, A p>                                         (halo 1)
+//   down        x += alpha p, r -= alpha A p, ||r||^2; both sweeps; restriction      (halo 3 of p)
+//   post        prolongation, both sweeps, <r, z>                                    (halo 2)
+// The halo's values are recomputed instead of exchanged. A coarser level of more than kMgBottomCells
+// costs two kernels of the same build; the levels below run in one workgroup that keeps them in LDS
+// (a 16^3 grid fills one CU, and a launch costs more than its sweeps). Every scalar comes from FP64
+// per-block partials that each consumer block reduces in the same order, so the iteration is
+// deterministic. Every kernel returns at once after the stopping test has fired.
+// Measured (128^3, kernel trace): 8 launches and about 110 us an iteration, 9 iterations from x0 = 0,
+// where thirteen launches took 108 us and 19 iterations; 64^3: 6 launches, 40 us, 8 iterations against
+// 11, 50 us, 12; 256^3: 620 us, 11 iterations against 720 us, 24.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <bit>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "context.hpp"
@@ -38,319 +50,807 @@ namespace ds {
 
 namespace {
 
-// Level 0 runs V(2,2) (two damped Jacobi sweeps before and after the coarse correction), the coarser
-// levels V(1,1): an FP64 CPU model of the 128^3 plume with random right-hand sides needs 14 CG
-// iterations to 1e-6 for these parameters, 13 with V(2,2) on every level (four launches per level
-// instead of two), 17 with V(1,1) everywhere.
-constexpr float kOmega0 = 0.9f;   // level-0 Jacobi damping
-constexpr float kOver0 = 1.8f;    // scale of the coarse correction prolonged to level 0
-constexpr float kOmegaC = 0.9f;   // coarser levels
-constexpr float kOverC = 1.5f;
-constexpr uint32_t kMgThreads = 512;   // the kernels over contiguous ranges of level 0
-constexpr uint32_t kMgUnroll = 4;      // cells per thread whose loads are in flight together there
+// 1 / (centre -+ half width cos(pi / 4)) of [0.45, 2]: the roots of the second Chebyshev polynomial.
+constexpr float kCheb[2]{0.564013325f, 1.477121796f};
+constexpr float kOver = 1.9f;   // scale of the prolonged coarse correction
+constexpr uint32_t kMgDotThreads = 512;
+constexpr uint32_t kMgLargeCells = 1u << 19, kMgMediumCells = 1u << 16;   // box of level 0 by its cells
+constexpr uint32_t kMgCoarseLarge = 1u << 17;                             // box of a coarser level
 
-__device__ __forceinline__ void mg_coords(const MgLevel& L, uint32_t i, int& x, int& y, int& z) {
-    const uint32_t t = fdiv(i, L.dx);
-    x = (int)(i - t * (uint32_t)L.nx);
-    const uint32_t u = fdiv(t, L.dy);
-    y = (int)(t - u * (uint32_t)L.ny);
-    z = (int)u;
-}
+// 1 / d for a level-0 diagonal count (the hardware reciprocal: every use of a cell's value is the
+// same, so the smoother stays symmetric). Counts of 0 (not an unknown) give 1; the values they scale
+// are 0 there.
+__device__ __forceinline__ float mg_dinv(uint32_t d) { return __builtin_amdgcn_rcpf((float)max(d, 1u)); }
 
-// omega / d for a level-0 diagonal count (the hardware reciprocal: every use of a cell's value is
-// the same, so the smoother stays symmetric). Counts of 0 (not an unknown, or the zero pad) give
-// omega; the values they scale are 0 there.
-__device__ __forceinline__ float mg_wdinv(uint32_t d) { return kOmega0 * __builtin_amdgcn_rcpf((float)max(d, 1u)); }
-
-// Level-0 neighbours of cell i = (x, y, z) in the order -x, +x, -y, +y, -z, +z. A periodic axis
-// wraps (on an extent of 1 both neighbours are i itself, as in the matrix-vector product); a
-// neighbour beyond a non-periodic axis is index n, the zero pad every level-0 vector and the code
-// carry, so it reads 0 and adds nothing: no branch per neighbour.
-struct Nb0 {
-    uint32_t j[6];
-};
-__device__ __forceinline__ Nb0 mg_nb0(const MgLevel& L, uint32_t per, int x, int y, int z, uint32_t i) {
-    const uint32_t n = L.n, sy = (uint32_t)L.nx, sz = (uint32_t)L.nx * (uint32_t)L.ny;
-    Nb0 s;
-    s.j[0] = x > 0 ? i - 1u : ((per & 1u) ? i + (uint32_t)(L.nx - 1) : n);
-    s.j[1] = x + 1 < L.nx ? i + 1u : ((per & 1u) ? i - (uint32_t)(L.nx - 1) : n);
-    s.j[2] = y > 0 ? i - sy : ((per & 2u) ? i + (uint32_t)(L.ny - 1) * sy : n);
-    s.j[3] = y + 1 < L.ny ? i + sy : ((per & 2u) ? i - (uint32_t)(L.ny - 1) * sy : n);
-    s.j[4] = z > 0 ? i - sz : ((per & 4u) ? i + (uint32_t)(L.nz - 1) * sz : n);
-    s.j[5] = z + 1 < L.nz ? i + sz : ((per & 4u) ? i - (uint32_t)(L.nz - 1) * sz : n);
-    return s;
-}
-
-// Level-1 aggregates of cell (x, y, z)'s level-0 neighbours, in mg_nb0's order (a neighbour beyond
-// a non-periodic axis gets the cell's own aggregate: its value is not used), and of the cell itself.
-__device__ __forceinline__ uint32_t mg_nb0_parents(const MgLevel& L, const MgLevel& C, uint32_t per, int x, int y, int z, uint32_t (&P)[6]) {
-    const int X = x >> 1, Y = y >> 1, Z = z >> 1;
-    const uint32_t sy = (uint32_t)C.nx, sz = (uint32_t)C.nx * (uint32_t)C.ny;
-    const uint32_t P0 = (uint32_t)X + sy * (uint32_t)Y + sz * (uint32_t)Z;
-    int q;
-    q = x > 0 ? x - 1 : ((per & 1u) ? L.nx - 1 : x);
-    P[0] = P0 + (uint32_t)((q >> 1) - X);
-    q = x + 1 < L.nx ? x + 1 : ((per & 1u) ? 0 : x);
-    P[1] = P0 + (uint32_t)((q >> 1) - X);
-    q = y > 0 ? y - 1 : ((per & 2u) ? L.ny - 1 : y);
-    P[2] = P0 + (uint32_t)((q >> 1) - Y) * sy;
-    q = y + 1 < L.ny ? y + 1 : ((per & 2u) ? 0 : y);
-    P[3] = P0 + (uint32_t)((q >> 1) - Y) * sy;
-    q = z > 0 ? z - 1 : ((per & 4u) ? L.nz - 1 : z);
-    P[4] = P0 + (uint32_t)((q >> 1) - Z) * sz;
-    q = z + 1 < L.nz ? z + 1 : ((per & 4u) ? 0 : z);
-    P[5] = P0 + (uint32_t)((q >> 1) - Z) * sz;
-    return P0;
-}
-
-// Calls f(j, q, w) for every neighbour j of cell i = (x, y, z) on level L: q its coordinates, w the
-// coupling A_ij (level 0: -1, to be applied to values that are 0 off the unknowns; coarser levels:
-// i's + coupling, or the - neighbour's own). A periodic axis wraps (on an extent of 1 both
-// neighbours are i itself, as in the level-0 matrix-vector product); a non-periodic one ends.
-template <bool Fine, typename F>
-__device__ __forceinline__ void mg_for_neighbours(const MgLevel& L, uint32_t per, int x, int y, int z, uint32_t i, F&& f) {
-    const int ext[3]{L.nx, L.ny, L.nz};
-    const uint32_t stride[3]{1u, (uint32_t)L.nx, (uint32_t)L.nx * (uint32_t)L.ny};
-    const int c[3]{x, y, z};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const bool pa = per & (1u << a);
-        if (c[a] + 1 < ext[a] || pa) {
-            int q[3]{x, y, z};
-            q[a] = c[a] + 1 < ext[a] ? c[a] + 1 : 0;
-            const uint32_t j = i + (uint32_t)(q[a] - c[a]) * stride[a];
-            f(j, q, Fine ? -1.0f : L.wp[a][i]);
-        }
-        if (c[a] > 0 || pa) {
-            int q[3]{x, y, z};
-            q[a] = c[a] > 0 ? c[a] - 1 : ext[a] - 1;
-            const uint32_t j = i + (uint32_t)(q[a] - c[a]) * stride[a];
-            f(j, q, Fine ? -1.0f : L.wp[a][j]);
-        }
-    }
-}
-
-// Off-diagonal part of (A v)_i, v given by value(j, q) (0 off the level's unknowns).
-template <bool Fine, typename F>
-__device__ __forceinline__ float mg_offdiag(const MgLevel& L, uint32_t per, int x, int y, int z, uint32_t i, F&& value) {
-    float s = 0.0f;
-    mg_for_neighbours<Fine>(L, per, x, y, z, i, [&](uint32_t j, const int (&q)[3], float w) {
-        if constexpr (Fine) s -= value(j, q);
-        else s = __fmaf_rn(w, value(j, q), s);
-    });
-    return s;
-}
-
-// Index on level C of the aggregate holding the finer cell with coordinates q.
-__device__ __forceinline__ uint32_t mg_parent(const MgLevel& C, const int (&q)[3]) {
-    return (uint32_t)(q[0] >> 1) + (uint32_t)C.nx * ((uint32_t)(q[1] >> 1) + (uint32_t)C.ny * (uint32_t)(q[2] >> 1));
-}
-
-// Contiguous cell range of this block (XCD-remapped) for the kernels that reduce over level 0.
-__device__ __forceinline__ void mg_range(uint32_t n, uint32_t& lb, uint32_t& start, uint32_t& end) {
-    lb = xcd_block();
-    uint32_t chunk = (n + gridDim.x - 1) / gridDim.x;
-    chunk = (chunk + blockDim.x - 1) / blockDim.x * blockDim.x;
-    start = min(n, lb * chunk);
-    end = min(n, start + chunk);
-}
-
-// Level 0, two damped Jacobi sweeps from zero for A x = r: x1 = w D^-1 r, x = x1 + w D^-1 (r - A x1),
-// with x1 at the neighbours formed on the fly.
-// Advances the iteration index (the first kernel of every V-cycle; nothing else reads it here).
-__global__ __launch_bounds__(kBlock) void mg_pre0_kernel(MgLevel L, uint32_t per, const float* __restrict__ r, float* __restrict__ x,
-                                                         PcgStatus* status) {
-    if (status->stop) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) status->k = status->k + 1u;
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
-    if (i >= L.n) return;
-    const uint32_t d = L.code[i];
-    if (d == 0u) {
-        x[i] = 0.0f;
-        return;
-    }
-    int cx, cy, cz;
-    mg_coords(L, i, cx, cy, cz);
-    const Nb0 nb = mg_nb0(L, per, cx, cy, cz, i);
-    float s1 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) s1 += mg_wdinv(L.code[nb.j[k]]) * r[nb.j[k]];
-    const float ri = r[i], w = mg_wdinv(d);
-    const float xi1 = w * ri;
-    const float ax1 = __fmaf_rn((float)d, xi1, -s1);
-    x[i] = __fmaf_rn(w, ri - ax1, xi1);
-}
-
-// Restriction on the coarser levels with one thread per cell (there are few aggregates to spread
-// the work over): thread t handles child k = t mod 8 of aggregate I = t / 8
-// (k = 1 x-bit + 2 y-bit + 4 z-bit), so the 8 lanes of an aligned group share I and their values are
-// summed with three butterfly shuffles (the same association in every lane). Sets the child's cell
-// coordinates and index; false when the child lies beyond an odd extent (it contributes 0).
-__device__ __forceinline__ bool mg_child(const MgLevel& L, const MgLevel& C, uint32_t t, uint32_t& I, int (&q)[3], uint32_t& i) {
-    I = t >> 3;
-    const uint32_t k = t & 7u;
-    int X, Y, Z;
-    mg_coords(C, I, X, Y, Z);
-    q[0] = 2 * X + (int)(k & 1u);
-    q[1] = 2 * Y + (int)((k >> 1) & 1u);
-    q[2] = 2 * Z + (int)(k >> 2);
-    i = (uint32_t)q[0] + (uint32_t)L.nx * ((uint32_t)q[1] + (uint32_t)L.ny * (uint32_t)q[2]);
-    return q[0] < L.nx && q[1] < L.ny && q[2] < L.nz;
-}
-
-__device__ __forceinline__ float mg_group8_sum(float v) {
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
-    v += __shfl_xor(v, 4, 64);
-    return v;
-}
-
-// Level 0 to 1: rc_I = sum of (r - A x)_i over the cells i of aggregate I (x: the pre-smoothed
-// iterate), one thread per aggregate (consecutive lanes read consecutive pairs of cells of each
-// row: coalesced, unlike one lane per cell of a 2 x 2 x 2 block). Children beyond an odd extent are
-// clamped onto the last cell and masked out, so every load is issued unconditionally.
-__global__ __launch_bounds__(kBlock) void mg_restrict0_kernel(MgLevel L, MgLevel C, uint32_t per, const float* __restrict__ r,
-                                                              const float* __restrict__ x, float* __restrict__ rc, const PcgStatus* status) {
-    if (status->stop) return;
-    const uint32_t I = xcd_block() * blockDim.x + threadIdx.x;
-    if (I >= C.n) return;
-    int X, Y, Z;
-    mg_coords(C, I, X, Y, Z);
-    float s = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int qx = 2 * X + (k & 1), qy = 2 * Y + ((k >> 1) & 1), qz = 2 * Z + (k >> 2);
-        const bool inside = qx < L.nx && qy < L.ny && qz < L.nz;
-        const int cx = min(qx, L.nx - 1), cy = min(qy, L.ny - 1), cz = min(qz, L.nz - 1);
-        const uint32_t i = (uint32_t)cx + (uint32_t)L.nx * ((uint32_t)cy + (uint32_t)L.ny * (uint32_t)cz);
-        const uint32_t d = L.code[i];
-        const Nb0 nb = mg_nb0(L, per, cx, cy, cz, i);
-        float sx = 0.0f;
-#pragma unroll
-        for (int m = 0; m < 6; ++m) sx += x[nb.j[m]];
-        const float v = r[i] - __fmaf_rn((float)d, x[i], -sx);
-        s += (inside && d != 0u) ? v : 0.0f;
-    }
-    rc[I] = s;
-}
-
-// A coarser level l >= 1 on the way down (V(1,1)): the pre-smoothing x1 = w D^-1 r is formed on the
-// fly, so one launch gives rc_I = sum of (r - A x1)_i over the cells i of aggregate I on level l + 1.
-// Grid: 8 threads per aggregate.
-__global__ __launch_bounds__(kBlock) void mg_down_kernel(MgLevel L, MgLevel C, uint32_t per, const float* __restrict__ r,
-                                                         float* __restrict__ rc, const PcgStatus* status) {
-    if (status->stop) return;
-    const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
-    if ((t >> 3) >= C.n) return;   // whole groups of 8 leave together
-    uint32_t I, i;
-    int q[3];
-    float v = 0.0f;
-    if (mg_child(L, C, t, I, q, i)) {
-        const float aii = L.diag[i];
-        if (aii > 0.0f) {
-            auto x1 = [&](uint32_t j, const int (&)[3]) { return kOmegaC * L.idiag[j] * r[j]; };
-            const float ax = __fmaf_rn(aii, x1(i, q), mg_offdiag<false>(L, per, q[0], q[1], q[2], i, x1));
-            v = r[i] - ax;
-        }
-    }
-    v = mg_group8_sum(v);
-    if ((t & 7u) == 0u) rc[I] = v;
-}
-
-// A coarser level l >= 1 on the way up: xc = w D^-1 r + over P e (the pre-smoothed iterate plus the
-// prolonged correction, both formed on the fly), then one sweep z = xc + w D^-1 (r - A xc).
-__global__ __launch_bounds__(kBlock) void mg_up_kernel(MgLevel L, MgLevel C, uint32_t per, const float* __restrict__ r,
-                                                       const float* __restrict__ e, float* __restrict__ z, const PcgStatus* status) {
-    if (status->stop) return;
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
-    if (i >= L.n) return;
-    const float aii = L.diag[i];
-    if (!(aii > 0.0f)) {
-        z[i] = 0.0f;
-        return;
-    }
-    int cx, cy, cz;
-    mg_coords(L, i, cx, cy, cz);
-    auto xc = [&](uint32_t j, const int (&q)[3]) {
-        const float inv = L.idiag[j];
-        return inv > 0.0f ? __fmaf_rn(kOverC, e[mg_parent(C, q)], kOmegaC * inv * r[j]) : 0.0f;
+// A box of cells handled by a workgroup of T threads. With a halo of H cells its planes are
+// X(H) x Y(H) points, Z(H) of them. A thread owns one column (x, y) of the halo-2 planes for the whole
+// kernel and walks z: coordinates, wraps and bounds of x and y are formed once per box, those of z are
+// uniform, and a column's own values and its z neighbours stay in registers; LDS serves the four
+// neighbours in the plane. (One thread per tile element, decoding each, took 3.5 times the
+// instructions and 63 instead of 32 us for the down kernel at 128^3.)
+template <int BX_, int BY_, int BZ_, int T_>
+struct Box {
+    static constexpr int BX = BX_, BY = BY_, BZ = BZ_, T = T_;
+    template <int H>
+    static constexpr int X = BX + 2 * H;
+    template <int H>
+    static constexpr int Y = BY + 2 * H;
+    template <int H>
+    static constexpr int Z = BZ + 2 * H;
+    template <int H>
+    static constexpr int P = X<H> * Y<H>;
+    static_assert(T % 64 == 0 && T >= P<2>, "one column per thread");
+    struct Grid {   // the boxes that cover a level
+        uint32_t nx, ny, count;
     };
-    const int c[3]{cx, cy, cz};
-    const float xi = xc(i, c);
-    const float axc = __fmaf_rn(aii, xi, mg_offdiag<false>(L, per, cx, cy, cz, i, xc));
-    z[i] = __fmaf_rn(kOmegaC * L.idiag[i], r[i] - axc, xi);
-}
-
-// Level 0 on the way up, first sweep, with the prolonged correction applied on the fly:
-// xc = x + over P e, y = xc + w D^-1 (r - A xc).
-__global__ __launch_bounds__(kBlock) void mg_post0_kernel(MgLevel L, MgLevel C, uint32_t per, const float* __restrict__ r,
-                                                          const float* __restrict__ x, const float* __restrict__ e, float* __restrict__ y,
-                                                          const PcgStatus* status) {
-    if (status->stop) return;
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
-    if (i >= L.n) return;
-    const uint32_t d = L.code[i];
-    if (d == 0u) {
-        y[i] = 0.0f;
-        return;
+    static __host__ __device__ Grid grid(const MgLevel& L) {
+        const uint32_t nx = (uint32_t)(L.nx + BX - 1) / BX, ny = (uint32_t)(L.ny + BY - 1) / BY;
+        return Grid{nx, ny, nx * ny * ((uint32_t)(L.nz + BZ - 1) / BZ)};
     }
-    int cx, cy, cz;
-    mg_coords(L, i, cx, cy, cz);
-    const Nb0 nb = mg_nb0(L, per, cx, cy, cz, i);
-    uint32_t P[6];
-    const uint32_t Pi = mg_nb0_parents(L, C, per, cx, cy, cz, P);
-    float sx = 0.0f;
+    static __device__ __forceinline__ void origin(const Grid& g, uint32_t b, int& x, int& y, int& z) {
+        const uint32_t r = b / g.nx;
+        x = (int)(b - r * g.nx) * BX;
+        const uint32_t q = r / g.ny;
+        y = (int)(r - q * g.ny) * BY;
+        z = (int)q * BZ;
+    }
+};
+// Level 0 (large, medium, small grids) and the coarser levels (large, small). 32 x 8 x 8 keeps the
+// halo's share of the work low (2.5 times the cells with a halo of 2); smaller boxes fill the 256 CUs
+// of a small grid.
+using BoxL = Box<32, 8, 8, 448>;
+using BoxM = Box<16, 8, 4, 256>;
+using BoxS = Box<16, 4, 4, 192>;
+using BoxC = Box<16, 8, 8, 256>;
+using BoxD = Box<8, 8, 4, 192>;
+
+// Column (x, y) of a level, wrapped along the periodic axes: its offset in a plane, and whether it
+// lies in the grid and is the thread's to handle (the offset is 0 when not).
+struct Column {
+    uint32_t at;
+    bool in;
+};
+__device__ __forceinline__ Column mg_column(const MgLevel& L, uint32_t per, int x, int y, bool mine = true) {
+    if (per & 1u) x = wrapi(x, L.nx);
+    if (per & 2u) y = wrapi(y, L.ny);
+    Column c;
+    c.in = mine && (unsigned)x < (unsigned)L.nx && (unsigned)y < (unsigned)L.ny;
+    c.at = c.in ? (uint32_t)x + __umul24((uint32_t)y, (uint32_t)L.nx) : 0u;
+    return c;
+}
+// N consecutive planes of a level from z0 on (uniform over the workgroup), wrapped along a periodic
+// axis: first elements, and the set that lies in the grid (offset 0 else). Formed once per box: the
+// scalar unit's instructions bound these kernels when every access formed its own.
+template <int N>
+struct Planes {
+    uint32_t at[N], in;
+};
+template <int N>
+__device__ __forceinline__ Planes<N> mg_planes(const MgLevel& L, uint32_t per, int z0) {
+    Planes<N> p;
+    p.in = 0u;
+    const uint32_t stride = (uint32_t)L.nx * (uint32_t)L.ny;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const uint32_t j = nb.j[k];
-        sx += L.code[j] ? __fmaf_rn(kOver0, e[P[k]], x[j]) : 0.0f;
+    for (int k = 0; k < N; ++k) {
+        int z = z0 + k;
+        if (per & 4u) z = wrapi(z, L.nz);
+        const bool in = (unsigned)z < (unsigned)L.nz;
+        p.at[k] = in ? (uint32_t)z * stride : 0u;
+        p.in |= in ? 1u << k : 0u;
     }
-    const float xi = __fmaf_rn(kOver0, e[Pi], x[i]);
-    const float axc = __fmaf_rn((float)d, xi, -sx);
-    y[i] = __fmaf_rn(mg_wdinv(d), r[i] - axc, xi);
+    return p;
+}
+// Element i of v. The byte offset stays a 32-bit register beside a uniform base (a level has at most
+// 2^30 cells of 4 bytes).
+template <typename V>
+__device__ __forceinline__ V& mg_at(V* v, uint32_t i) {
+    return *reinterpret_cast<V*>(reinterpret_cast<std::conditional_t<std::is_const_v<V>, const char, char>*>(v) + i * (uint32_t)sizeof(V));
+}
+template <typename V, int N>
+__device__ __forceinline__ V mg_load(const V* __restrict__ v, const Planes<N>& p, int k, const Column& c) {
+    const V l = mg_at(v, c.at + p.at[k]);
+    return (p.in >> k & 1u) && c.in ? l : (V)0;
 }
 
-// Level 0, second sweep z = y + w D^-1 (r - A y), over contiguous block ranges, with the partials of
-// <r, z>.
-__global__ __launch_bounds__(kMgThreads) void mg_post0_last_kernel(MgLevel L, uint32_t per, const float* __restrict__ r,
-                                                                   const float* __restrict__ y, float* __restrict__ z,
-                                                                   double* __restrict__ partials, const PcgStatus* status) {
+struct Pair2 {   // double-buffered vector: iteration k's value is p[k & 1]
+    float* p[2];
+};
+
+// The aggregates' values over N planes of a column, from plane z0 (even) of the finer level on (nz its
+// planes): one aggregate serves two planes unless a periodic axis wraps in between.
+template <int N>
+__device__ __forceinline__ void mg_load_coarse(const MgLevel& C, uint32_t per, int z0, int nz, const float* __restrict__ e, const Column& cc,
+                                               float (&v)[N]) {
+    const uint32_t stride = (uint32_t)C.nx * (uint32_t)C.ny;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        if ((k & 1) == 0 || (per & 4u)) {
+            int z = z0 + k;
+            if (per & 4u) z = wrapi(z, nz);
+            const bool in = (unsigned)z < (unsigned)nz;
+            const float l = mg_at(e, cc.at + (in ? (uint32_t)(z >> 1) * stride : 0u));
+            v[k] = in && cc.in ? l : 0.0f;
+        } else {
+            v[k] = v[k - 1];
+        }
+    }
+}
+
+// In-plane neighbours of LDS element i of planes X wide.
+template <int X>
+__device__ __forceinline__ float mg_plane_sum(const float* v, int i) {
+    return (v[i - 1] + v[i + 1]) + (v[i - X] + v[i + X]);
+}
+
+// Level 0 on the way down, with the PCG update of the iteration fused in front (Update): alpha =
+// rz / <p, A p>; x += alpha p; r' = r - alpha A p, partials of ||r'||^2 (r is double-buffered: the
+// neighbouring boxes read the old one). The solution pair (hi + lo, about 48 bits) takes alpha p in
+// FP64 and A p is formed in FP64 from p, exactly as the direction kernel forms it, so the recursive
+// residual follows the true one to FP32 rounding of r itself: with the near-null mode of the matrix
+// the solution is some 10^3 ||b|| large, and an FP32 increment (or an FP32 A p) would leave a gap of
+// about 1e-4 ||b|| between them after the first, largest steps.
+// Then (Smooth) the two sweeps from zero for A x = r' and the restriction of r' - A x to level 1.
+template <typename B, bool Update, bool Smooth>
+__global__ __launch_bounds__(B::T) void mg_down0_kernel(MgLevel L, MgLevel C, uint32_t per, Pair2 r, Pair2 p, float* __restrict__ xh,
+                                                        float* __restrict__ xl, float* __restrict__ x, float* __restrict__ rc,
+                                                        double* __restrict__ partials, const double* __restrict__ hist,
+                                                        const PcgStatus* status) {
+    constexpr int X3 = B::template X<3>, X2 = B::template X<2>, X1 = B::template X<1>;
+    constexpr int P3 = B::template P<3>, P2 = B::template P<2>, P1 = B::template P<1>;
+    constexpr int Z3 = B::template Z<3>, Z2 = B::template Z<2>, Z1 = B::template Z<1>;
+    constexpr int kPasses = (P3 + B::T - 1) / B::T;
+    __shared__ float sp[P3 * Z3];   // p, then the first sweep's iterate, then the residual's z pairs
+    __shared__ float sx[P1 * Z1];
     __shared__ double lds[kMaxWaves];
     if (status->stop) return;
-    uint32_t lb, start, end;
-    mg_range(L.n, lb, start, end);
-    double rz = 0.0;
-    for (uint32_t base = start + threadIdx.x; base < end; base += kMgUnroll * blockDim.x) {
+    const uint32_t k = status->k;
+    const float* __restrict__ r_in = r.p[k & 1u];
+    float* __restrict__ r_out = r.p[(k + 1u) & 1u];
+    const float* __restrict__ pk = p.p[k & 1u];
+    const int t = (int)threadIdx.x;
+    const uint32_t lb = xcd_block();
+    const typename B::Grid grid = B::grid(L);
+    const uint32_t first = (uint32_t)((uint64_t)grid.count * lb / gridDim.x), last = (uint32_t)((uint64_t)grid.count * (lb + 1u) / gridDim.x);
+    const int cy = t / X2, cx = t - cy * X2;   // column in the halo-2 planes
+    const bool mine2 = t < P2;
+    const bool mine1 = mine2 && cx >= 1 && cx < X2 - 1 && cy >= 1 && cy < B::template Y<2> - 1;
+    const bool mine0 = mine2 && cx >= 2 && cx < X2 - 2 && cy >= 2 && cy < B::template Y<2> - 2;
+    const int i3 = (cy + 1) * X3 + cx + 1, i1 = (cy - 1) * X1 + cx - 1;   // the column's element in a plane
+    double alpha = 0.0, rr = 0.0;
+    bool have_alpha = false;
+    for (uint32_t b = first; b < last; ++b) {
+        int x0, y0, z0;
+        B::origin(grid, b, x0, y0, z0);
+        const Planes<Z3> pl3 = mg_planes<Z3>(L, per, z0 - 3);
+        if (Update) {
 #pragma unroll
-        for (int m = 0; m < kMgUnroll; ++m) {
-            const uint32_t i0 = base + (uint32_t)m * blockDim.x;
-            const bool valid = i0 < end;
-            const uint32_t i = min(i0, L.n - 1u);
-            const uint32_t d = L.code[i];
-            int cx, cy, cz;
-            mg_coords(L, i, cx, cy, cz);
-            const Nb0 nb = mg_nb0(L, per, cx, cy, cz, i);
-            float sy = 0.0f;
+            for (int s = 0; s < kPasses; ++s) {
+                const int e = s * B::T + t;
+                const int ey = e / X3, ex = e - ey * X3;
+                const Column c = mg_column(L, per, x0 - 3 + ex, y0 - 3 + ey);
+                if (e < P3) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) sy += y[nb.j[k]];
-            const float yi = y[i], ri = r[i];
-            const float zi = d ? __fmaf_rn(mg_wdinv(d), ri - __fmaf_rn((float)d, yi, -sy), yi) : 0.0f;
-            if (valid) z[i] = zi;
-            rz = valid ? __fma_rn((double)ri, (double)zi, rz) : rz;
+                    for (int z = 0; z < Z3; ++z) sp[z * P3 + e] = mg_load(pk, pl3, z, c);
+                }
+            }
         }
+        const Column c = mg_column(L, per, x0 - 2 + cx, y0 - 2 + cy, mine2);
+        float rv[Z2];
+        uint32_t dv[Z2];
+#pragma unroll
+        for (int z = 0; z < Z2; ++z) {
+            rv[z] = mg_load(r_in, pl3, z + 1, c);
+            dv[z] = mg_load(L.code, pl3, z + 1, c);
+        }
+        if (Update && !have_alpha) {
+            const double* parts[1]{partials + kPartPQ * kPcgMaxBlocks};
+            double red[1];
+            reduce_partials<1>(parts, gridDim.x, red, lds);
+            alpha = hist[2 * k] / red[0];
+            have_alpha = true;
+        }
+        const bool own = mine0 && x0 - 2 + cx < L.nx && y0 - 2 + cy < L.ny;   // the box's own cells (not wrapped ones)
+        if (Update) {
+            __syncthreads();
+            if (mine2) {
+                double lo = (double)sp[i3], mid = (double)sp[P3 + i3];
+#pragma unroll
+                for (int z = 0; z < Z2; ++z) {
+                    const float* pl = sp + (z + 1) * P3;
+                    const double hi = (double)pl[P3 + i3];
+                    const double around = ((double)pl[i3 - 1] + (double)pl[i3 + 1]) + ((double)pl[i3 - X3] + (double)pl[i3 + X3]) + (lo + hi);
+                    const double q = (double)dv[z] * mid - around;
+                    const float rn = dv[z] ? (float)__fma_rn(-alpha, q, (double)rv[z]) : 0.0f;
+                    rv[z] = rn;
+                    if (z >= 2 && z < Z2 - 2) {
+                        const uint32_t i = c.at + pl3.at[z + 1];
+                        if (own && z0 - 2 + z < L.nz) {
+                            mg_at(r_out, i) = rn;
+                            rr = __fma_rn((double)rn, (double)rn, rr);
+                            if (dv[z]) {
+                                float &h = mg_at(xh, i), &l = mg_at(xl, i);
+                                const double xv = __fma_rn(alpha, mid, (double)h + (double)l);
+                                const float hi32 = (float)xv;
+                                h = hi32;
+                                l = (float)(xv - (double)hi32);
+                            }
+                        }
+                    }
+                    lo = mid;
+                    mid = hi;
+                }
+            }
+            __syncthreads();   // p is done with
+        }
+        if (Smooth) {
+            // first sweep, x1 = w D^-1 r, into LDS (planes P2)
+            if (mine2) {
+#pragma unroll
+                for (int z = 0; z < Z2; ++z) sp[z * P2 + t] = kCheb[0] * mg_dinv(dv[z]) * rv[z];
+            }
+            __syncthreads();
+            float x2[Z1];
+            if (mine1) {
+                float lo = sp[t], mid = sp[P2 + t];
+#pragma unroll
+                for (int z = 0; z < Z1; ++z) {
+                    const float hi = sp[(z + 2) * P2 + t];
+                    const uint32_t d = dv[z + 1];
+                    const float sum = mg_plane_sum<X2>(sp + (z + 1) * P2, t) + (lo + hi);
+                    const float res = rv[z + 1] - __fmaf_rn((float)d, mid, -sum);
+                    x2[z] = d ? __fmaf_rn(kCheb[1] * mg_dinv(d), res, mid) : 0.0f;
+                    sx[z * P1 + i1] = x2[z];
+                    lo = mid;
+                    mid = hi;
+                }
+            }
+            __syncthreads();
+            // x stored, the residual's sums over z pairs into LDS
+            if (mine0) {
+#pragma unroll
+                for (int z = 0; z < B::BZ; z += 2) {
+                    float pair = 0.0f;
+#pragma unroll
+                    for (int m = z; m < z + 2; ++m) {
+                        const bool in = own && z0 + m < L.nz;
+                        if (in) mg_at(x, c.at + pl3.at[m + 3]) = x2[m + 1];
+                        const uint32_t d = dv[m + 2];
+                        const float sum = mg_plane_sum<X1>(sx + (m + 1) * P1, i1) + (x2[m] + x2[m + 2]);
+                        const float res = rv[m + 2] - __fmaf_rn((float)d, x2[m + 1], -sum);
+                        // (beyond an odd extent a periodic axis wraps: not a cell of this aggregate)
+                        pair += d && in ? res : 0.0f;
+                    }
+                    sp[(z / 2) * (B::BX * B::BY) + (cy - 2) * B::BX + cx - 2] = pair;
+                }
+            }
+            __syncthreads();
+            constexpr int CX = B::BX / 2, CY = B::BY / 2;
+            for (int I = t; I < CX * CY * (B::BZ / 2); I += B::T) {
+                const int lx = I % CX, ly = I / CX % CY, lz = I / (CX * CY);
+                const float* v = sp + lz * (B::BX * B::BY) + 2 * ly * B::BX + 2 * lx;
+                const int gX = (x0 >> 1) + lx, gY = (y0 >> 1) + ly, gZ = (z0 >> 1) + lz;
+                if (gX < C.nx && gY < C.ny && gZ < C.nz)
+                    rc[lattice_index(gX, gY, gZ, C.nx, C.ny)] = (v[0] + v[1]) + (v[B::BX] + v[B::BX + 1]);
+            }
+            __syncthreads();   // the next box reuses the tiles
+        }
+    }
+    if (Update) {
+        double v[1]{rr};
+        block_sum<1>(v, lds);
+        if (t == 0) partials[kPartRR * kPcgMaxBlocks + lb] = v[0];
+    }
+}
+
+// Level 0 on the way up: xc = x + over P e (x the pre-smoothed iterate), the two sweeps in the
+// reverse order, z, partials of <r, z>.
+template <typename B>
+__global__ __launch_bounds__(B::T) void mg_post0_kernel(MgLevel L, MgLevel C, uint32_t per, Pair2 r, const float* __restrict__ x,
+                                                        const float* __restrict__ e_c, float* __restrict__ z_out, double* __restrict__ partials,
+                                                        const PcgStatus* status) {
+    constexpr int X2 = B::template X<2>, X1 = B::template X<1>, P2 = B::template P<2>, P1 = B::template P<1>;
+    constexpr int Z2 = B::template Z<2>, Z1 = B::template Z<1>;
+    __shared__ float sx[P2 * Z2];
+    __shared__ float sy[P1 * Z1];
+    __shared__ double lds[kMaxWaves];
+    if (status->stop) return;
+    const float* __restrict__ rk = r.p[status->k & 1u];
+    const int t = (int)threadIdx.x;
+    const uint32_t lb = xcd_block();
+    const typename B::Grid grid = B::grid(L);
+    const uint32_t first = (uint32_t)((uint64_t)grid.count * lb / gridDim.x), last = (uint32_t)((uint64_t)grid.count * (lb + 1u) / gridDim.x);
+    const int cy = t / X2, cx = t - cy * X2;
+    const bool mine2 = t < P2;
+    const bool mine1 = mine2 && cx >= 1 && cx < X2 - 1 && cy >= 1 && cy < B::template Y<2> - 1;
+    const bool mine0 = mine2 && cx >= 2 && cx < X2 - 2 && cy >= 2 && cy < B::template Y<2> - 2;
+    const int i1 = (cy - 1) * X1 + cx - 1;
+    double rz = 0.0;
+    for (uint32_t b = first; b < last; ++b) {
+        int x0, y0, z0;
+        B::origin(grid, b, x0, y0, z0);
+        const Column c = mg_column(L, per, x0 - 2 + cx, y0 - 2 + cy, mine2);
+        const uint32_t gy = c.at / (uint32_t)L.nx, gx = c.at - gy * (uint32_t)L.nx;
+        const Column cc{(gx >> 1) + __umul24(gy >> 1, (uint32_t)C.nx), c.in};   // the column's aggregate
+        const Planes<Z2> pl2 = mg_planes<Z2>(L, per, z0 - 2);
+        float xv[Z2], rv[Z1];
+        uint32_t dv[Z2];
+#pragma unroll
+        for (int z = 0; z < Z2; ++z) {
+            dv[z] = mg_load(L.code, pl2, z, c);
+            xv[z] = mg_load(x, pl2, z, c);
+        }
+        float ev[Z2];
+        mg_load_coarse<Z2>(C, per, z0 - 2, L.nz, e_c, cc, ev);
+#pragma unroll
+        for (int z = 0; z < Z2; ++z) xv[z] = dv[z] ? __fmaf_rn(kOver, ev[z], xv[z]) : 0.0f;
+#pragma unroll
+        for (int z = 0; z < Z1; ++z) rv[z] = mg_load(rk, pl2, z + 1, c);
+        if (mine2) {
+#pragma unroll
+            for (int z = 0; z < Z2; ++z) sx[z * P2 + t] = xv[z];
+        }
+        __syncthreads();
+        float y[Z1];
+        if (mine1) {
+#pragma unroll
+            for (int z = 0; z < Z1; ++z) {
+                const uint32_t d = dv[z + 1];
+                const float sum = mg_plane_sum<X2>(sx + (z + 1) * P2, t) + (xv[z] + xv[z + 2]);
+                const float res = rv[z] - __fmaf_rn((float)d, xv[z + 1], -sum);
+                y[z] = d ? __fmaf_rn(kCheb[1] * mg_dinv(d), res, xv[z + 1]) : 0.0f;
+                sy[z * P1 + i1] = y[z];
+            }
+        }
+        __syncthreads();
+        if (mine0 && x0 - 2 + cx < L.nx && y0 - 2 + cy < L.ny) {
+#pragma unroll
+            for (int z = 0; z < B::BZ; ++z) {
+                const uint32_t d = dv[z + 2];
+                const float ri = rv[z + 1];
+                const float sum = mg_plane_sum<X1>(sy + (z + 1) * P1, i1) + (y[z] + y[z + 2]);
+                const float res = ri - __fmaf_rn((float)d, y[z + 1], -sum);
+                const float zi = d ? __fmaf_rn(kCheb[0] * mg_dinv(d), res, y[z + 1]) : 0.0f;
+                if (z0 + z < L.nz) {
+                    mg_at(z_out, c.at + pl2.at[z + 2]) = zi;
+                    rz = __fma_rn((double)ri, (double)zi, rz);
+                }
+            }
+        }
+        __syncthreads();
     }
     double v[1]{rz};
     block_sum<1>(v, lds);
-    if (threadIdx.x == 0) partials[kPartRZ * kPcgMaxBlocks + lb] = v[0];
+    if (t == 0) partials[kPartRZ * kPcgMaxBlocks + lb] = v[0];
 }
 
-// Coarsest level: x = A^-1 r in FP64, one block per row of the inverse. When level 0 is the coarsest
-// this is the V-cycle's first kernel and advances the iteration index.
-__global__ __launch_bounds__(kBlock) void mg_dense_kernel(uint32_t n, const double* __restrict__ inv, const float* __restrict__ r,
-                                                          float* __restrict__ x, PcgStatus* status, uint32_t advance) {
+// PCG direction of iteration k: beta = rz_k / rz_{k-1} (RZ partials of the V-cycle), p = z + beta p_old
+// (p = z when k = 0), partials of <p, A p> with A p in FP64 (exact, as the update forms it).
+template <typename B>
+__global__ __launch_bounds__(B::T) void mg_direction_kernel(MgLevel L, uint32_t per, const float* __restrict__ z_in, Pair2 p,
+                                                            double* __restrict__ partials, double* __restrict__ hist,
+                                                            const PcgStatus* status) {
+    constexpr int X1 = B::template X<1>, P1 = B::template P<1>, Z1 = B::template Z<1>;
+    __shared__ float sp[P1 * Z1];
     __shared__ double lds[kMaxWaves];
     if (status->stop) return;
-    if (advance && blockIdx.x == 0 && threadIdx.x == 0) status->k = status->k + 1u;
+    const uint32_t k = status->k;
+    float* __restrict__ p_new = p.p[k & 1u];
+    const float* __restrict__ p_old = p.p[(k + 1u) & 1u];
+    const int t = (int)threadIdx.x;
+    const uint32_t lb = xcd_block();
+    const typename B::Grid grid = B::grid(L);
+    const uint32_t first = (uint32_t)((uint64_t)grid.count * lb / gridDim.x), last = (uint32_t)((uint64_t)grid.count * (lb + 1u) / gridDim.x);
+    const int cy = t / X1, cx = t - cy * X1;
+    const bool mine1 = t < P1;
+    const bool mine0 = mine1 && cx >= 1 && cx < X1 - 1 && cy >= 1 && cy < B::template Y<1> - 1;
+    float beta = 0.0f;
+    bool have_beta = false;
+    double pq = 0.0;
+    for (uint32_t b = first; b < last; ++b) {
+        int x0, y0, z0;
+        B::origin(grid, b, x0, y0, z0);
+        const Column c = mg_column(L, per, x0 - 1 + cx, y0 - 1 + cy, mine1);
+        const Planes<Z1> pl1 = mg_planes<Z1>(L, per, z0 - 1);
+        float zv[Z1], pv[Z1];
+        uint32_t dv[B::BZ];
+#pragma unroll
+        for (int z = 0; z < Z1; ++z) {
+            zv[z] = mg_load(z_in, pl1, z, c);
+            pv[z] = k > 0u ? mg_load(p_old, pl1, z, c) : 0.0f;
+        }
+#pragma unroll
+        for (int z = 0; z < B::BZ; ++z) dv[z] = mg_load(L.code, pl1, z + 1, c);
+        if (!have_beta) {
+            const double* parts[1]{partials + kPartRZ * kPcgMaxBlocks};
+            double red[1];
+            reduce_partials<1>(parts, gridDim.x, red, lds);
+            if (b == 0 && t == 0) hist[2 * k] = red[0];   // the block of the first box
+            beta = k > 0u ? (float)(red[0] / hist[2 * (k - 1u)]) : 0.0f;
+            have_beta = true;
+        }
+#pragma unroll
+        for (int z = 0; z < Z1; ++z) {
+            zv[z] = k > 0u ? __fmaf_rn(beta, pv[z], zv[z]) : zv[z];
+            if (mine1) sp[z * P1 + t] = zv[z];
+        }
+        __syncthreads();
+        if (mine0 && x0 - 1 + cx < L.nx && y0 - 1 + cy < L.ny) {
+#pragma unroll
+            for (int z = 0; z < B::BZ; ++z) {
+                const float* pl = sp + (z + 1) * P1;
+                const double pi = (double)zv[z + 1];   // 0 off the unknowns
+                const double around = ((double)pl[t - 1] + (double)pl[t + 1]) + ((double)pl[t - X1] + (double)pl[t + X1]) +
+                                      ((double)zv[z] + (double)zv[z + 2]);
+                if (z0 + z < L.nz) {
+                    mg_at(p_new, c.at + pl1.at[z + 1]) = zv[z + 1];
+                    pq = __fma_rn(pi, (double)dv[z] * pi - around, pq);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    double v[1]{pq};
+    block_sum<1>(v, lds);
+    if (t == 0) partials[kPartPQ * kPcgMaxBlocks + lb] = v[0];
+}
+
+// A row of a coarser level's operator: the + couplings are the cell's own, the - couplings the
+// - neighbours' (along z the previous plane's).
+struct CoarseRow {
+    float diag, xp, xm, yp, ym, zp;
+};
+struct CoarseColumn {   // a column and its - neighbours along x and y
+    Column c, xm, ym;
+};
+__device__ __forceinline__ CoarseColumn mg_coarse_column(const MgLevel& L, uint32_t per, int x, int y, bool mine) {
+    CoarseColumn k{mg_column(L, per, x, y, mine), mg_column(L, per, x - 1, y), mg_column(L, per, x, y - 1)};
+    k.xm.in = k.xm.in && k.c.in;
+    k.ym.in = k.ym.in && k.c.in;
+    return k;
+}
+template <int N>
+__device__ __forceinline__ CoarseRow mg_row(const MgLevel& L, const Planes<N>& p, int z, const CoarseColumn& k) {
+    return CoarseRow{mg_load(L.diag, p, z, k.c),  mg_load(L.wp[0], p, z, k.c),  mg_load(L.wp[0], p, z, k.xm),
+                     mg_load(L.wp[1], p, z, k.c), mg_load(L.wp[1], p, z, k.ym), mg_load(L.wp[2], p, z, k.c)};
+}
+// (A v)_i: v's plane in LDS at pl (element i), its z neighbours lo, mid, hi; zm: the - z coupling.
+template <int X>
+__device__ __forceinline__ float mg_coarse_apply(const CoarseRow& w, float zm, const float* pl, int i, float lo, float mid, float hi) {
+    float s = w.diag * mid;
+    s = __fmaf_rn(w.xp, pl[i + 1], s);
+    s = __fmaf_rn(w.xm, pl[i - 1], s);
+    s = __fmaf_rn(w.yp, pl[i + X], s);
+    s = __fmaf_rn(w.ym, pl[i - X], s);
+    s = __fmaf_rn(w.zp, hi, s);
+    return __fmaf_rn(zm, lo, s);
+}
+
+// A coarser level on the way down: both sweeps from zero, x stored, r - A x restricted.
+template <typename B>
+__global__ __launch_bounds__(B::T) void mg_down_kernel(MgLevel L, MgLevel C, uint32_t per, const float* __restrict__ r,
+                                                       float* __restrict__ x, float* __restrict__ rc, const PcgStatus* status) {
+    constexpr int X2 = B::template X<2>, X1 = B::template X<1>, P2 = B::template P<2>, P1 = B::template P<1>;
+    constexpr int Z2 = B::template Z<2>, Z1 = B::template Z<1>;
+    __shared__ float s1[P2 * Z2], sx[P1 * Z1];
+    if (status->stop) return;
+    const int t = (int)threadIdx.x;
+    const typename B::Grid grid = B::grid(L);
+    const uint32_t b = xcd_block();
+    if (b >= grid.count) return;
+    const int cy = t / X2, cx = t - cy * X2;
+    const bool mine2 = t < P2;
+    const bool mine1 = mine2 && cx >= 1 && cx < X2 - 1 && cy >= 1 && cy < B::template Y<2> - 1;
+    const bool mine0 = mine2 && cx >= 2 && cx < X2 - 2 && cy >= 2 && cy < B::template Y<2> - 2;
+    const int i1 = (cy - 1) * X1 + cx - 1;
+    int x0, y0, z0;
+    B::origin(grid, b, x0, y0, z0);
+    const CoarseColumn k = mg_coarse_column(L, per, x0 - 2 + cx, y0 - 2 + cy, mine2);
+    const Planes<Z2> pl2 = mg_planes<Z2>(L, per, z0 - 2);
+    float rv[Z2], iv[Z2], x1[Z2];
+#pragma unroll
+    for (int z = 0; z < Z2; ++z) {
+        rv[z] = mg_load(r, pl2, z, k.c);
+        iv[z] = mg_load(L.idiag, pl2, z, k.c);
+    }
+    CoarseRow w[Z1];
+    const float zm0 = mg_load(L.wp[2], pl2, 0, k.c);
+#pragma unroll
+    for (int z = 0; z < Z1; ++z) w[z] = mg_row(L, pl2, z + 1, k);
+#pragma unroll
+    for (int z = 0; z < Z2; ++z) {
+        x1[z] = kCheb[0] * iv[z] * rv[z];   // 0 off the unknowns (1 / diag is 0 there)
+        if (mine2) s1[z * P2 + t] = x1[z];
+    }
+    __syncthreads();
+    float x2[Z1];
+    if (mine1) {
+#pragma unroll
+        for (int z = 0; z < Z1; ++z) {
+            const float ax = mg_coarse_apply<X2>(w[z], z ? w[z ? z - 1 : 0].zp : zm0, s1 + (z + 1) * P2, t, x1[z], x1[z + 1], x1[z + 2]);
+            x2[z] = __fmaf_rn(kCheb[1] * iv[z + 1], rv[z + 1] - ax, x1[z + 1]);
+            sx[z * P1 + i1] = x2[z];
+        }
+    }
+    __syncthreads();
+    if (mine0) {
+        const bool own = x0 - 2 + cx < L.nx && y0 - 2 + cy < L.ny;
+#pragma unroll
+        for (int z = 0; z < B::BZ; z += 2) {
+            float pair = 0.0f;
+#pragma unroll
+            for (int m = z; m < z + 2; ++m) {
+                const bool in = own && z0 + m < L.nz;
+                if (in) mg_at(x, k.c.at + pl2.at[m + 2]) = x2[m + 1];
+                const float ax = mg_coarse_apply<X1>(w[m + 1], w[m].zp, sx + (m + 1) * P1, i1, x2[m], x2[m + 1], x2[m + 2]);
+                pair += in && iv[m + 2] > 0.0f ? rv[m + 2] - ax : 0.0f;
+            }
+            s1[(z / 2) * (B::BX * B::BY) + (cy - 2) * B::BX + cx - 2] = pair;   // (every read of s1 is behind the barrier)
+        }
+    }
+    __syncthreads();
+    constexpr int CX = B::BX / 2, CY = B::BY / 2;
+    for (int I = t; I < CX * CY * (B::BZ / 2); I += B::T) {
+        const int lx = I % CX, ly = I / CX % CY, lz = I / (CX * CY);
+        const float* v = s1 + lz * (B::BX * B::BY) + 2 * ly * B::BX + 2 * lx;
+        const int gX = (x0 >> 1) + lx, gY = (y0 >> 1) + ly, gZ = (z0 >> 1) + lz;
+        if (gX < C.nx && gY < C.ny && gZ < C.nz) rc[lattice_index(gX, gY, gZ, C.nx, C.ny)] = (v[0] + v[1]) + (v[B::BX] + v[B::BX + 1]);
+    }
+}
+
+// A coarser level on the way up: xc = x + over P e, the two sweeps in the reverse order.
+template <typename B>
+__global__ __launch_bounds__(B::T) void mg_up_kernel(MgLevel L, MgLevel C, uint32_t per, const float* __restrict__ r,
+                                                     const float* __restrict__ x, const float* __restrict__ e_c, float* __restrict__ z_out,
+                                                     const PcgStatus* status) {
+    constexpr int X2 = B::template X<2>, X1 = B::template X<1>, P2 = B::template P<2>, P1 = B::template P<1>;
+    constexpr int Z2 = B::template Z<2>, Z1 = B::template Z<1>;
+    __shared__ float sx[P2 * Z2], sy[P1 * Z1];
+    if (status->stop) return;
+    const int t = (int)threadIdx.x;
+    const typename B::Grid grid = B::grid(L);
+    const uint32_t b = xcd_block();
+    if (b >= grid.count) return;
+    const int cy = t / X2, cx = t - cy * X2;
+    const bool mine2 = t < P2;
+    const bool mine1 = mine2 && cx >= 1 && cx < X2 - 1 && cy >= 1 && cy < B::template Y<2> - 1;
+    const bool mine0 = mine2 && cx >= 2 && cx < X2 - 2 && cy >= 2 && cy < B::template Y<2> - 2;
+    const int i1 = (cy - 1) * X1 + cx - 1;
+    int x0, y0, z0;
+    B::origin(grid, b, x0, y0, z0);
+    const CoarseColumn k = mg_coarse_column(L, per, x0 - 2 + cx, y0 - 2 + cy, mine2);
+    const uint32_t gy = k.c.at / (uint32_t)L.nx, gx = k.c.at - gy * (uint32_t)L.nx;
+    const Column cc{(gx >> 1) + __umul24(gy >> 1, (uint32_t)C.nx), k.c.in};
+    const Planes<Z2> pl2 = mg_planes<Z2>(L, per, z0 - 2);
+    float xv[Z2], iv[Z2], ev[Z2], rv[Z1];
+#pragma unroll
+    for (int z = 0; z < Z2; ++z) {
+        iv[z] = mg_load(L.idiag, pl2, z, k.c);
+        xv[z] = mg_load(x, pl2, z, k.c);
+    }
+    mg_load_coarse<Z2>(C, per, z0 - 2, L.nz, e_c, cc, ev);
+    CoarseRow w[Z1];
+    const float zm0 = mg_load(L.wp[2], pl2, 0, k.c);
+#pragma unroll
+    for (int z = 0; z < Z1; ++z) {
+        w[z] = mg_row(L, pl2, z + 1, k);
+        rv[z] = mg_load(r, pl2, z + 1, k.c);
+    }
+#pragma unroll
+    for (int z = 0; z < Z2; ++z) xv[z] = iv[z] > 0.0f ? __fmaf_rn(kOver, ev[z], xv[z]) : 0.0f;
+    if (mine2) {
+#pragma unroll
+        for (int z = 0; z < Z2; ++z) sx[z * P2 + t] = xv[z];
+    }
+    __syncthreads();
+    float y[Z1];
+    if (mine1) {
+#pragma unroll
+        for (int z = 0; z < Z1; ++z) {
+            const float ax = mg_coarse_apply<X2>(w[z], z ? w[z ? z - 1 : 0].zp : zm0, sx + (z + 1) * P2, t, xv[z], xv[z + 1], xv[z + 2]);
+            y[z] = __fmaf_rn(kCheb[1] * iv[z + 1], rv[z] - ax, xv[z + 1]);
+            sy[z * P1 + i1] = y[z];
+        }
+    }
+    __syncthreads();
+    if (mine0 && x0 - 2 + cx < L.nx && y0 - 2 + cy < L.ny) {
+#pragma unroll
+        for (int z = 0; z < B::BZ; ++z) {
+            const float ax = mg_coarse_apply<X1>(w[z + 1], w[z].zp, sy + (z + 1) * P1, i1, y[z], y[z + 1], y[z + 2]);
+            if (z0 + z < L.nz) mg_at(z_out, k.c.at + pl2.at[z + 2]) = __fmaf_rn(kCheb[0] * iv[z + 2], rv[z + 1] - ax, y[z + 1]);
+        }
+    }
+}
+
+// ---- the levels that one workgroup handles ------------------------------------------------------
+
+// A cell of such a level, as the host lays it out (kBottomWords arrays of n words per level): its row
+// of the operator, its neighbours' indices (two per word, in the order -x, +x, -y, ...), its
+// aggregate's index on the next level; and for cell I of the next level its first child's index with
+// a bit per existing child (-1: not used). One CU runs this kernel, and the instructions to form
+// these in place took most of its time.
+struct BottomCell {
+    float diag, idiag, w[6];
+    uint32_t nb[3], parent;
+};
+__device__ __forceinline__ BottomCell mg_bottom_cell(const uint32_t* __restrict__ words, uint32_t n, uint32_t i) {
+    BottomCell c;
+    c.diag = __uint_as_float(words[i]);
+    c.idiag = __uint_as_float(words[n + i]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) c.w[k] = __uint_as_float(words[(2 + k) * n + i]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) c.nb[k] = words[(8 + k) * n + i];
+    c.parent = words[11 * n + i];
+    return c;
+}
+__device__ __forceinline__ float mg_bottom_apply(const BottomCell& c, const float* v, float own) {
+    float s = c.diag * own;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        s = __fmaf_rn(c.w[2 * a], v[c.nb[a] & 0xffffu], s);
+        s = __fmaf_rn(c.w[2 * a + 1], v[c.nb[a] >> 16], s);
+    }
+    return s;
+}
+
+// The stopping test of an iteration (or of the initial residual), then the V-cycle of the levels of
+// at most kMgBottomCells cells in one workgroup: vectors in LDS, the rows of the first two levels in
+// registers, and the coarsest level's inverse (n x n, FP64, n <= kMgDense) spread over the threads.
+// Levels: how many (the last is the dense one; 0: only the test).
+// mode: bit 0 the iteration index advances (the update of iteration k ran before), bit 1 the first
+// test of a solve (||b||^2 from its partials, the initial residual kept), bit 2 the guess is rejected
+// when its residual exceeds ||b||, bit 3 when it is not finite. A rejection stops the solve: the
+// host, which reads the status once at its end, runs it again without the guess.
+constexpr int kBottomThreads = 1024;
+constexpr int kBottomWords = 13;
+template <int Levels>
+__global__ __launch_bounds__(kBottomThreads) void mg_bottom_kernel(MgBottom B, const float* __restrict__ r,
+                                                                   float* __restrict__ out, const double* __restrict__ partials,
+                                                                   uint32_t blocks, PcgStatus* status, double tol2, uint32_t mode) {
+    constexpr int T = kBottomThreads, last = Levels - 1;
+    __shared__ float vr[Levels ? kMgBottomLds : 1], vx[Levels ? kMgBottomLds : 1], vy[Levels ? kMgBottomLds : 1];
+    __shared__ double lds[(T / 64) * kMgDense];
+    if (status->stop) return;
+    const uint32_t t = threadIdx.x;
+    const uint32_t k = status->k + (mode & 1u);
+    const double bb0 = status->bb;
+    // everything the cycle reads from memory, up front
+    BottomCell c0[4], c1[2];
+    double inv[4];
+    if constexpr (last >= 0) {
+        for (uint32_t i = t; i < B.n[0]; i += T) vr[i] = r[i];
+        const uint32_t n = B.n[last];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const uint32_t j = (t >> 6) + 16u * m;
+            inv[m] = (t & 63u) < n && j < n ? B.dense[j * n + (t & 63u)] : 0.0;
+        }
+    }
+    if constexpr (last >= 1) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            if (t + m * T < B.n[0]) c0[m] = mg_bottom_cell(B.words[0], B.n[0], t + m * T);
+    }
+    if constexpr (last >= 2) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            if (t + m * T < B.n[1]) c1[m] = mg_bottom_cell(B.words[1], B.n[1], t + m * T);
+    }
+    const bool opening = mode & 2u;
+    double red[2]{0.0, 0.0};
+    for (uint32_t i = t; i < blocks; i += T) {
+        red[0] += partials[kPartRR * kPcgMaxBlocks + i];
+        if (opening) red[1] += partials[kPartBB * kPcgMaxBlocks + i];
+    }
+    block_sum<2>(red, lds);
+    const double rr = red[0], bb = opening ? red[1] : bb0;
+    const bool finite = isfinite(rr);
+    const bool rejected = ((mode & 4u) && !(finite && rr <= bb)) || ((mode & 8u) && !finite);
+    const bool stop = rejected || !(rr > tol2 * bb);
+    if (t == 0) {
+        status->k = k;
+        status->rr = rr;
+        status->iterations = k;
+        if (opening) {
+            status->bb = bb;
+            status->rr0 = rr;
+        }
+        if (rejected) status->rejected = 1u;
+        if (stop) status->stop = 1u;
+    }
+    if (stop) return;
+    if constexpr (last >= 0) {
+        // f(row, cell) over the cells of level l
+        auto cells = [&]<int l>(auto&& f) {
+            if constexpr (l == 0) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    if (t + m * T < B.n[0]) f(c0[m], t + m * T);
+            } else if constexpr (l == 1) {
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    if (t + m * T < B.n[1]) f(c1[m], t + m * T);
+            } else {
+                for (uint32_t i = t; i < B.n[l]; i += T) f(mg_bottom_cell(B.words[l], B.n[l], i), i);
+            }
+        };
+        auto down = [&]<int l>() {
+            float *rl = vr + B.off[l], *xl = vx + B.off[l], *yl = vy + B.off[l];
+            cells.template operator()<l>([&](const BottomCell& c, uint32_t i) { xl[i] = kCheb[0] * c.idiag * rl[i]; });
+            __syncthreads();
+            cells.template operator()<l>([&](const BottomCell& c, uint32_t i) {
+                const float v = xl[i];
+                yl[i] = __fmaf_rn(kCheb[1] * c.idiag, rl[i] - mg_bottom_apply(c, xl, v), v);
+            });
+            __syncthreads();
+            cells.template operator()<l>(
+                [&](const BottomCell& c, uint32_t i) { xl[i] = c.idiag > 0.0f ? rl[i] - mg_bottom_apply(c, yl, yl[i]) : 0.0f; });
+            __syncthreads();
+            float* rn = vr + B.off[l + 1];
+            const uint32_t sy = B.nx[l], sz = B.nxy[l];
+            for (uint32_t I = t; I < B.n[l + 1]; I += T) {
+                const uint32_t w = B.words[l][12u * B.n[l] + I], i = w & 0xffffu;
+                float s = 0.0f;
+#pragma unroll
+                for (int ch = 0; ch < 8; ++ch) {
+                    const bool in = w >> (16 + ch) & 1u;
+                    const float v = xl[in ? i + (ch & 1) + (ch >> 1 & 1) * sy + (ch >> 2) * sz : 0u];
+                    s += in ? v : 0.0f;
+                }
+                rn[I] = s;
+            }
+            __syncthreads();
+        };
+        auto up = [&]<int l>() {
+            float *rl = vr + B.off[l], *xl = vx + B.off[l], *yl = vy + B.off[l];
+            const float* e = vx + B.off[l + 1];
+            cells.template operator()<l>([&](const BottomCell& c, uint32_t i) { yl[i] = c.idiag > 0.0f ? __fmaf_rn(kOver, e[c.parent], yl[i]) : 0.0f; });
+            __syncthreads();
+            cells.template operator()<l>([&](const BottomCell& c, uint32_t i) {
+                const float v = yl[i];
+                xl[i] = __fmaf_rn(kCheb[1] * c.idiag, rl[i] - mg_bottom_apply(c, yl, v), v);
+            });
+            __syncthreads();
+            float* res = l == 0 ? out : yl;
+            cells.template operator()<l>([&](const BottomCell& c, uint32_t i) {
+                const float v = xl[i];
+                res[i] = __fmaf_rn(kCheb[0] * c.idiag, rl[i] - mg_bottom_apply(c, xl, v), v);
+            });
+            if (l > 0) {
+                __syncthreads();
+                for (uint32_t i = t; i < B.n[l]; i += T) xl[i] = yl[i];
+                __syncthreads();
+            }
+        };
+        __syncthreads();
+        [&]<int... l>(std::integer_sequence<int, l...>) { (down.template operator()<l>(), ...); }(std::make_integer_sequence<int, last>{});
+        {   // coarsest: e = A^-1 r; thread t sums columns t / 64 + 16 m of row t % 64
+            const uint32_t n = B.n[last], row = t & 63u, part = t >> 6;
+            const float* rl = vr + B.off[last];
+            double s = 0.0;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) s = __fma_rn(inv[m], (double)rl[min(part + 16u * m, n - 1u)], s);
+            lds[part * kMgDense + row] = s;
+            __syncthreads();
+            if (t < n) {
+                double e = 0.0;
+#pragma unroll
+                for (int m = 0; m < T / 64; ++m) e += lds[m * kMgDense + t];
+                if (last == 0) out[t] = (float)e;
+                else vx[B.off[last] + t] = (float)e;
+            }
+            __syncthreads();
+        }
+        [&]<int... l>(std::integer_sequence<int, l...>) { (up.template operator()<last - 1 - l>(), ...); }(std::make_integer_sequence<int, last>{});
+    }
+}
+
+// A grid of at most kMgCoarsest cells: z = A^-1 r in FP64, one block per row of the inverse.
+__global__ __launch_bounds__(kBlock) void mg_dense_kernel(uint32_t n, const double* __restrict__ inv, Pair2 rp, float* __restrict__ x,
+                                                          const PcgStatus* status) {
+    __shared__ double lds[kMaxWaves];
+    if (status->stop) return;
+    const float* __restrict__ r = rp.p[status->k & 1u];
     const uint32_t I = blockIdx.x;
     double s = 0.0;
     for (uint32_t j = threadIdx.x; j < n; j += blockDim.x) s = __fma_rn(inv[(size_t)I * n + j], (double)r[j], s);
@@ -359,129 +859,17 @@ __global__ __launch_bounds__(kBlock) void mg_dense_kernel(uint32_t n, const doub
     if (threadIdx.x == 0) x[I] = (float)v[0];
 }
 
-// Partials of <r, z> on level 0 (when level 0 is the coarsest and the dense solve produced z).
-__global__ __launch_bounds__(kMgThreads) void mg_dot_kernel(uint32_t n, const float* __restrict__ r, const float* __restrict__ z,
-                                                            double* __restrict__ partials, const PcgStatus* status) {
+// Partials of <r, z> on such a grid.
+__global__ __launch_bounds__(kMgDotThreads) void mg_dot_kernel(uint32_t n, Pair2 rp, const float* __restrict__ z, double* __restrict__ partials,
+                                                               const PcgStatus* status) {
     __shared__ double lds[kMaxWaves];
     if (status->stop) return;
-    uint32_t lb, start, end;
-    mg_range(n, lb, start, end);
+    const float* __restrict__ r = rp.p[status->k & 1u];
     double rz = 0.0;
-    for (uint32_t i = start + threadIdx.x; i < end; i += blockDim.x) rz = __fma_rn((double)r[i], (double)z[i], rz);
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) rz = __fma_rn((double)r[i], (double)z[i], rz);
     double v[1]{rz};
     block_sum<1>(v, lds);
-    if (threadIdx.x == 0) partials[kPartRZ * kPcgMaxBlocks + lb] = v[0];
-}
-
-// PCG direction of iteration k: stopping test on ||r||^2 (RR partials) against tol^2 ||b||^2 (BB
-// partials on the first launch of a solve, then the status), beta = rz_k / rz_{k-1} (RZ partials of
-// the V-cycle), p = z + beta p_old (p = z when k = 0), partials of <p, A p>; A p is formed from p
-// at the neighbours on the fly.
-__global__ __launch_bounds__(kMgThreads) void mg_direction_kernel(MgLevel L, uint32_t per, const float* __restrict__ z,
-                                                                  float* __restrict__ p0, float* __restrict__ p1,
-                                                                  double* __restrict__ partials, double* __restrict__ hist,
-                                                                  PcgStatus* status, double tol2, uint32_t check_only) {
-    __shared__ double lds[2 * kMaxWaves];
-    if (status->stop) return;
-    const uint32_t k = status->k;
-    const double* parts[2]{partials + kPartRR * kPcgMaxBlocks, partials + kPartRZ * kPcgMaxBlocks};
-    double red[2];
-    reduce_partials<2>(parts, gridDim.x, red, lds);
-    const double bb = status->bb, rho = red[0], rz = red[1];
-    uint32_t lb, start, end;
-    mg_range(L.n, lb, start, end);
-    const bool converged = !(rho > tol2 * bb);
-    if (converged || check_only) {
-        if (lb == 0 && threadIdx.x == 0) {
-            status->rr = rho;
-            status->iterations = k;
-            if (converged) status->stop = 1u;
-        }
-        return;
-    }
-    if (lb == 0 && threadIdx.x == 0) hist[2 * k] = rz;
-    float* __restrict__ p_new = (k & 1u) ? p1 : p0;
-    const float* __restrict__ p_old = (k & 1u) ? p0 : p1;
-    const bool with_old = k > 0;
-    const float beta = with_old ? (float)(rz / hist[2 * (k - 1)]) : 0.0f;
-    const uint8_t* __restrict__ code = L.code;
-    // z and p_old are 0 off the unknowns, so p_new is too
-    auto pn = [&](uint32_t j) -> float { return with_old ? __fmaf_rn(beta, p_old[j], z[j]) : z[j]; };
-    double pq = 0.0;
-    for (uint32_t base = start + threadIdx.x; base < end; base += kMgUnroll * blockDim.x) {
-#pragma unroll
-        for (int m = 0; m < kMgUnroll; ++m) {
-            const uint32_t i0 = base + (uint32_t)m * blockDim.x;
-            const bool valid = i0 < end;
-            const uint32_t i = min(i0, L.n - 1u);
-            const uint32_t d = code[i];
-            int cx, cy, cz;
-            mg_coords(L, i, cx, cy, cz);
-            const float pi = pn(i);   // 0 off the unknowns
-            if (valid) p_new[i] = pi;
-            // A p as the update forms it (exactly), so alpha and the residual recurrence agree
-            const Nb0 nb = mg_nb0(L, per, cx, cy, cz, i);
-            double sp = 0.0;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) sp += (double)pn(nb.j[k]);
-            const double q = (double)d * (double)pi - sp;
-            pq = valid ? __fma_rn((double)pi, q, pq) : pq;
-        }
-    }
-    double v[1]{pq};
-    block_sum<1>(v, lds);
-    if (threadIdx.x == 0) partials[kPartPQ * kPcgMaxBlocks + lb] = v[0];
-}
-
-// PCG update of iteration k: alpha = rz_k / <p, A p>; x += alpha p; r -= alpha A p; partials of
-// ||r||^2. The solution pair (hi + lo, about 48 bits) takes alpha p in FP64 and A p is exact, so
-// the recursive residual follows the true one to FP32 rounding of r itself: with the near-null
-// mode of the matrix the solution is some 10^3 ||b|| large, and an FP32 increment (or an FP32
-// A p) would leave a gap of about 1e-4 ||b|| between them after the first, largest steps.
-__global__ __launch_bounds__(kMgThreads) void mg_update_kernel(MgLevel L, uint32_t per, const float* __restrict__ p0,
-                                                               const float* __restrict__ p1, float* __restrict__ r, float* __restrict__ xh,
-                                                               float* __restrict__ xl, double* __restrict__ partials,
-                                                               const double* __restrict__ hist, const PcgStatus* status) {
-    __shared__ double lds[kMaxWaves];
-    if (status->stop) return;
-    const uint32_t k = status->k;
-    const float* __restrict__ p = (k & 1u) ? p1 : p0;
-    const double* parts[1]{partials + kPartPQ * kPcgMaxBlocks};
-    double red[1];
-    reduce_partials<1>(parts, gridDim.x, red, lds);
-    const double alpha = hist[2 * k] / red[0];
-    uint32_t lb, start, end;
-    mg_range(L.n, lb, start, end);
-    double rr = 0.0;
-    for (uint32_t base = start + threadIdx.x; base < end; base += kMgUnroll * blockDim.x) {
-#pragma unroll
-        for (int m = 0; m < kMgUnroll; ++m) {
-            const uint32_t i0 = base + (uint32_t)m * blockDim.x;
-            const uint32_t i = min(i0, L.n - 1u);
-            const uint32_t d = L.code[i];
-            const bool live = i0 < end && d != 0u;
-            int cx, cy, cz;
-            mg_coords(L, i, cx, cy, cz);
-            const Nb0 nb = mg_nb0(L, per, cx, cy, cz, i);
-            const float pi = p[i];
-            double sp = 0.0;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) sp += (double)p[nb.j[k]];
-            const double q = (double)d * (double)pi - sp;
-            const double xv = __fma_rn(alpha, (double)pi, (double)xh[i] + (double)xl[i]);
-            const float hi = (float)xv;
-            const float ri = (float)__fma_rn(-alpha, q, (double)r[i]);
-            if (live) {
-                xh[i] = hi;
-                xl[i] = (float)(xv - (double)hi);
-                r[i] = ri;
-            }
-            rr = live ? __fma_rn((double)ri, (double)ri, rr) : rr;
-        }
-    }
-    double v[1]{rr};
-    block_sum<1>(v, lds);
-    if (threadIdx.x == 0) partials[kPartRR * kPcgMaxBlocks + lb] = v[0];
+    if (threadIdx.x == 0) partials[kPartRZ * kPcgMaxBlocks + blockIdx.x] = v[0];
 }
 
 // ---- hierarchy (host) ------------------------------------------------------------------------
@@ -537,6 +925,43 @@ HostLevel coarsen(const HostLevel& f, const bool per[3]) {
                 }
             }
     return c;
+}
+
+// The words of level f for the single-workgroup kernel (BottomCell; c: the next level).
+std::vector<uint32_t> bottom_words(const HostLevel& f, const HostLevel& c, const bool per[3]) {
+    const size_t n = f.cells();
+    std::vector<uint32_t> out(kBottomWords * n, 0u);
+    auto bits = [](double v) { return std::bit_cast<uint32_t>((float)v); };
+    for (int z = 0; z < f.nz; ++z)
+        for (int y = 0; y < f.ny; ++y)
+            for (int x = 0; x < f.nx; ++x) {
+                const size_t i = (size_t)x + (size_t)f.nx * ((size_t)y + (size_t)f.ny * (size_t)z);
+                const bool live = f.diag[i] > 0.0;
+                out[i] = bits(f.diag[i]);
+                out[n + i] = bits(live ? 1.0 / f.diag[i] : 0.0);
+                for (int a = 0; a < 3; ++a) {
+                    int q[3]{x, y, z};
+                    const int e[3]{f.nx, f.ny, f.nz};
+                    const size_t hi = plus_neighbour(f, per, x, y, z, a);
+                    size_t lo = SIZE_MAX;
+                    if (q[a] > 0 || per[a]) {
+                        q[a] = q[a] > 0 ? q[a] - 1 : e[a] - 1;
+                        lo = (size_t)q[0] + (size_t)f.nx * ((size_t)q[1] + (size_t)f.ny * (size_t)q[2]);
+                    }
+                    out[(2 + 2 * a) * n + i] = bits(lo == SIZE_MAX ? 0.0 : f.wp[a][lo]);
+                    out[(3 + 2 * a) * n + i] = bits(hi == SIZE_MAX ? 0.0 : f.wp[a][i]);
+                    out[(8 + a) * n + i] = (uint32_t)(lo == SIZE_MAX ? i : lo) | (uint32_t)(hi == SIZE_MAX ? i : hi) << 16;
+                }
+                const size_t I = (size_t)(x / 2) + (size_t)c.nx * ((size_t)(y / 2) + (size_t)c.ny * (size_t)(z / 2));
+                out[11 * n + i] = (uint32_t)I;
+                if (!(x & 1) && !(y & 1) && !(z & 1)) {
+                    uint32_t w = (uint32_t)i;
+                    for (int k = 0; k < 8; ++k)
+                        if (x + (k & 1) < f.nx && y + (k >> 1 & 1) < f.ny && z + (k >> 2) < f.nz) w |= 1u << (16 + k);
+                    out[12 * n + I] = w;
+                }
+            }
+    return out;
 }
 
 // Inverse of level L's operator over its unknowns (diag > 0), FP64 Cholesky, as a symmetric
@@ -604,10 +1029,6 @@ std::vector<double> dense_inverse(const HostLevel& L, const bool per[3]) {
     return out;
 }
 
-uint32_t periodic_mask(const ds_context* c) {
-    return (c->pressure_periodic[0] ? 1u : 0u) | (c->pressure_periodic[1] ? 2u : 0u) | (c->pressure_periodic[2] ? 4u : 0u);
-}
-
 }  // namespace
 
 void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
@@ -638,7 +1059,9 @@ void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
                     }
                 }
     }
-    while (levels.back().cells() > kMgCoarsest) {
+    // a grid of at most kMgCoarsest cells is solved directly; else down to kMgDense cells
+    const bool direct = levels[0].cells() <= kMgCoarsest;
+    while (!direct && levels.back().cells() > kMgDense) {
         if ((int)levels.size() == kMgMaxLevels) throw Failure{DS_ERROR_UNSUPPORTED, "multigrid: too many levels"};
         HostLevel next = coarsen(levels.back(), per);
         levels.push_back(std::move(next));
@@ -670,81 +1093,156 @@ void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
             for (uint32_t i = 0; i < L.n; ++i) inv[i] = H.diag[i] > 0.0 ? 1.0 / H.diag[i] : 0.0;
             L.idiag = put(inv);
             for (int a = 0; a < 3; ++a) L.wp[a] = put(H.wp[a]);
-            // right-hand side and result
-            w.vec[l][0] = device_alloc<float>(c, L.n);
-            w.vec[l][3] = device_alloc<float>(c, L.n);
-        } else {
-            // the pre-smoothed iterate and the iterate after the first post sweep, each with the
-            // zero pad element n that out-of-domain neighbours read
-            w.vec[l][1] = device_alloc<float>(c, (size_t)L.n + 1);
-            w.vec[l][2] = device_alloc<float>(c, (size_t)L.n + 1);
+            // right-hand side, pre-smoothed iterate, result
+            for (int k = 0; k < 3; ++k) w.vec[l][k] = device_alloc<float>(c, L.n);
+        } else if (!direct) {
+            w.vec[l][1] = device_alloc<float>(c, L.n);   // pre-smoothed iterate
         }
-        for (int k = 0; k < 4; ++k) fill_zero(c, w.vec[l][k], (size_t)L.n + (l == 0 ? 1 : 0));
+        for (int k = 0; k < 3; ++k) fill_zero(c, w.vec[l][k], L.n);
     }
     const std::vector<double> inv = dense_inverse(levels.back(), per);
     w.dense = device_alloc<double>(c, inv.size());
     DS_HIP(hipMemcpy(w.dense, inv.data(), inv.size() * sizeof(double), hipMemcpyHostToDevice));
-    w.z = device_alloc<float>(c, (size_t)g.n + 1);
-    fill_zero(c, w.z, (size_t)g.n + 1);
-}
-
-// z = M^-1 r, the V-cycle from level 0 (r: level 0's right-hand side), with the partials of <r, z>.
-// Level 0: pre-smoothing, restriction; each coarser level but the last: one launch down (its
-// right-hand side to the next level's); the coarsest: the dense solve; back up one launch per
-// coarser level (its result from the next level's); level 0: the two post sweeps.
-void mg_precondition(ds_context* c, const float* r, float* z) {
-    MgWork& w = c->mg;
-    PcgWork& pw = c->pcg;
-    const uint32_t per = periodic_mask(c);
-    const int Lc = w.levels - 1;
-    hipStream_t s = c->stream;
-    PcgStatus* st = pw.status;
-    if (Lc == 0) {
-        mg_dense_kernel<<<w.lv[0].n, kBlock, 0, s>>>(w.lv[0].n, w.dense, r, z, st, 1u);
-        mg_dot_kernel<<<pw.blocks, kMgThreads, 0, s>>>(w.lv[0].n, r, z, pw.partials, st);
-        check_launch("multigrid direct solve");
-        return;
+    w.z = device_alloc<float>(c, g.n);
+    fill_zero(c, w.z, g.n);
+    // the levels one workgroup handles
+    w.bottom_first = direct ? 1 : w.levels - 1;
+    while (!direct && w.bottom_first > 1 && w.lv[w.bottom_first - 1].n <= kMgBottomCells) --w.bottom_first;
+    MgBottom& bt = w.bottom;
+    uint32_t off = 0;
+    for (int l = w.bottom_first; l < w.levels; ++l) {
+        require(bt.count < (uint32_t)kMgBottomLevels, "multigrid: too many coarse levels");
+        bt.n[bt.count] = w.lv[l].n;
+        bt.nx[bt.count] = (uint32_t)w.lv[l].nx;
+        bt.nxy[bt.count] = (uint32_t)w.lv[l].nx * (uint32_t)w.lv[l].ny;
+        bt.words[bt.count] = nullptr;
+        if (l + 1 < w.levels) {
+            const std::vector<uint32_t> words = bottom_words(levels[l], levels[l + 1], per);
+            uint32_t* d = device_alloc<uint32_t>(c, words.size());
+            DS_HIP(hipMemcpy(d, words.data(), words.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+            bt.words[bt.count] = d;
+        }
+        bt.off[bt.count++] = off;
+        off += w.lv[l].n;
     }
-    const MgLevel& L0 = w.lv[0];
-    mg_pre0_kernel<<<xcd_blocks_for(L0.n), kBlock, 0, s>>>(L0, per, r, w.vec[0][1], st);
-    mg_restrict0_kernel<<<xcd_blocks_for(w.lv[1].n), kBlock, 0, s>>>(L0, w.lv[1], per, r, w.vec[0][1], w.vec[1][0], st);
-    for (int l = 1; l < Lc; ++l)
-        mg_down_kernel<<<xcd_blocks_for(8ull * w.lv[l + 1].n), kBlock, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l + 1][0],
-                                                                                st);
-    mg_dense_kernel<<<w.lv[Lc].n, kBlock, 0, s>>>(w.lv[Lc].n, w.dense, w.vec[Lc][0], w.vec[Lc][3], st, 0u);
-    for (int l = Lc - 1; l >= 1; --l)
-        mg_up_kernel<<<xcd_blocks_for(w.lv[l].n), kBlock, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l + 1][3], w.vec[l][3], st);
-    mg_post0_kernel<<<xcd_blocks_for(L0.n), kBlock, 0, s>>>(L0, w.lv[1], per, r, w.vec[0][1], w.vec[1][3], w.vec[0][2], st);
-    mg_post0_last_kernel<<<pw.blocks, kMgThreads, 0, s>>>(L0, per, r, w.vec[0][2], z, pw.partials, st);
-    check_launch("multigrid V-cycle");
-}
-
-void mg_direction(ds_context* c, const float* z, double tol2, bool check_only) {
-    PcgWork& w = c->pcg;
-    mg_direction_kernel<<<w.blocks, kMgThreads, 0, c->stream>>>(c->mg.lv[0], periodic_mask(c), z, w.p[0], w.p[1], w.partials, w.hist,
-                                                               w.status, tol2, check_only ? 1u : 0u);
-}
-
-void mg_update(ds_context* c, float* xh, float* xl) {
-    PcgWork& w = c->pcg;
-    mg_update_kernel<<<w.blocks, kMgThreads, 0, c->stream>>>(c->mg.lv[0], periodic_mask(c), w.p[0], w.p[1], w.r, xh, xl, w.partials,
-                                                            w.hist, w.status);
+    require(off <= kMgBottomLds, "multigrid: the coarse levels do not fit one workgroup");
+    bt.dense = w.dense;
 }
 
 namespace {
 
+Pair2 residuals(const ds_context* c) { return Pair2{{c->pcg.r, c->pcg.r_alt}}; }
+Pair2 directions(const ds_context* c) { return Pair2{{c->pcg.p[0], c->pcg.p[1]}}; }
+
+// Runs f with the box type of the context's level 0: enough boxes to fill the chip, the larger box
+// where there are.
+template <typename F>
+void with_box(const ds_context* c, F&& f) {
+    const uint32_t n = c->geo.n;
+    if (n >= kMgLargeCells) f.template operator()<BoxL>();
+    else if (n >= kMgMediumCells) f.template operator()<BoxM>();
+    else f.template operator()<BoxS>();
+}
+
+template <typename F>
+void with_coarse_box(const MgLevel& L, F&& f) {
+    if (L.n >= kMgCoarseLarge) f.template operator()<BoxC>();
+    else f.template operator()<BoxD>();
+}
+
+void launch_bottom(const MgBottom& B, const float* r, float* out, const double* partials, uint32_t blocks, PcgStatus* st,
+                   double tol2, uint32_t mode, hipStream_t s) {
+    auto launch = [&]<int N>() { mg_bottom_kernel<N><<<1, kBottomThreads, 0, s>>>(B, r, out, partials, blocks, st, tol2, mode); };
+    switch (B.count) {
+        case 0: return launch.template operator()<0>();
+        case 1: return launch.template operator()<1>();
+        case 2: return launch.template operator()<2>();
+        case 3: return launch.template operator()<3>();
+        case 4: return launch.template operator()<4>();
+        default: return launch.template operator()<5>();
+    }
+}
+
+// Level 0's down kernel, the coarser levels, level 0's post kernel: the V-cycle of the residual that
+// iteration k leaves (advance: after its direction kernel; else of the residual as it stands).
+void launch_cycle(ds_context* c, bool advance, float* xh, float* xl, double tol2, uint32_t mode) {
+    MgWork& w = c->mg;
+    PcgWork& pw = c->pcg;
+    hipStream_t s = c->stream;
+    PcgStatus* st = pw.status;
+    const uint32_t per = pcg_periodic_bits(c);
+    const Pair2 r = residuals(c), p = directions(c);
+    const bool direct = w.levels == 1;
+    const MgLevel &L0 = w.lv[0], &L1 = w.lv[direct ? 0 : 1];
+    with_box(c, [&]<typename B>() {
+        if (direct && advance) mg_down0_kernel<B, true, false><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, nullptr, nullptr, pw.partials, pw.hist, st);
+        else if (advance) mg_down0_kernel<B, true, true><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, w.vec[0][1], w.vec[1][0], pw.partials, pw.hist, st);
+        else if (!direct) mg_down0_kernel<B, false, true><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, w.vec[0][1], w.vec[1][0], pw.partials, pw.hist, st);
+    });
+    const int bf = w.bottom_first;
+    for (int l = 1; l < bf; ++l)
+        with_coarse_box(w.lv[l], [&]<typename B>() {
+            mg_down_kernel<B><<<(B::grid(w.lv[l]).count + 7u) & ~7u, B::T, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l][1], w.vec[l + 1][0],
+                                                                                 st);
+        });
+    launch_bottom(w.bottom, direct ? nullptr : w.vec[bf][0], direct ? nullptr : w.vec[bf][2], pw.partials, pw.blocks, st, tol2,
+                  mode | (advance ? 1u : 0u), s);
+    for (int l = bf - 1; l >= 1; --l)
+        with_coarse_box(w.lv[l], [&]<typename B>() {
+            mg_up_kernel<B><<<(B::grid(w.lv[l]).count + 7u) & ~7u, B::T, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l][1], w.vec[l + 1][2],
+                                                                               w.vec[l][2], st);
+        });
+    if (direct) {
+        mg_dense_kernel<<<L0.n, kBlock, 0, s>>>(L0.n, w.dense, r, w.z, st);
+        mg_dot_kernel<<<pw.blocks, kMgDotThreads, 0, s>>>(L0.n, r, w.z, pw.partials, st);
+    } else {
+        with_box(c, [&]<typename B>() {
+            mg_post0_kernel<B><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, w.vec[0][1], w.vec[1][2], w.z, pw.partials, st);
+        });
+    }
+    check_launch("multigrid V-cycle");
+}
+
 __global__ void mg_set_iteration_kernel(PcgStatus* status, uint32_t k) {
-    if (threadIdx.x == 0) status->k = k;
+    if (threadIdx.x == 0) {
+        status->k = k;
+        status->stop = 0u;
+    }
 }
 
 constexpr size_t kMgMaxGraphs = 8;
 
 }  // namespace
 
-void mg_set_iteration(ds_context* c, uint32_t k_before) {
-    mg_set_iteration_kernel<<<1, 64, 0, c->stream>>>(c->pcg.status, k_before);
+uint32_t mg_blocks(const ds_context* c) {
+    uint32_t n = 8;
+    with_box(c, [&]<typename B>() { n = B::grid(c->mg.lv[0]).count; });
+    return std::min<uint32_t>(kPcgMaxBlocks, (n + 7u) & ~7u);
+}
+
+void mg_start(ds_context* c, double tol2, uint32_t first, uint32_t reject) {
+    launch_cycle(c, false, nullptr, nullptr, tol2, (first ? 2u : 0u) | (reject << 2));
+}
+
+void mg_set_iteration(ds_context* c, uint32_t k) {
+    mg_set_iteration_kernel<<<1, 64, 0, c->stream>>>(c->pcg.status, k);
     check_launch("mg_set_iteration_kernel");
 }
+
+float* mg_residual(const ds_context* c, uint32_t k) { return residuals(c).p[k & 1u]; }
+
+namespace {
+
+void launch_iteration(ds_context* c, float* xh, float* xl, double tol2) {
+    PcgWork& pw = c->pcg;
+    with_box(c, [&]<typename B>() {
+        mg_direction_kernel<B><<<pw.blocks, B::T, 0, c->stream>>>(c->mg.lv[0], pcg_periodic_bits(c), c->mg.z, directions(c), pw.partials, pw.hist,
+                                                                 pw.status);
+    });
+    launch_cycle(c, true, xh, xl, tol2, 0u);
+}
+
+}  // namespace
 
 void mg_iteration(ds_context* c, float* xh, float* xl, double tol2) {
     MgWork& w = c->mg;
@@ -759,10 +1257,7 @@ void mg_iteration(ds_context* c, float* xh, float* xl, double tol2) {
         hipGraph_t graph = nullptr;
         DS_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
         try {
-            mg_precondition(c, c->pcg.r, w.z);
-            mg_direction(c, w.z, tol2, false);
-            mg_update(c, xh, xl);
-            check_launch("multigrid iteration (capture)");
+            launch_iteration(c, xh, xl, tol2);
         } catch (...) {
             hipGraph_t partial = nullptr;
             (void)hipStreamEndCapture(c->stream, &partial);
@@ -784,3 +1279,4 @@ void mg_release(ds_context* c) {
 }
 
 }  // namespace ds
+
