@@ -566,18 +566,32 @@ __global__ __launch_bounds__(256) void wgrad_kernel(Dims d, int batch, const uin
             for (int i = 0; i < 4; ++i) out[(size_t)(ab * 16 + 4 * kq + i) * NC + bb * 16 + m] = acc[ab][bb][i];
 }
 
-// dW[mi][ni][tap] (mi < MC, ni < NREAL) = sum over the waves' slots, in wave order (FP64 sums).
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ partials, uint32_t waves, int taps, int mc, int nc,
-                                                           int nreal, float* __restrict__ dw) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// dW[mi][ni][tap] (mi < MC, ni < NREAL) = sum over the waves' slots (FP64 sums in a fixed order). A
+// block reduces 64 neighbouring elements: its 16 waves each add every 16th slot, then the 16 partial
+// sums in order. (One thread per element walked up to 1024 slots by dependent loads from 27 blocks:
+// 212 us a call on the 64^3 batch of 4, now 12.)
+constexpr int kReduceWaves = 16;
+__global__ __launch_bounds__(64 * kReduceWaves) void wgrad_reduce_kernel(const float* __restrict__ partials, uint32_t waves, int taps, int mc,
+                                                                         int nc, int nreal, float* __restrict__ dw) {
+    __shared__ double lds[kReduceWaves][64];
+    const uint32_t lane = threadIdx.x & 63u, part = threadIdx.x >> 6;
+    const uint32_t i = blockIdx.x * 64u + lane;
     const uint32_t per = (uint32_t)taps * mc * nc;
-    if (i >= per) return;
+    double s = 0.0;
+    if (i < per) {
+#pragma unroll 8
+        for (uint32_t w = part; w < waves; w += kReduceWaves) s += (double)partials[(size_t)w * per + i];
+    }
+    lds[part][lane] = s;
+    __syncthreads();
+    if (part != 0 || i >= per) return;
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < kReduceWaves; ++k) t += lds[k][lane];
     const int tap = (int)(i / ((uint32_t)mc * nc));
     const int mi = (int)((i / (uint32_t)nc) % (uint32_t)mc);
     const int ni = (int)(i % (uint32_t)nc);
-    double s = 0.0;
-    for (uint32_t w = 0; w < waves; ++w) s += (double)partials[(size_t)w * per + i];
-    if (ni < nreal) dw[((size_t)mi * nreal + ni) * taps + tap] = (float)s;
+    if (ni < nreal) dw[((size_t)mi * nreal + ni) * taps + tap] = (float)t;
 }
 
 // Per-block FP64 channel sums of a BF16 tensor with C channels over n voxels:
@@ -599,14 +613,21 @@ __global__ __launch_bounds__(256) void channel_sum_kernel(uint32_t n, const uint
     }
 }
 
-// out[c] = sum over `blocks` partial rows (fixed order).
+// out[c] = sum over `blocks` partial rows of c channels (fixed order; c divides 256): thread t adds
+// the rows t / c, t / c + 256 / c, ... of channel t % c, then one thread per channel the partial sums.
 __global__ __launch_bounds__(256) void channel_sum_finish_kernel(const double* __restrict__ partials, uint32_t blocks, int c,
                                                                  float* __restrict__ out) {
-    const int i = (int)threadIdx.x;
-    if (i >= c) return;
+    __shared__ double lds[256];
+    const uint32_t ch = threadIdx.x % (uint32_t)c, part = threadIdx.x / (uint32_t)c, parts = 256u / (uint32_t)c;
     double s = 0.0;
-    for (uint32_t b = 0; b < blocks; ++b) s += partials[(size_t)b * c + i];
-    out[i] = (float)s;
+#pragma unroll 8
+    for (uint32_t b = part; b < blocks; b += parts) s += partials[(size_t)b * c + ch];
+    lds[threadIdx.x] = s;
+    __syncthreads();
+    if (part != 0) return;
+    double t = 0.0;
+    for (uint32_t k = 0; k < parts; ++k) t += lds[k * (uint32_t)c + ch];
+    out[ch] = (float)t;
 }
 
 // Per-sample sum of r^2 over the unknowns: partials[b * G + block] (blockIdx.y = sample b).

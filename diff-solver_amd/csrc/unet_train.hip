@@ -133,7 +133,7 @@ WgradPlan wgrad_plan(uint64_t groups, int taps, int mc, int nc) {
 template <int C>
 void channel_sum(uint64_t n, const uint16_t* t, double* cpart, float* out, hipStream_t s) {
     channel_sum_kernel<C><<<256, 256, 0, s>>>((uint32_t)n, t, cpart);
-    channel_sum_finish_kernel<<<1, 64, 0, s>>>(cpart, 256, C, out);
+    channel_sum_finish_kernel<<<1, 256, 0, s>>>(cpart, 256, C, out);
 }
 
 void channel_sum_any(int c, uint64_t n, const uint16_t* t, double* cpart, float* out, hipStream_t s) {
@@ -168,7 +168,7 @@ void conv_wgrad(int c1, int c2, int cout, const Dims& d, int batch, const uint16
 #undef DS_WGRAD
     if (!done) throw Failure{DS_ERROR_UNSUPPORTED, "3x3x3 convolution weight gradient: shape not in the network"};
     const uint32_t per = 27u * cout * nc;
-    wgrad_reduce_kernel<<<blocks_for(per), 256, 0, s>>>(slots, p.waves, 27, cout, nc, c1 + c2, dw);
+    wgrad_reduce_kernel<<<blocks_for(per, 64), 64 * kReduceWaves, 0, s>>>(slots, p.waves, 27, cout, nc, c1 + c2, dw);
     channel_sum_any(cout, (uint64_t)d.nx * d.ny * d.nz * batch, dz, cpart, db, s);
 }
 
@@ -199,7 +199,7 @@ void tconv_wgrad(int cin, int cout, const Dims& dc, int batch, const uint16_t* i
     else if (cin == 32 && cout == 16) wgrad_kernel<1, 32, 16, 0><<<grid, 256, 0, s>>>(dc, batch, in, dout, nullptr, p.per_wave, slots);
     else throw Failure{DS_ERROR_UNSUPPORTED, "transposed convolution shape not in the network"};
     const uint32_t per = 8u * cin * cout;
-    wgrad_reduce_kernel<<<blocks_for(per), 256, 0, s>>>(slots, p.waves, 8, cin, cout, cout, dw);
+    wgrad_reduce_kernel<<<blocks_for(per, 64), 64 * kReduceWaves, 0, s>>>(slots, p.waves, 8, cin, cout, cout, dw);
     channel_sum_any(cout, (uint64_t)dc.nx * dc.ny * dc.nz * batch * 8, dout, cpart, db, s);
 }
 
@@ -381,14 +381,22 @@ __global__ __launch_bounds__(256) void head_backward_kernel(uint32_t total, cons
         for (int k = 0; k < 17; ++k) partials[(size_t)blockIdx.x * 17 + k] = v[k];
 }
 
-__global__ __launch_bounds__(64) void head_backward_finish_kernel(const double* __restrict__ partials, uint32_t blocks,
-                                                                  float* __restrict__ dw, float* __restrict__ db) {
-    const int k = (int)threadIdx.x;
-    if (k >= 17) return;
-    double s = 0.0;
-    for (uint32_t b = 0; b < blocks; ++b) s += partials[(size_t)b * 17 + k];
-    if (k < 16) dw[k] = (float)s;
-    else db[0] = (float)s;
+// The head's gradients from the partial rows of 17 sums (fixed order): thread t adds every 256th row.
+__global__ __launch_bounds__(256) void head_backward_finish_kernel(const double* __restrict__ partials, uint32_t blocks,
+                                                                   float* __restrict__ dw, float* __restrict__ db) {
+    __shared__ double lds[17 * kMaxWaves];
+    double v[17];
+#pragma unroll
+    for (int k = 0; k < 17; ++k) {
+        v[k] = 0.0;
+        for (uint32_t b = threadIdx.x; b < blocks; b += 256u) v[k] += partials[(size_t)b * 17 + k];
+    }
+    block_sum<17>(v, lds);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) dw[k] = (float)v[k];
+        db[0] = (float)v[16];
+    }
 }
 
 // Adam (Kingma & Ba, with bias correction): m = b1 m + (1 - b1) g, v = b2 v + (1 - b2) g^2,
@@ -544,7 +552,7 @@ void trainer_backward(ds_unet_trainer* t) {
     auto gw = [&](int k) { return G + t->off_w[k]; };
     auto gb = [&](int k) { return G + t->off_b[k]; };
     head_backward_kernel<<<256, 256, 0, s>>>(total, t->dg, t->dd1, t->params + t->off_w[12], t->gd1, t->hpart);
-    head_backward_finish_kernel<<<1, 64, 0, s>>>(t->hpart, 256, gw(12), gb(12));
+    head_backward_finish_kernel<<<1, 256, 0, s>>>(t->hpart, 256, gw(12), gb(12));
     // level 1 decoder
     conv_wgrad(16, 0, 16, t->d1, B, t->a5, nullptr, t->gd1, t->slots, t->cpart, gw(11), gb(11), s);
     conv_dgrad(16, 0, 16, t->d1, B, t->gd1, t->wd[11], t->a5, t->ga5, nullptr, s);
