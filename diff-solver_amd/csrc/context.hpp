@@ -107,7 +107,7 @@ struct PcgStatus {
     uint32_t aborted;       // 1 when a resident launch's grid barrier exceeded its bound
     double bb;              // ||b||^2
     double rr;              // last reduced ||r||^2 (recursive or true)
-    uint32_t k;             // DS_CG_MULTIGRID: updates applied so far (advanced on the device)
+    uint32_t k;             // DS_CG_MULTIGRID: updates applied so far
     uint32_t unused;
     double rr0;             // DS_CG_MULTIGRID: ||r||^2 of the initial guess
 };
@@ -230,16 +230,6 @@ struct MgWork {
     float* z = nullptr;             // the preconditioned residual
     int bottom_first = 1;           // first level of the single-workgroup kernel
     MgBottom bottom{};
-    // one iteration (V-cycle, direction, update) captured as a HIP graph per solution pair and
-    // tolerance: a kernel launch costs the host about as long as the kernels of a coarse level
-    // take on the device, a graph launch replays all thirteen for about the cost of one
-    struct Graph {
-        const float* xh;
-        const float* xl;
-        double tol2;
-        hipGraphExec_t exec;
-    };
-    std::vector<Graph> graphs;
 };
 
 }  // namespace ds
@@ -377,20 +367,17 @@ void window_allocate(ds_context* c, SolveWindow& w);
 // per block, cooperative launch possible with every block co-resident) and allocates its state.
 void pcg_resident_prepare(ds_context* c);
 // DS_CG_MULTIGRID (pcg_mg.hip): builds the hierarchy from the host copy of the code. A solve is
-// mg_start (stopping test and V-cycle of the residual as it stands; first: take ||b||^2 and the
-// initial residual; reject: 1 a guess with a residual above ||b||, 2 only a non-finite one), then one
-// mg_iteration per iteration: direction, update of the solution pair (xh, xl) and the residual,
-// stopping test, V-cycle. The kernels take the iteration index k from the status (set-up and
-// mg_set_iteration set it, the stopping test of an iteration advances it), so one captured iteration
-// (per pair and tolerance) replays for every k; the residual of index k is mg_residual(k).
-// mg_blocks: blocks of the level-0 kernels, one partial each; mg_release destroys the graphs.
+// mg_start (stopping test and V-cycle of the residual of index k as it stands; first: take ||b||^2 and
+// the initial residual; reject: 1 a guess with a residual above ||b||, 2 only a non-finite one), then
+// one mg_iteration per iteration k: direction, update of the solution pair (xh, xl) and the residual,
+// stopping test, V-cycle. The residual after k updates is pcg.r for even k, pcg.r_alt for odd; the
+// stopping test leaves k in the status. mg_set_iteration sets it and clears the stop. mg_blocks: blocks
+// of the level-0 kernels, one partial each.
 void mg_prepare(ds_context* c, const std::vector<uint8_t>& code);
 uint32_t mg_blocks(const ds_context* c);
-void mg_start(ds_context* c, double tol2, uint32_t first, uint32_t reject);
+void mg_start(ds_context* c, uint32_t k, double tol2, uint32_t first, uint32_t reject);
 void mg_set_iteration(ds_context* c, uint32_t k);
-float* mg_residual(const ds_context* c, uint32_t k);
-void mg_iteration(ds_context* c, float* xh, float* xl, double tol2);
-void mg_release(ds_context* c);
+void mg_iteration(ds_context* c, uint32_t k, float* xh, float* xl, double tol2);
 // DS_PROJECTION_RBGS (rbgs.hip): the diagonal table, then the solve of a right-hand-side kind
 // (1 forward, 2 the unrolled reverse, 3 tangent) into xh with xl = 0.
 void rbgs_prepare(ds_context* c);

@@ -752,7 +752,7 @@ bool pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, uint32_t ma
         check_launch("pcg_true_residual_kernel");
         return read_status(c);
     };
-    mg_start(c, tol2, 1u, reject);
+    mg_start(c, 0u, tol2, 1u, reject);
     uint32_t k = 0;
     uint32_t restarts = 0;
     Profiler& prof = c->profiler;
@@ -768,7 +768,7 @@ bool pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, uint32_t ma
                     e1 = prof.take();
                 }
                 if (e0) DS_HIP(hipEventRecord(e0, c->stream));
-                mg_iteration(c, xh, xl, tol2);
+                mg_iteration(c, k, xh, xl, tol2);
                 if (e1) {
                     DS_HIP(hipEventRecord(e1, c->stream));
                     prof.recs.push_back({5, e0, e1});
@@ -777,7 +777,7 @@ bool pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, uint32_t ma
                 ++k;
                 if (k % R == 0u && k < max_it) {   // residual replacement, and its V-cycle
                     true_residual(1u);
-                    mg_start(c, tol2, 0u, 0u);
+                    mg_start(c, k, tol2, 0u, 0u);
                 }
             }
             st = finish(2u);
@@ -802,7 +802,7 @@ bool pcg_iterate_mg(ds_context* c, float* xh, float* xl, double tol, uint32_t ma
         // from it with the previous direction discarded
         fill_zero(c, w.p[(k + 1u) & 1u], c->geo.n);
         mg_set_iteration(c, k);
-        mg_start(c, tol2, 0u, 0u);
+        mg_start(c, k, tol2, 0u, 0u);
     }
     return false;
 }

@@ -176,6 +176,36 @@ __device__ __forceinline__ void mg_load_coarse(const MgLevel& C, uint32_t per, i
     }
 }
 
+// The end of a solve's queue finds status->stop set and every kernel returns. The test stands behind
+// the kernel's first loads, which do not depend on it (the host passes the iteration index), so that
+// its latency hides behind theirs; the barrier keeps the compiler from moving them below the branch.
+__device__ __forceinline__ bool mg_stopped(uint32_t stop) {
+    asm volatile("" ::: "memory");
+    return stop != 0u;
+}
+
+// A producer's per-block partial sums: the loads, issued before the kernel's others, and their sum
+// over the workgroup of T threads in a fixed order.
+template <int T>
+struct Partials {
+    static constexpr int N = ((int)kPcgMaxBlocks + T - 1) / T;
+    double v[N];
+    __device__ __forceinline__ Partials(const double* __restrict__ parts, uint32_t count) {
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const uint32_t i = threadIdx.x + (uint32_t)(m * T);
+            v[m] = i < count ? parts[i] : 0.0;
+        }
+    }
+    __device__ __forceinline__ double sum(double* lds) const {
+        double s[1]{v[0]};
+#pragma unroll
+        for (int m = 1; m < N; ++m) s[0] += v[m];
+        block_sum<1>(s, lds);
+        return s[0];
+    }
+};
+
 // In-plane neighbours of LDS element i of planes X wide.
 template <int X>
 __device__ __forceinline__ float mg_plane_sum(const float* v, int i) {
@@ -194,7 +224,7 @@ template <typename B, bool Update, bool Smooth>
 __global__ __launch_bounds__(B::T) void mg_down0_kernel(MgLevel L, MgLevel C, uint32_t per, Pair2 r, Pair2 p, float* __restrict__ xh,
                                                         float* __restrict__ xl, float* __restrict__ x, float* __restrict__ rc,
                                                         double* __restrict__ partials, const double* __restrict__ hist,
-                                                        const PcgStatus* status) {
+                                                        const PcgStatus* status, uint32_t k) {
     constexpr int X3 = B::template X<3>, X2 = B::template X<2>, X1 = B::template X<1>;
     constexpr int P3 = B::template P<3>, P2 = B::template P<2>, P1 = B::template P<1>;
     constexpr int Z3 = B::template Z<3>, Z2 = B::template Z<2>, Z1 = B::template Z<1>;
@@ -202,8 +232,9 @@ __global__ __launch_bounds__(B::T) void mg_down0_kernel(MgLevel L, MgLevel C, ui
     __shared__ float sp[P3 * Z3];   // p, then the first sweep's iterate, then the residual's z pairs
     __shared__ float sx[P1 * Z1];
     __shared__ double lds[kMaxWaves];
-    if (status->stop) return;
-    const uint32_t k = status->k;
+    const uint32_t stop = status->stop;
+    const Partials<B::T> pq(partials + kPartPQ * kPcgMaxBlocks, Update ? gridDim.x : 0u);
+    const double rz = Update ? hist[2 * k] : 0.0;
     const float* __restrict__ r_in = r.p[k & 1u];
     float* __restrict__ r_out = r.p[(k + 1u) & 1u];
     const float* __restrict__ pk = p.p[k & 1u];
@@ -217,7 +248,7 @@ __global__ __launch_bounds__(B::T) void mg_down0_kernel(MgLevel L, MgLevel C, ui
     const bool mine0 = mine2 && cx >= 2 && cx < X2 - 2 && cy >= 2 && cy < B::template Y<2> - 2;
     const int i3 = (cy + 1) * X3 + cx + 1, i1 = (cy - 1) * X1 + cx - 1;   // the column's element in a plane
     double alpha = 0.0, rr = 0.0;
-    bool have_alpha = false;
+    if (first == last && stop) return;   // (no boxes here)
     for (uint32_t b = first; b < last; ++b) {
         int x0, y0, z0;
         B::origin(grid, b, x0, y0, z0);
@@ -242,12 +273,9 @@ __global__ __launch_bounds__(B::T) void mg_down0_kernel(MgLevel L, MgLevel C, ui
             rv[z] = mg_load(r_in, pl3, z + 1, c);
             dv[z] = mg_load(L.code, pl3, z + 1, c);
         }
-        if (Update && !have_alpha) {
-            const double* parts[1]{partials + kPartPQ * kPcgMaxBlocks};
-            double red[1];
-            reduce_partials<1>(parts, gridDim.x, red, lds);
-            alpha = hist[2 * k] / red[0];
-            have_alpha = true;
+        if (b == first) {
+            if (mg_stopped(stop)) return;
+            if (Update) alpha = rz / pq.sum(lds);
         }
         const bool own = mine0 && x0 - 2 + cx < L.nx && y0 - 2 + cy < L.ny;   // the box's own cells (not wrapped ones)
         if (Update) {
@@ -347,14 +375,14 @@ __global__ __launch_bounds__(B::T) void mg_down0_kernel(MgLevel L, MgLevel C, ui
 template <typename B>
 __global__ __launch_bounds__(B::T) void mg_post0_kernel(MgLevel L, MgLevel C, uint32_t per, Pair2 r, const float* __restrict__ x,
                                                         const float* __restrict__ e_c, float* __restrict__ z_out, double* __restrict__ partials,
-                                                        const PcgStatus* status) {
+                                                        const PcgStatus* status, uint32_t k) {
     constexpr int X2 = B::template X<2>, X1 = B::template X<1>, P2 = B::template P<2>, P1 = B::template P<1>;
     constexpr int Z2 = B::template Z<2>, Z1 = B::template Z<1>;
     __shared__ float sx[P2 * Z2];
     __shared__ float sy[P1 * Z1];
     __shared__ double lds[kMaxWaves];
-    if (status->stop) return;
-    const float* __restrict__ rk = r.p[status->k & 1u];
+    const uint32_t stop = status->stop;
+    const float* __restrict__ rk = r.p[k & 1u];
     const int t = (int)threadIdx.x;
     const uint32_t lb = xcd_block();
     const typename B::Grid grid = B::grid(L);
@@ -365,6 +393,7 @@ __global__ __launch_bounds__(B::T) void mg_post0_kernel(MgLevel L, MgLevel C, ui
     const bool mine0 = mine2 && cx >= 2 && cx < X2 - 2 && cy >= 2 && cy < B::template Y<2> - 2;
     const int i1 = (cy - 1) * X1 + cx - 1;
     double rz = 0.0;
+    if (first == last && stop) return;
     for (uint32_t b = first; b < last; ++b) {
         int x0, y0, z0;
         B::origin(grid, b, x0, y0, z0);
@@ -385,6 +414,7 @@ __global__ __launch_bounds__(B::T) void mg_post0_kernel(MgLevel L, MgLevel C, ui
         for (int z = 0; z < Z2; ++z) xv[z] = dv[z] ? __fmaf_rn(kOver, ev[z], xv[z]) : 0.0f;
 #pragma unroll
         for (int z = 0; z < Z1; ++z) rv[z] = mg_load(rk, pl2, z + 1, c);
+        if (b == first && mg_stopped(stop)) return;
         if (mine2) {
 #pragma unroll
             for (int z = 0; z < Z2; ++z) sx[z * P2 + t] = xv[z];
@@ -428,12 +458,13 @@ __global__ __launch_bounds__(B::T) void mg_post0_kernel(MgLevel L, MgLevel C, ui
 template <typename B>
 __global__ __launch_bounds__(B::T) void mg_direction_kernel(MgLevel L, uint32_t per, const float* __restrict__ z_in, Pair2 p,
                                                             double* __restrict__ partials, double* __restrict__ hist,
-                                                            const PcgStatus* status) {
+                                                            const PcgStatus* status, uint32_t k) {
     constexpr int X1 = B::template X<1>, P1 = B::template P<1>, Z1 = B::template Z<1>;
     __shared__ float sp[P1 * Z1];
     __shared__ double lds[kMaxWaves];
-    if (status->stop) return;
-    const uint32_t k = status->k;
+    const uint32_t stop = status->stop;
+    const Partials<B::T> rz(partials + kPartRZ * kPcgMaxBlocks, gridDim.x);
+    const double rz_old = k > 0u ? hist[2 * (k - 1u)] : 1.0;
     float* __restrict__ p_new = p.p[k & 1u];
     const float* __restrict__ p_old = p.p[(k + 1u) & 1u];
     const int t = (int)threadIdx.x;
@@ -444,8 +475,8 @@ __global__ __launch_bounds__(B::T) void mg_direction_kernel(MgLevel L, uint32_t 
     const bool mine1 = t < P1;
     const bool mine0 = mine1 && cx >= 1 && cx < X1 - 1 && cy >= 1 && cy < B::template Y<1> - 1;
     float beta = 0.0f;
-    bool have_beta = false;
     double pq = 0.0;
+    if (first == last && stop) return;
     for (uint32_t b = first; b < last; ++b) {
         int x0, y0, z0;
         B::origin(grid, b, x0, y0, z0);
@@ -460,13 +491,11 @@ __global__ __launch_bounds__(B::T) void mg_direction_kernel(MgLevel L, uint32_t 
         }
 #pragma unroll
         for (int z = 0; z < B::BZ; ++z) dv[z] = mg_load(L.code, pl1, z + 1, c);
-        if (!have_beta) {
-            const double* parts[1]{partials + kPartRZ * kPcgMaxBlocks};
-            double red[1];
-            reduce_partials<1>(parts, gridDim.x, red, lds);
-            if (b == 0 && t == 0) hist[2 * k] = red[0];   // the block of the first box
-            beta = k > 0u ? (float)(red[0] / hist[2 * (k - 1u)]) : 0.0f;
-            have_beta = true;
+        if (b == first) {
+            if (mg_stopped(stop)) return;
+            const double rz_new = rz.sum(lds);
+            if (b == 0 && t == 0) hist[2 * k] = rz_new;   // the block of the first box
+            beta = k > 0u ? (float)(rz_new / rz_old) : 0.0f;
         }
 #pragma unroll
         for (int z = 0; z < Z1; ++z) {
@@ -532,7 +561,7 @@ __global__ __launch_bounds__(B::T) void mg_down_kernel(MgLevel L, MgLevel C, uin
     constexpr int X2 = B::template X<2>, X1 = B::template X<1>, P2 = B::template P<2>, P1 = B::template P<1>;
     constexpr int Z2 = B::template Z<2>, Z1 = B::template Z<1>;
     __shared__ float s1[P2 * Z2], sx[P1 * Z1];
-    if (status->stop) return;
+    const uint32_t stop = status->stop;
     const int t = (int)threadIdx.x;
     const typename B::Grid grid = B::grid(L);
     const uint32_t b = xcd_block();
@@ -556,6 +585,7 @@ __global__ __launch_bounds__(B::T) void mg_down_kernel(MgLevel L, MgLevel C, uin
     const float zm0 = mg_load(L.wp[2], pl2, 0, k.c);
 #pragma unroll
     for (int z = 0; z < Z1; ++z) w[z] = mg_row(L, pl2, z + 1, k);
+    if (mg_stopped(stop)) return;
 #pragma unroll
     for (int z = 0; z < Z2; ++z) {
         x1[z] = kCheb[0] * iv[z] * rv[z];   // 0 off the unknowns (1 / diag is 0 there)
@@ -605,7 +635,7 @@ __global__ __launch_bounds__(B::T) void mg_up_kernel(MgLevel L, MgLevel C, uint3
     constexpr int X2 = B::template X<2>, X1 = B::template X<1>, P2 = B::template P<2>, P1 = B::template P<1>;
     constexpr int Z2 = B::template Z<2>, Z1 = B::template Z<1>;
     __shared__ float sx[P2 * Z2], sy[P1 * Z1];
-    if (status->stop) return;
+    const uint32_t stop = status->stop;
     const int t = (int)threadIdx.x;
     const typename B::Grid grid = B::grid(L);
     const uint32_t b = xcd_block();
@@ -635,6 +665,7 @@ __global__ __launch_bounds__(B::T) void mg_up_kernel(MgLevel L, MgLevel C, uint3
         w[z] = mg_row(L, pl2, z + 1, k);
         rv[z] = mg_load(r, pl2, z + 1, k.c);
     }
+    if (mg_stopped(stop)) return;
 #pragma unroll
     for (int z = 0; z < Z2; ++z) xv[z] = iv[z] > 0.0f ? __fmaf_rn(kOver, ev[z], xv[z]) : 0.0f;
     if (mine2) {
@@ -697,7 +728,7 @@ __device__ __forceinline__ float mg_bottom_apply(const BottomCell& c, const floa
 // at most kMgBottomCells cells in one workgroup: vectors in LDS, the rows of the first two levels in
 // registers, and the coarsest level's inverse (n x n, FP64, n <= kMgDense) spread over the threads.
 // Levels: how many (the last is the dense one; 0: only the test).
-// mode: bit 0 the iteration index advances (the update of iteration k ran before), bit 1 the first
+// k: updates applied so far. mode: bit 1 the first
 // test of a solve (||b||^2 from its partials, the initial residual kept), bit 2 the guess is rejected
 // when its residual exceeds ||b||, bit 3 when it is not finite. A rejection stops the solve: the
 // host, which reads the status once at its end, runs it again without the guess.
@@ -706,14 +737,16 @@ constexpr int kBottomWords = 13;
 template <int Levels>
 __global__ __launch_bounds__(kBottomThreads) void mg_bottom_kernel(MgBottom B, const float* __restrict__ r,
                                                                    float* __restrict__ out, const double* __restrict__ partials,
-                                                                   uint32_t blocks, PcgStatus* status, double tol2, uint32_t mode) {
+                                                                   uint32_t blocks, PcgStatus* status, double tol2, uint32_t mode, uint32_t k) {
     constexpr int T = kBottomThreads, last = Levels - 1;
     __shared__ float vr[Levels ? kMgBottomLds : 1], vx[Levels ? kMgBottomLds : 1], vy[Levels ? kMgBottomLds : 1];
     __shared__ double lds[(T / 64) * kMgDense];
-    if (status->stop) return;
+    const uint32_t stopped = status->stop;
     const uint32_t t = threadIdx.x;
-    const uint32_t k = status->k + (mode & 1u);
     const double bb0 = status->bb;
+    const bool opening = mode & 2u;
+    const Partials<T> rr_parts(partials + kPartRR * kPcgMaxBlocks, blocks);
+    const Partials<T> bb_parts(partials + kPartBB * kPcgMaxBlocks, opening ? blocks : 0u);
     // everything the cycle reads from memory, up front
     BottomCell c0[4], c1[2];
     double inv[4];
@@ -736,12 +769,9 @@ __global__ __launch_bounds__(kBottomThreads) void mg_bottom_kernel(MgBottom B, c
         for (int m = 0; m < 2; ++m)
             if (t + m * T < B.n[1]) c1[m] = mg_bottom_cell(B.words[1], B.n[1], t + m * T);
     }
-    const bool opening = mode & 2u;
-    double red[2]{0.0, 0.0};
-    for (uint32_t i = t; i < blocks; i += T) {
-        red[0] += partials[kPartRR * kPcgMaxBlocks + i];
-        if (opening) red[1] += partials[kPartBB * kPcgMaxBlocks + i];
-    }
+    if (mg_stopped(stopped)) return;
+    double red[2]{rr_parts.v[0], bb_parts.v[0]};
+    static_assert(Partials<T>::N == 1, "one partial per thread");
     block_sum<2>(red, lds);
     const double rr = red[0], bb = opening ? red[1] : bb0;
     const bool finite = isfinite(rr);
@@ -847,10 +877,10 @@ __global__ __launch_bounds__(kBottomThreads) void mg_bottom_kernel(MgBottom B, c
 
 // A grid of at most kMgCoarsest cells: z = A^-1 r in FP64, one block per row of the inverse.
 __global__ __launch_bounds__(kBlock) void mg_dense_kernel(uint32_t n, const double* __restrict__ inv, Pair2 rp, float* __restrict__ x,
-                                                          const PcgStatus* status) {
+                                                          const PcgStatus* status, uint32_t k) {
     __shared__ double lds[kMaxWaves];
     if (status->stop) return;
-    const float* __restrict__ r = rp.p[status->k & 1u];
+    const float* __restrict__ r = rp.p[k & 1u];
     const uint32_t I = blockIdx.x;
     double s = 0.0;
     for (uint32_t j = threadIdx.x; j < n; j += blockDim.x) s = __fma_rn(inv[(size_t)I * n + j], (double)r[j], s);
@@ -861,10 +891,10 @@ __global__ __launch_bounds__(kBlock) void mg_dense_kernel(uint32_t n, const doub
 
 // Partials of <r, z> on such a grid.
 __global__ __launch_bounds__(kMgDotThreads) void mg_dot_kernel(uint32_t n, Pair2 rp, const float* __restrict__ z, double* __restrict__ partials,
-                                                               const PcgStatus* status) {
+                                                               const PcgStatus* status, uint32_t k) {
     __shared__ double lds[kMaxWaves];
     if (status->stop) return;
-    const float* __restrict__ r = rp.p[status->k & 1u];
+    const float* __restrict__ r = rp.p[k & 1u];
     double rz = 0.0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) rz = __fma_rn((double)r[i], (double)z[i], rz);
     double v[1]{rz};
@@ -1151,8 +1181,8 @@ void with_coarse_box(const MgLevel& L, F&& f) {
 }
 
 void launch_bottom(const MgBottom& B, const float* r, float* out, const double* partials, uint32_t blocks, PcgStatus* st,
-                   double tol2, uint32_t mode, hipStream_t s) {
-    auto launch = [&]<int N>() { mg_bottom_kernel<N><<<1, kBottomThreads, 0, s>>>(B, r, out, partials, blocks, st, tol2, mode); };
+                   double tol2, uint32_t mode, uint32_t k, hipStream_t s) {
+    auto launch = [&]<int N>() { mg_bottom_kernel<N><<<1, kBottomThreads, 0, s>>>(B, r, out, partials, blocks, st, tol2, mode, k); };
     switch (B.count) {
         case 0: return launch.template operator()<0>();
         case 1: return launch.template operator()<1>();
@@ -1164,8 +1194,9 @@ void launch_bottom(const MgBottom& B, const float* r, float* out, const double* 
 }
 
 // Level 0's down kernel, the coarser levels, level 0's post kernel: the V-cycle of the residual that
-// iteration k leaves (advance: after its direction kernel; else of the residual as it stands).
-void launch_cycle(ds_context* c, bool advance, float* xh, float* xl, double tol2, uint32_t mode) {
+// iteration k leaves (advance: after its direction kernel; else of the residual of index k as it stands).
+void launch_cycle(ds_context* c, uint32_t k, bool advance, float* xh, float* xl, double tol2, uint32_t mode) {
+    const uint32_t after = k + (advance ? 1u : 0u);
     MgWork& w = c->mg;
     PcgWork& pw = c->pcg;
     hipStream_t s = c->stream;
@@ -1175,9 +1206,9 @@ void launch_cycle(ds_context* c, bool advance, float* xh, float* xl, double tol2
     const bool direct = w.levels == 1;
     const MgLevel &L0 = w.lv[0], &L1 = w.lv[direct ? 0 : 1];
     with_box(c, [&]<typename B>() {
-        if (direct && advance) mg_down0_kernel<B, true, false><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, nullptr, nullptr, pw.partials, pw.hist, st);
-        else if (advance) mg_down0_kernel<B, true, true><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, w.vec[0][1], w.vec[1][0], pw.partials, pw.hist, st);
-        else if (!direct) mg_down0_kernel<B, false, true><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, w.vec[0][1], w.vec[1][0], pw.partials, pw.hist, st);
+        if (direct && advance) mg_down0_kernel<B, true, false><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, nullptr, nullptr, pw.partials, pw.hist, st, k);
+        else if (advance) mg_down0_kernel<B, true, true><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, w.vec[0][1], w.vec[1][0], pw.partials, pw.hist, st, k);
+        else if (!direct) mg_down0_kernel<B, false, true><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, p, xh, xl, w.vec[0][1], w.vec[1][0], pw.partials, pw.hist, st, k);
     });
     const int bf = w.bottom_first;
     for (int l = 1; l < bf; ++l)
@@ -1186,18 +1217,18 @@ void launch_cycle(ds_context* c, bool advance, float* xh, float* xl, double tol2
                                                                                  st);
         });
     launch_bottom(w.bottom, direct ? nullptr : w.vec[bf][0], direct ? nullptr : w.vec[bf][2], pw.partials, pw.blocks, st, tol2,
-                  mode | (advance ? 1u : 0u), s);
+                  mode, after, s);
     for (int l = bf - 1; l >= 1; --l)
         with_coarse_box(w.lv[l], [&]<typename B>() {
             mg_up_kernel<B><<<(B::grid(w.lv[l]).count + 7u) & ~7u, B::T, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l][1], w.vec[l + 1][2],
                                                                                w.vec[l][2], st);
         });
     if (direct) {
-        mg_dense_kernel<<<L0.n, kBlock, 0, s>>>(L0.n, w.dense, r, w.z, st);
-        mg_dot_kernel<<<pw.blocks, kMgDotThreads, 0, s>>>(L0.n, r, w.z, pw.partials, st);
+        mg_dense_kernel<<<L0.n, kBlock, 0, s>>>(L0.n, w.dense, r, w.z, st, after);
+        mg_dot_kernel<<<pw.blocks, kMgDotThreads, 0, s>>>(L0.n, r, w.z, pw.partials, st, after);
     } else {
         with_box(c, [&]<typename B>() {
-            mg_post0_kernel<B><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, w.vec[0][1], w.vec[1][2], w.z, pw.partials, st);
+            mg_post0_kernel<B><<<pw.blocks, B::T, 0, s>>>(L0, L1, per, r, w.vec[0][1], w.vec[1][2], w.z, pw.partials, st, after);
         });
     }
     check_launch("multigrid V-cycle");
@@ -1210,8 +1241,6 @@ __global__ void mg_set_iteration_kernel(PcgStatus* status, uint32_t k) {
     }
 }
 
-constexpr size_t kMgMaxGraphs = 8;
-
 }  // namespace
 
 uint32_t mg_blocks(const ds_context* c) {
@@ -1220,8 +1249,8 @@ uint32_t mg_blocks(const ds_context* c) {
     return std::min<uint32_t>(kPcgMaxBlocks, (n + 7u) & ~7u);
 }
 
-void mg_start(ds_context* c, double tol2, uint32_t first, uint32_t reject) {
-    launch_cycle(c, false, nullptr, nullptr, tol2, (first ? 2u : 0u) | (reject << 2));
+void mg_start(ds_context* c, uint32_t k, double tol2, uint32_t first, uint32_t reject) {
+    launch_cycle(c, k, false, nullptr, nullptr, tol2, (first ? 2u : 0u) | (reject << 2));
 }
 
 void mg_set_iteration(ds_context* c, uint32_t k) {
@@ -1229,53 +1258,17 @@ void mg_set_iteration(ds_context* c, uint32_t k) {
     check_launch("mg_set_iteration_kernel");
 }
 
-float* mg_residual(const ds_context* c, uint32_t k) { return residuals(c).p[k & 1u]; }
 
-namespace {
-
-void launch_iteration(ds_context* c, float* xh, float* xl, double tol2) {
+// Eight direct launches at 128^3, six at 64^3: the host queues them faster (2.9 us each) than the GPU
+// runs them. (Replayed as a graph per iteration they cost about 8 us more at each graph's edge:
+// simulate at 64^3, 20 steps, 9.59 against 9.03 ms.)
+void mg_iteration(ds_context* c, uint32_t k, float* xh, float* xl, double tol2) {
     PcgWork& pw = c->pcg;
     with_box(c, [&]<typename B>() {
         mg_direction_kernel<B><<<pw.blocks, B::T, 0, c->stream>>>(c->mg.lv[0], pcg_periodic_bits(c), c->mg.z, directions(c), pw.partials, pw.hist,
-                                                                 pw.status);
+                                                                 pw.status, k);
     });
-    launch_cycle(c, true, xh, xl, tol2, 0u);
-}
-
-}  // namespace
-
-void mg_iteration(ds_context* c, float* xh, float* xl, double tol2) {
-    MgWork& w = c->mg;
-    hipGraphExec_t exec = nullptr;
-    for (const MgWork::Graph& g : w.graphs)
-        if (g.xh == xh && g.xl == xl && g.tol2 == tol2) exec = g.exec;
-    if (!exec) {
-        if (w.graphs.size() == kMgMaxGraphs) {
-            (void)hipGraphExecDestroy(w.graphs.front().exec);
-            w.graphs.erase(w.graphs.begin());
-        }
-        hipGraph_t graph = nullptr;
-        DS_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
-        try {
-            launch_iteration(c, xh, xl, tol2);
-        } catch (...) {
-            hipGraph_t partial = nullptr;
-            (void)hipStreamEndCapture(c->stream, &partial);
-            if (partial) (void)hipGraphDestroy(partial);
-            throw;
-        }
-        DS_HIP(hipStreamEndCapture(c->stream, &graph));
-        const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        DS_HIP(e);
-        w.graphs.push_back({xh, xl, tol2, exec});
-    }
-    DS_HIP(hipGraphLaunch(exec, c->stream));
-}
-
-void mg_release(ds_context* c) {
-    for (const MgWork::Graph& g : c->mg.graphs) (void)hipGraphExecDestroy(g.exec);
-    c->mg.graphs.clear();
+    launch_cycle(c, k, true, xh, xl, tol2, 0u);
 }
 
 }  // namespace ds
