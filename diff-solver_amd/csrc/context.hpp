@@ -80,8 +80,7 @@ constexpr uint32_t kPcgBlocks = 512;
 constexpr uint32_t kForceBlocks = 2048;
 // Blocks of the example metric reduction (one partial per block per metric, finished in order).
 constexpr uint32_t kMetricBlocks = 512;
-// PCG iteration kernels: 1024-thread blocks, each over a contiguous range of whole multiples of
-// kPcgUnroll * 1024 cells; the block count (<= kPcgMaxBlocks, a multiple of 8) is per context.
+// PCG iteration kernels: the block count (<= kPcgMaxBlocks, a multiple of 8) is per context.
 // (measured on the 128^3 plume: 512 threads / ~512 blocks, i.e. two independent 8-wave blocks per
 // CU, 29.3 us per fused iteration; 1024 / 256: 32.1 us; 512 / 256: 30.8 us; 1024 / 512: 44.3 us)
 constexpr uint32_t kPcgThreads = 512;
@@ -89,7 +88,6 @@ constexpr uint32_t kPcgThreads = 512;
 constexpr uint64_t kPcgTargetBlocks = 512;
 // the s-step kernel: one 512-thread block per CU, each with a longer z chunk and deeper prefetch
 constexpr uint64_t kPcgTargetBlocksS2 = 256;
-constexpr uint32_t kPcgUnroll = 4;
 constexpr uint32_t kPcgMaxBlocks = 1024;
 
 enum Partial : int {

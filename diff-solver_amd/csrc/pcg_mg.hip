@@ -728,10 +728,10 @@ __device__ __forceinline__ float mg_bottom_apply(const BottomCell& c, const floa
 // at most kMgBottomCells cells in one workgroup: vectors in LDS, the rows of the first two levels in
 // registers, and the coarsest level's inverse (n x n, FP64, n <= kMgDense) spread over the threads.
 // Levels: how many (the last is the dense one; 0: only the test).
-// k: updates applied so far. mode: bit 1 the first
-// test of a solve (||b||^2 from its partials, the initial residual kept), bit 2 the guess is rejected
-// when its residual exceeds ||b||, bit 3 when it is not finite. A rejection stops the solve: the
-// host, which reads the status once at its end, runs it again without the guess.
+// k: updates applied so far. mode: bit 1 the first test of a solve (||b||^2 from its partials, the
+// initial residual kept), bit 2 the guess is rejected when its residual exceeds ||b||, bit 3 when it
+// is not finite. A rejection stops the solve: the host, which reads the status once at its end, runs
+// it again without the guess.
 constexpr int kBottomThreads = 1024;
 constexpr int kBottomWords = 13;
 template <int Levels>
@@ -1257,7 +1257,6 @@ void mg_set_iteration(ds_context* c, uint32_t k) {
     mg_set_iteration_kernel<<<1, 64, 0, c->stream>>>(c->pcg.status, k);
     check_launch("mg_set_iteration_kernel");
 }
-
 
 // Eight direct launches at 128^3, six at 64^3: the host queues them faster (2.9 us each) than the GPU
 // runs them. (Replayed as a graph per iteration they cost about 8 us more at each graph's edge:
