@@ -533,6 +533,8 @@ ds_status ds_context_destroy(ds_context* c) {
         set_error("ds_context_destroy: stream synchronisation failed");
         st = DS_ERROR_RUNTIME;
     }
+    c->buffers.trim(true, c->stream);
+    if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : c->allocations) (void)hipFree(p);
     unet_release(c->unet);
     if (c->pcg.host_status) (void)hipHostFree(c->pcg.host_status);

@@ -232,6 +232,32 @@ struct MgWork {
 
 }  // namespace ds
 
+namespace ds {
+
+// Device buffers of the trajectory calls (checkpoints, segment states, step caches, tapes), kept by
+// the context between calls. Freed through the stream-ordered allocator they went back to the
+// operating system at every call's last synchronisation and were mapped again in the next call:
+// 39 + 4 ms of a 154 ms gradient (128^3, 32 steps). One stream per context, so a buffer that is
+// given back is taken again in stream order. Kept: what the last call used, at most 1/16 of the
+// card's memory, and only while a quarter of the card is free; all of it is freed when an
+// allocation fails and with the context.
+struct Buffers {
+    struct Block {
+        void* p;
+        size_t bytes;
+        uint64_t call;   // trajectory call that used it last
+    };
+    std::vector<Block> idle;
+    size_t idle_bytes = 0, limit = 0;
+    uint64_t call = 0;
+    void* take(size_t bytes, hipStream_t s);
+    void give(void* p, size_t bytes, hipStream_t s) noexcept;
+    // frees the idle buffers that the call before did not use (all: every one)
+    void trim(bool all, hipStream_t s) noexcept;
+};
+
+}  // namespace ds
+
 struct ds_context {
     ds_config config{};
     std::vector<ds_collider> colliders;
@@ -325,6 +351,7 @@ struct ds_context {
     ds::UNet* unet = nullptr;         // warm-start network, loaded by ds_warm_start_load
 
     std::vector<void*> allocations;   // everything above, released at destroy
+    ds::Buffers buffers;              // states and step caches of the trajectory calls
 };
 
 namespace ds {

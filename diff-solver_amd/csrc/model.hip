@@ -242,30 +242,90 @@ ds_solve_info vjp_step(ds_context* c, const ds_parameters* p, const ds_state* st
     return si;
 }
 
+void* Buffers::take(size_t bytes, hipStream_t s) {
+    for (size_t i = idle.size(); i-- > 0;)   // the one given back last: its lines may still be cached
+        if (idle[i].bytes == bytes) {
+            void* p = idle[i].p;
+            idle.erase(idle.begin() + (std::ptrdiff_t)i);
+            idle_bytes -= bytes;
+            return p;
+        }
+    void* p = nullptr;
+    if (hipMallocAsync(&p, bytes, s) == hipSuccess) return p;
+    (void)hipGetLastError();
+    trim(true, s);
+    DS_HIP(hipStreamSynchronize(s));
+    DS_HIP(hipMallocAsync(&p, bytes, s));
+    return p;
+}
+
+void Buffers::give(void* p, size_t bytes, hipStream_t s) noexcept {
+    if (limit == 0) {
+        size_t free_bytes = 0, total = 0;
+        if (hipMemGetInfo(&free_bytes, &total) == hipSuccess) limit = total / 16;
+    }
+    if (idle_bytes + bytes <= limit) {
+        try {
+            idle.push_back({p, bytes, call});
+            idle_bytes += bytes;
+            return;
+        } catch (...) {
+        }
+    }
+    (void)hipFreeAsync(p, s);
+}
+
+void Buffers::trim(bool all, hipStream_t s) noexcept {
+    size_t kept = 0;
+    for (const Block& b : idle) {
+        if (!all && b.call == call) {
+            idle[kept++] = b;
+        } else {
+            (void)hipFreeAsync(b.p, s);
+            idle_bytes -= b.bytes;
+        }
+    }
+    idle.resize(kept, Block{});
+}
+
 namespace {
+
+// One trajectory call: the buffers that it did not use are freed at its end, and every one when
+// less than a quarter of the card's memory is left.
+struct Trajectory {
+    ds_context* c;
+    explicit Trajectory(ds_context* ctx) : c(ctx) { ++c->buffers.call; }
+    ~Trajectory() {
+        size_t free_bytes = 0, total = 0;
+        const bool short_of = hipMemGetInfo(&free_bytes, &total) != hipSuccess || free_bytes < total / 4;
+        c->buffers.trim(short_of, c->stream);
+    }
+    Trajectory(const Trajectory&) = delete;
+    Trajectory& operator=(const Trajectory&) = delete;
+};
 
 // ---- adapter of the C-ABI views to the templates of xayah/solver.hpp ----------------------------
 template <typename T>
-struct DBuf {   // stream-ordered device buffer
+struct DBuf {   // stream-ordered device buffer of the context
     T* p = nullptr;
-    hipStream_t s = nullptr;
+    size_t bytes = 0;
+    ds_context* c = nullptr;
     DBuf() = default;
-    DBuf(hipStream_t stream, size_t n) : s(stream) {
-        void* q = nullptr;
-        DS_HIP(hipMallocAsync(&q, n * sizeof(T) > 0 ? n * sizeof(T) : 1, stream));
-        p = static_cast<T*>(q);
+    DBuf(ds_context* ctx, size_t n) : bytes(n * sizeof(T) > 0 ? n * sizeof(T) : 1), c(ctx) {
+        p = static_cast<T*>(c->buffers.take(bytes, c->stream));
     }
     ~DBuf() {
-        if (p) (void)hipFreeAsync(p, s);
+        if (p) c->buffers.give(p, bytes, c->stream);
     }
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
-    DBuf(DBuf&& o) noexcept : p(std::exchange(o.p, nullptr)), s(o.s) {}
+    DBuf(DBuf&& o) noexcept : p(std::exchange(o.p, nullptr)), bytes(o.bytes), c(o.c) {}
     DBuf& operator=(DBuf&& o) noexcept {
         if (this != &o) {
-            if (p) (void)hipFreeAsync(p, s);
+            if (p) c->buffers.give(p, bytes, c->stream);
             p = std::exchange(o.p, nullptr);
-            s = o.s;
+            bytes = o.bytes;
+            c = o.c;
         }
         return *this;
     }
@@ -305,9 +365,9 @@ struct AbiModel {
     AState allocate_state(ACtx& x) const {
         const Geo& g = x.c->geo;
         AState s;
-        s.own.emplace_back(x.c->stream, g.n);
-        s.own.emplace_back(x.c->stream, g.n);
-        for (int a = 0; a < 3; ++a) s.own.emplace_back(x.c->stream, g.nf[a]);
+        s.own.emplace_back(x.c, g.n);
+        s.own.emplace_back(x.c, g.n);
+        for (int a = 0; a < 3; ++a) s.own.emplace_back(x.c, g.nf[a]);
         s.v.density = s.own[0].p;
         s.v.temperature = s.own[1].p;
         for (int a = 0; a < 3; ++a) s.v.velocity[a] = s.own[2 + a].p;
@@ -316,9 +376,9 @@ struct AbiModel {
     ACache allocate_step_cache(ACtx& x) const {
         const Geo& g = x.c->geo;
         ACache k;
-        k.rs = DBuf<float>(x.c->stream, g.n);
-        k.ts = DBuf<float>(x.c->stream, g.n);
-        for (int a = 0; a < 3; ++a) k.us[a] = DBuf<float>(x.c->stream, g.nf[a]);
+        k.rs = DBuf<float>(x.c, g.n);
+        k.ts = DBuf<float>(x.c, g.n);
+        for (int a = 0; a < 3; ++a) k.us[a] = DBuf<float>(x.c, g.nf[a]);
         k.v.sourced_density = k.rs.p;
         k.v.sourced_temperature = k.ts.p;
         for (int a = 0; a < 3; ++a) k.v.forced_velocity[a] = k.us[a].p;
@@ -333,7 +393,7 @@ struct AbiModel {
     ds_parameter_adjoint allocate_parameter_adjoint(ACtx&) const { return {}; }
     ATape allocate_pressure_tape(ACtx& x) const {
         ATape t;
-        t.buf = DBuf<float>(x.c->stream, 2 * (size_t)x.c->geo.n);
+        t.buf = DBuf<float>(x.c, 2 * (size_t)x.c->geo.n);
         t.data = t.buf.p;
         return t;
     }
@@ -501,6 +561,7 @@ ds_status ds_trajectory_jvp(ds_context* c, const ds_state* initial, const ds_con
         info->steps = steps;
     }
     const ds_status st = guard([&] {
+        const Trajectory call(c);
         check_state(initial, "ds_trajectory_jvp: initial state has a null field");
         check_state(initial_tangent, "ds_trajectory_jvp: initial tangent has a null field");
         check_state(final_state, "ds_trajectory_jvp: final state has a null field");
@@ -537,6 +598,7 @@ ds_status ds_simulate(ds_context* c, const ds_state* initial, const ds_control* 
         info->checkpoint_interval = steps;
     }
     const ds_status st = guard([&] {
+        const Trajectory call(c);
         check_state(initial, "ds_simulate: initial state has a null field");
         check_state(final_state, "ds_simulate: final state has a null field");
         c->pressure_prev_count = 0;   // an extrapolated or projected guess spans solves of one sweep only
@@ -584,6 +646,7 @@ ds_status trajectory_gradient(const char* who, ds_context* c, const ds_state* in
     ti->checkpoint_interval = checkpoint_interval ? checkpoint_interval : 1u;
     ACtx x{c, ti};
     const ds_status st = guard([&] {
+        const Trajectory call(c);
         check_state(initial, "initial state has a null field");
         const ds_state init_view = as_state(*initial_adj);
         check_state(&init_view, "initial adjoint has a null field");
@@ -602,7 +665,7 @@ ds_status trajectory_gradient(const char* who, ds_context* c, const ds_state* in
         // terminal adjoint (and loss)
         AState final_adj = m.allocate_state_adjoint(x);
         if (target_density) {
-            DBuf<double> partials(c->stream, 1024), loss(c->stream, 1);
+            DBuf<double> partials(c, 1024), loss(c, 1);
             density_loss_kernel<<<1024, kBlock, 0, c->stream>>>(c->geo.n, t.final_state->v.density, target_density, final_adj.v.density,
                                                                 partials.p);
             sum_partials_kernel<<<1, kBlock, 0, c->stream>>>(partials.p, 1024, loss.p);
