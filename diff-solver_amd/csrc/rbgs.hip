@@ -5,7 +5,8 @@
 // :1015-1018: the same sweeps with the fixed boundary values zeroed).
 //
 // A sweep updates one colour, so one launch covers only that colour's cells (x advances by 2
-// within a row). The reverse of a sweep of colour P scatters p_bar[i] / diag_i (i of colour P) to
+// within a row); the forward sweeps run two iterations to a launch in boxes with a halo
+// (rbgs_box_kernel). The reverse of a sweep of colour P scatters p_bar[i] / diag_i (i of colour P) to
 // i's connected neighbours, adds it to rhs_bar[i] and clears p_bar[i]; here it is a gather: the
 // neighbours (colour 1 - P) read p_bar[i] / diag_i, and the clearing and the rhs_bar update of
 // colour P are deferred into the next launch, which runs over colour P. So each launch writes
@@ -14,6 +15,8 @@
 // A periodic axis with an odd cell count puts cells of one colour side by side across the seam;
 // the reference's kernel then reads a neighbour that the same launch writes, and so does this one.
 #include <hip/hip_runtime.h>
+
+#include <utility>
 
 #include "context.hpp"
 #include "kernels.hpp"
@@ -128,6 +131,161 @@ __global__ __launch_bounds__(256) void rbgs_sweep_kernel(Geo g, const SBound* __
     p[i] = sum / (float)d;
 }
 
+// `iterations` <= S red-black iterations (a red and a black sweep each) in one launch. A workgroup
+// loads a box and 2 S cells around it; every sweep shrinks what is up to date by one cell, so after
+// the last one the box is, and it is written to the other buffer (p_in is still read by others).
+//
+// Thread (k, j) holds two cells of row j, x = 2k and 2k + 1 (one less in odd rows), on every plane of
+// the box: p, rhs and the diagonal in registers. So shifted, the first cell has the colour of its
+// plane's parity in every row, and which cell a sweep updates is known at compile time. The partner
+// and the neighbours along z are the thread's own registers, the other three come from LDS (one array
+// for the first cells, one for the second: consecutive lanes on consecutive words). A box starts at
+// even coordinates, so the parity of the local coordinates is the colour; a periodic axis of odd
+// extent has no such colouring.
+//
+// A cell outside the domain holds what a sweep adds for it, the face's fixed value or 0, and a solid
+// one holds 0; neither is updated. So the sum is the six neighbours in the order of
+// rbgs_sweep_kernel, without tests: the same values (a zero can have the other sign).
+//
+// Bound by the loads of the halo (4 1/2 times the box, in lines of 128 bytes) and the latency of a
+// workgroup's load, sweep and store phases. At 128 x 192 x 128, us per iteration: a launch per colour
+// 35.4 (seven mask tests and loads, an index division and a rounded division per cell); boxes of
+// 32 x 16 x 8, two iterations a launch, 11.7 (23.5 a launch: 14.1 without the paired loads, 18.7
+// with the selects of unshifted rows and the full division); one iteration a launch: 32 x 16 x 8
+// 19.2, 64 x 8 x 8 16.0, 64 x 16 x 8 17.8, 128 x 8 x 8 18.8; two: 64 x 16 x 8 15.2, 32 x 16 x 16
+// 19.8, 32 x 24 x 8 16.0; three, 32 x 16 x 8: 21.3. Small grids (two steps of 160 iterations): 24^3
+// 3707 -> 1245 us, 64^3 3472 -> 1352, 96 x 100 x 75 5535 -> 2152.
+template <int S_, int X_, int Y_, int Z_>
+struct SweepBox {
+    static constexpr int S = S_, X = X_, Y = Y_, Z = Z_, H = 2 * S_;   // iterations, box, halo
+    static constexpr int K = X / 2 + H + 1, RY = Y + 2 * H, RZ = Z + 2 * H, P = K * RY;
+    static constexpr int T = (P + 63) / 64 * 64;
+};
+
+// Index of coordinate v along an axis of n cells, or -1 outside, where `value` becomes what a sweep adds.
+__device__ __forceinline__ int sweep_coord(const SBound& b, int d, int v, int n, float& value) {
+    if ((unsigned)v < (unsigned)n) return v;
+    if (b.modes[2 * d] == 2u && b.modes[2 * d + 1] == 2u) return wrapi(v, n);
+    const int face = 2 * d + (v < 0 ? 0 : 1);
+    value = b.modes[face] == 0u ? b.values[face] : 0.0f;
+    return -1;
+}
+
+// sum / d, rounded to nearest, for d = 1 .. 6: the reciprocal of such a d is the nearest FP32 number,
+// so one corrected step gives the nearest quotient (Markstein 1990; tiny results, below 2^-100, can
+// be one unit off); the fix-up is for zeros, infinities and NaN. d = 0 gives what the caller drops.
+__device__ __forceinline__ float divide_small(float sum, float d) {
+    const float rd = __builtin_amdgcn_rcpf(d);
+    const float q = sum * rd;
+    return __builtin_amdgcn_div_fixupf(__fmaf_rn(__fmaf_rn(-d, q, sum), rd, q), d, sum);
+}
+
+// Wide: the thread's two cells in one load; x is not periodic then and nx >= 2 (a pair that has one
+// cell outside reads the pair next to it).
+template <typename B, bool Wide>
+__global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __restrict__ bp, const uint8_t* __restrict__ diag,
+                                                        const float* __restrict__ rhs, const float* __restrict__ p_in,
+                                                        float* __restrict__ p_out, uint32_t ntx, uint32_t nty, uint32_t boxes, int ex, int ey,
+                                                        int ez, int iterations) {
+    constexpr int H = B::H, K = B::K, RY = B::RY, RZ = B::RZ, P = B::P, Pad = K + 2;
+    __shared__ float s[2][RZ * P + 2 * Pad];
+    const uint32_t b = xcd_block();
+    if (b >= boxes) return;
+    const int bx = (int)(b % ntx), by = (int)(b / ntx % nty), bz = (int)(b / ntx / nty);
+    const int t = (int)threadIdx.x, j = t / K, k = t - j * K, odd = j & 1;
+    const bool active = j < RY;
+    const int x = bx * ex - H + 2 * k - odd, y = by * ey - H + j, z0 = bz * ez - H;
+    float out[2]{}, out_y = 0.0f;
+    const int iy = sweep_coord(*bp, 1, y, g.ny, out_y);
+    const int ix[2]{sweep_coord(*bp, 0, x, g.nx, out[0]), sweep_coord(*bp, 0, x + 1, g.nx, out[1])};
+    bool in[2];
+    uint32_t at[2], keep[2];   // keep: 0 where there is nothing to update, or a neighbour is not loaded
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        in[f] = active && iy >= 0 && ix[f] >= 0;
+        if (iy < 0) out[f] = out_y;
+        at[f] = in[f] ? (uint32_t)iy * (uint32_t)g.nx + (uint32_t)ix[f] : 0u;
+        keep[f] = in[f] && j != 0 && j != RY - 1 && k != (f == 0 ? 0 : K - 1) ? 7u : 0u;
+    }
+    const uint32_t pair = in[0] || in[1] ? (uint32_t)iy * (uint32_t)g.nx + (uint32_t)min(max(x, 0), g.nx - 2) : 0u;
+    const bool first_high = x == g.nx - 1, second_low = x == -1;
+    const uint32_t plane = (uint32_t)g.nx * (uint32_t)g.ny;
+    float p[2][RZ], r[2][RZ];
+    uint32_t d[2][(RZ + 3) / 4]{};
+    float out_z[2]{};
+    const bool wraps = sweep_coord(*bp, 2, -1, g.nz, out_z[0]) >= 0;
+    (void)sweep_coord(*bp, 2, g.nz, g.nz, out_z[1]);
+    int wz = wraps ? wrapi(z0, g.nz) : 0;
+#pragma unroll
+    for (int z = 0; z < RZ; ++z) {
+        const bool inside = wraps || (unsigned)(z0 + z) < (unsigned)g.nz;
+        const float outside = z0 + z < 0 ? out_z[0] : out_z[1];
+        const size_t base = (size_t)(wraps ? wz : min(max(z0 + z, 0), g.nz - 1)) * plane;
+        wz = wz + 1 == g.nz ? 0 : wz + 1;
+        float pv[2], rv[2];
+        uint32_t dv[2];
+        if constexpr (Wide) {
+            uint16_t dw;
+            __builtin_memcpy(pv, p_in + base + pair, sizeof pv);
+            __builtin_memcpy(rv, rhs + base + pair, sizeof rv);
+            __builtin_memcpy(&dw, diag + base + pair, sizeof dw);
+            dv[0] = first_high ? dw >> 8 : dw;   // (the bits above are masked below)
+            dv[1] = second_low ? dw : dw >> 8;
+            const float p0 = pv[0], r0 = rv[0];
+            pv[0] = first_high ? pv[1] : pv[0], rv[0] = first_high ? rv[1] : rv[0];
+            pv[1] = second_low ? p0 : pv[1], rv[1] = second_low ? r0 : rv[1];
+        } else {
+#pragma unroll
+            for (int f = 0; f < 2; ++f) pv[f] = p_in[base + at[f]], rv[f] = rhs[base + at[f]], dv[f] = diag[base + at[f]];
+        }
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            r[f][z] = rv[f];
+            p[f][z] = in[f] && inside ? pv[f] : inside ? out[f] : outside;
+            d[f][z / 4] |= (dv[f] & (inside ? keep[f] : 0u)) << (8 * (z % 4));
+        }
+    }
+    if (active) {
+#pragma unroll
+        for (int z = 1; z < RZ - 1; ++z) s[(z + 1) & 1][Pad + z * P + t] = p[(z + 1) & 1][z];   // the black cells
+    }
+    __syncthreads();
+    // sweep N of the launch, of colour N & 1: the planes that are not up to date any more are left out
+    auto sweep = [&]<int N>() {
+        constexpr int C = N & 1;
+        if (active) {
+#pragma unroll
+            for (int z = N + 1; z < RZ - 1 - N; ++z) {
+                const int f = (z + C) & 1;
+                const float* o = &s[1 - f][Pad + z * P + t];
+                const float* row = o + f - odd;
+                float sum = r[f][z] + (f == 0 ? o[-1] : p[0][z]);
+                sum += f == 0 ? p[1][z] : o[1];
+                sum += row[-K];
+                sum += row[K];
+                sum += p[f][z - 1];
+                sum += p[f][z + 1];
+                const float dz = (float)((d[f][z / 4] >> (8 * (z % 4))) & 255u);
+                p[f][z] = dz != 0.0f ? divide_small(sum, dz) : p[f][z];
+                s[f][Pad + z * P + t] = p[f][z];
+            }
+        }
+        __syncthreads();
+    };
+    [&]<int... It>(std::integer_sequence<int, It...>) {
+        ((It < iterations ? (sweep.template operator()<2 * It>(), sweep.template operator()<2 * It + 1>()) : void()), ...);
+    }(std::make_integer_sequence<int, B::S>{});
+    if (j < H || j >= H + ey) return;
+    const int lx = 2 * k - odd;
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        if (!in[f] || lx + f < H || lx + f >= H + ex || y >= g.ny || x + f >= g.nx) continue;   // (not a periodic image)
+#pragma unroll
+        for (int z = H; z < RZ - H; ++z)
+            if (z < H + ez && z0 + z < g.nz) p_out[(size_t)(z0 + z) * plane + at[f]] = p[f][z];
+    }
+}
+
 // One launch of the reverse over the cells of colour `parity`: with Finish, the deferred second
 // half of the previous reverse sweep (that colour's rhs_bar += p_bar / diag, p_bar = 0); with
 // Gather, the first half of the next one (p_bar += sum over connected neighbours of p_bar / diag).
@@ -166,6 +324,30 @@ __global__ __launch_bounds__(256) void rbgs_reverse_kernel(Geo g, const SBound* 
     pbar[i] = own;
 }
 
+template <typename B>
+uint64_t box_count(const Geo& g) {
+    auto count = [](int n, int most) { return ((uint64_t)n + (uint64_t)most - 1) / (uint64_t)most; };
+    return count(g.nx, B::X) * count(g.ny, B::Y) * count(g.nz, B::Z);
+}
+
+// One launch of rbgs_box_kernel; boxes of equal even extents that cover the grid.
+template <typename B>
+void launch_boxes(ds_context* c, const SBound* bp, const float* b, const float* p_in, float* p_out, uint32_t iterations) {
+    const Geo& g = c->geo;
+    auto split = [](int n, int most, uint32_t& count) {
+        count = ((uint32_t)n + (uint32_t)most - 1) / (uint32_t)most;
+        return (int)((((uint32_t)n + count - 1) / count + 1u) & ~1u);
+    };
+    uint32_t cx, cy, cz;
+    const int ex = split(g.nx, B::X, cx), ey = split(g.ny, B::Y, cy), ez = split(g.nz, B::Z, cz);
+    const uint32_t boxes = cx * cy * cz, blocks = (boxes + 7u) & ~7u;
+    auto launch = [&](auto kernel) {
+        kernel<<<blocks, B::T, 0, c->stream>>>(g, bp, c->rbgs_diag, b, p_in, p_out, cx, cy, boxes, ex, ey, ez, (int)iterations);
+    };
+    if (!c->pressure_periodic[0] && g.nx >= 2) launch(rbgs_box_kernel<B, true>);
+    else launch(rbgs_box_kernel<B, false>);
+}
+
 uint32_t colour_blocks(const Geo& g) {
     const uint64_t threads = (uint64_t)(((uint32_t)g.nx + 1u) / 2u) * (uint64_t)g.ny * (uint64_t)g.nz;
     return (uint32_t)((threads + kBlock - 1) / kBlock);
@@ -197,7 +379,30 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
     const uint32_t CB = colour_blocks(g);
     if (kind != kRhsAdjoint) {
         const SBound* bp = kind == kRhsTangent ? c->d_pb_zero : c->d_pb;
-        for (uint32_t it = 0; it < iterations; ++it) {
+        const bool coloured = (!c->pressure_periodic[0] || g.nx % 2 == 0) && (!c->pressure_periodic[1] || g.ny % 2 == 0) &&
+                              (!c->pressure_periodic[2] || g.nz % 2 == 0);
+        // boxes wherever the colouring holds: the launches of one colour remain for a periodic axis of
+        // odd extent, where a sweep reads a neighbour that it writes itself
+        if (coloured && iterations > 0) {
+            auto sweeps = [&]<typename B>() {
+                const uint32_t launches = (iterations + B::S - 1) / B::S;
+                float* from = launches % 2 ? xl : xh;   // both are zero; the last launch writes xh
+                for (uint32_t l = 0, done = 0; l < launches; ++l, done += B::S) {
+                    float* to = from == xh ? xl : xh;
+                    launch_boxes<B>(c, bp, b, from, to, std::min<uint32_t>(B::S, iterations - done));
+                    from = to;
+                }
+            };
+            // A small grid is bound by the latency of one workgroup, so its boxes are flat while they
+            // are at most one for each of the 256 CUs: 64^3 (256 flat boxes, 64 deep ones), two steps of
+            // 160 iterations, 1352 against 1929 us, 24^3 1245 against 1750; beyond that the halo
+            // decides: 96 x 100 x 75 (798 flat boxes, 210 deep ones) 2788 against 2152 us.
+            using Flat = SweepBox<2, 32, 16, 2>;
+            using Deep = SweepBox<2, 32, 16, 8>;
+            if (box_count<Flat>(g) <= 256u) sweeps.template operator()<Flat>();
+            else sweeps.template operator()<Deep>();
+            fill_zero(c, xl, g.n);
+        } else for (uint32_t it = 0; it < iterations; ++it) {
             rbgs_sweep_kernel<<<CB, kBlock, 0, c->stream>>>(g, bp, c->mask, c->rbgs_diag, b, xh, 0u);
             rbgs_sweep_kernel<<<CB, kBlock, 0, c->stream>>>(g, bp, c->mask, c->rbgs_diag, b, xh, 1u);
         }
