@@ -473,37 +473,21 @@ __global__ __launch_bounds__(256) void maxpool2_backward_kernel(Dims dc, uint32_
     }
 }
 
-// Weight gradient of a 3x3x3 convolution (KIND 0) or a 2x2x2 stride-2 transposed convolution
-// (KIND 1), one tap per blockIdx.y:
-//   KIND 0: dW[co][ci][tap] = sum_v dz(v)[co] x(v + off(tap))[ci]   (M = co: dz, N = ci: x = [in1, in2])
-//   KIND 1: dW[ci][co][t]  = sum_v in(v)[ci] dout(2 v + t)[co]       (M = ci: in1, N = co: dout)
-// The M tensor has MC channels at the wave's voxels (16 consecutive in x per step); the N tensor has
-// C1 + C2 channels (KIND 0; in1 stored with stride max(C1, 4)) or C1 (KIND 1). Wave w of the grid
-// leaves its sum in partials[(w * taps + tap) * MC * NC + m * NC + n] (NC = N channels rounded up to
-// 16); wgrad_reduce_kernel adds the waves' slots.
-template <int KIND, int MC, int C1, int C2>
-__global__ __launch_bounds__(256) void wgrad_kernel(Dims d, int batch, const uint16_t* __restrict__ mt, const uint16_t* __restrict__ in1,
-                                                    const uint16_t* __restrict__ in2, uint32_t groups_per_wave,
-                                                    float* __restrict__ partials) {
-    constexpr int NC = ((C1 + C2 + 15) / 16) * 16, NBM = MC / 16, NBN = NC / 16;
-    constexpr int NCH1 = (C1 + 15) / 16;
-    constexpr int S1 = C1 < 4 ? 4 : C1;
-    constexpr int TAPS = KIND == 0 ? 27 : 8;
+// Weight gradient of a 2x2x2 stride-2 transposed convolution, one tap per blockIdx.y:
+//   dW[ci][co][t] = sum_v in(v)[ci] dout(2 v + t)[co]   (M = ci: mt, N = co: in1)
+// The M tensor has MC channels at the wave's voxels (16 consecutive in x per step), the N tensor C1.
+// Wave w of the grid leaves its sum in partials[(w * 8 + tap) * MC * C1 + m * C1 + n];
+// wgrad_reduce_kernel adds the waves' slots.
+template <int MC, int C1>
+__global__ __launch_bounds__(256) void wgrad_tconv_kernel(Dims d, int batch, const uint16_t* __restrict__ mt, const uint16_t* __restrict__ in1,
+                                                          uint32_t groups_per_wave, float* __restrict__ partials) {
+    constexpr int NC = C1, NBM = MC / 16, NBN = NC / 16;
     const int lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
     const int tap = blockIdx.y;
     const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6);
     const int tiles_x = d.nx / 16;
     const uint32_t groups = (uint32_t)tiles_x * d.ny * d.nz * batch;
-    int dx = 0, dy = 0, dz = 0;
-    if (KIND == 0) {
-        dz = tap / 9 - 1;
-        dy = (tap / 3) % 3 - 1;
-        dx = tap % 3 - 1;
-    } else {
-        dz = tap >> 2;
-        dy = (tap >> 1) & 1;
-        dx = tap & 1;
-    }
+    const int dz = tap >> 2, dy = (tap >> 1) & 1, dx = tap & 1;
     const Dims df{2 * d.nx, 2 * d.ny, 2 * d.nz};
     floatx4_t acc[NBM][NBN];
 #pragma unroll
@@ -516,7 +500,6 @@ __global__ __launch_bounds__(256) void wgrad_kernel(Dims d, int batch, const uin
         const int tx = (int)(gi % (uint32_t)tiles_x);
         const int y = (int)((gi / (uint32_t)tiles_x) % (uint32_t)d.ny);
         const int zg = (int)(gi / ((uint32_t)tiles_x * d.ny));
-        const int zl = zg % d.nz;
         const int xb = tx * 16 + 4 * kq;   // this lane's 4 voxels: xb .. xb + 3
         bf16x4_t a[NBM], b[NBN];
 #pragma unroll
@@ -524,7 +507,74 @@ __global__ __launch_bounds__(256) void wgrad_kernel(Dims d, int batch, const uin
             const uint16_t* p = mt + (size_t)vox(d, xb, y, zg) * MC + ab * 16 + m;
             a[ab] = bf16x4_t{(short)p[0], (short)p[MC], (short)p[2 * MC], (short)p[3 * MC]};
         }
-        if (KIND == 0) {
+#pragma unroll
+        for (int bb = 0; bb < NBN; ++bb) {
+            const int c = bb * 16 + m;
+            short v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = (short)in1[(size_t)vox(df, 2 * (xb + j) + dx, 2 * y + dy, 2 * zg + dz) * C1 + c];
+            b[bb] = bf16x4_t{v[0], v[1], v[2], v[3]};
+        }
+#pragma unroll
+        for (int ab = 0; ab < NBM; ++ab)
+#pragma unroll
+            for (int bb = 0; bb < NBN; ++bb) acc[ab][bb] = mfma(a[ab], b[bb], acc[ab][bb]);
+    }
+    float* out = partials + ((size_t)wave * 8 + tap) * MC * NC;
+#pragma unroll
+    for (int ab = 0; ab < NBM; ++ab)
+#pragma unroll
+        for (int bb = 0; bb < NBN; ++bb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[(size_t)(ab * 16 + 4 * kq + i) * NC + bb * 16 + m] = acc[ab][bb][i];
+}
+
+// Weight gradient of a 3x3x3 convolution:
+//   dW[co][ci][tap] = sum_v dz(v)[co] x(v + off(tap))[ci]   (M = co: dz, N = ci: x = [in1, in2])
+// in1 is stored with stride max(C1, 4); wave w leaves its sums in partials[(w * 27 + tap) * MC * NC +
+// m * NC + n] (NC = N channels rounded up to 16). A wave takes ROWS (3 or 1) rows of three taps along
+// x: they share the M fragments, and a row's three N fragments come from six voxels instead of
+// twelve. (A tap a wave was bound by its 2-byte loads and their addresses, eight for one matrix
+// instruction. 64^3 batch of 4, 16 -> 16 channels:
+// 314 us,
+// now 102; 16 + 16 -> 16: 379, now 125; 2 -> 16: 293, now 131; 32 -> 32 on the 32^3 level: 58, now 40.)
+// ROWS 3 while the accumulators fit beside four waves a SIMD (MC * NC <= 512: 72 registers), else 1.
+template <int ROWS, int MC, int C1, int C2>
+__global__ __launch_bounds__(256) void wgrad_rows_kernel(Dims d, int batch, const uint16_t* __restrict__ mt, const uint16_t* __restrict__ in1,
+                                                         const uint16_t* __restrict__ in2, uint32_t groups_per_wave,
+                                                         float* __restrict__ partials) {
+    constexpr int NC = ((C1 + C2 + 15) / 16) * 16, NBM = MC / 16, NBN = NC / 16;
+    constexpr int NCH1 = (C1 + 15) / 16;
+    constexpr int S1 = C1 < 4 ? 4 : C1;
+    const int lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
+    const int row0 = (int)blockIdx.y * ROWS;   // rows 0 .. 8: dz = row / 3 - 1, dy = row % 3 - 1
+    const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6);
+    const int tiles_x = d.nx / 16;
+    const uint32_t groups = (uint32_t)tiles_x * d.ny * d.nz * batch;
+    floatx4_t acc[ROWS][3][NBM][NBN];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+#pragma unroll
+            for (int a = 0; a < NBM; ++a)
+#pragma unroll
+                for (int b = 0; b < NBN; ++b) acc[r][t][a][b] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t g0 = min(groups, wave * groups_per_wave);
+    const uint32_t g1 = min(groups, g0 + groups_per_wave);
+    int tx = (int)(g0 % (uint32_t)tiles_x), y = (int)((g0 / (uint32_t)tiles_x) % (uint32_t)d.ny), zg = (int)(g0 / ((uint32_t)tiles_x * d.ny));
+    for (uint32_t gi = g0; gi < g1; ++gi) {
+        const int zl = zg % d.nz;
+        const int xb = tx * 16 + 4 * kq;   // this lane's 4 voxels: xb .. xb + 3
+        bf16x4_t a[NBM];
+#pragma unroll
+        for (int ab = 0; ab < NBM; ++ab) {
+            const uint16_t* p = mt + (size_t)vox(d, xb, y, zg) * MC + ab * 16 + m;
+            a[ab] = bf16x4_t{(short)p[0], (short)p[MC], (short)p[2 * MC], (short)p[3 * MC]};
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const int dz = (row0 + r) / 3 - 1, dy = (row0 + r) % 3 - 1;
             const int yy = y + dy, zz = zl + dz;
             const bool okyz = yy >= 0 && yy < d.ny && zz >= 0 && zz < d.nz;
 #pragma unroll
@@ -532,38 +582,44 @@ __global__ __launch_bounds__(256) void wgrad_kernel(Dims d, int batch, const uin
                 const bool first = bb < NCH1;
                 const int c = (first ? bb * 16 : (bb - NCH1) * 16) + m;
                 const int cs = first ? S1 : C2;
-                const uint16_t* src = first ? in1 : in2;
-                const bool okc = first ? c < C1 : c < C2;
-                short v[4];
+                const bool ok = okyz && (first ? c < C1 : c < C2);
+                // where there is no voxel or channel the lane reads its own voxel's first channel and takes 0
+                const uint16_t* src = (first ? in1 : in2) + (size_t)vox(d, xb, ok ? yy : y, ok ? zg + dz : zg) * cs + (ok ? c : 0);
+                const bool left = ok && xb > 0, right = ok && xb + 4 < d.nx;
+                short v[6];
+                v[0] = (short)src[left ? -cs : 0];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int xx = xb + j + dx;
-                    v[j] = (okyz && okc && xx >= 0 && xx < d.nx) ? (short)src[(size_t)vox(d, xx, yy, zg + dz) * cs + c] : (short)0;
+                for (int j = 0; j < 4; ++j) v[j + 1] = (short)src[j * cs];
+                v[5] = (short)src[right ? 4 * cs : 0];
+                v[0] = left ? v[0] : (short)0;
+                v[5] = right ? v[5] : (short)0;
+#pragma unroll
+                for (int j = 1; j < 5; ++j) v[j] = ok ? v[j] : (short)0;
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    const bf16x4_t b{v[t], v[t + 1], v[t + 2], v[t + 3]};
+#pragma unroll
+                    for (int ab = 0; ab < NBM; ++ab) acc[r][t][ab][bb] = mfma(a[ab], b, acc[r][t][ab][bb]);
                 }
-                b[bb] = bf16x4_t{v[0], v[1], v[2], v[3]};
-            }
-        } else {
-#pragma unroll
-            for (int bb = 0; bb < NBN; ++bb) {
-                const int c = bb * 16 + m;
-                short v[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = (short)in1[(size_t)vox(df, 2 * (xb + j) + dx, 2 * y + dy, 2 * zg + dz) * C1 + c];
-                b[bb] = bf16x4_t{v[0], v[1], v[2], v[3]};
             }
         }
-#pragma unroll
-        for (int ab = 0; ab < NBM; ++ab)
-#pragma unroll
-            for (int bb = 0; bb < NBN; ++bb) acc[ab][bb] = mfma(a[ab], b[bb], acc[ab][bb]);
+        if (++tx == tiles_x) {
+            tx = 0;
+            if (++y == d.ny) y = 0, ++zg;
+        }
     }
-    float* out = partials + ((size_t)wave * TAPS + tap) * MC * NC;
 #pragma unroll
-    for (int ab = 0; ab < NBM; ++ab)
+    for (int r = 0; r < ROWS; ++r)
 #pragma unroll
-        for (int bb = 0; bb < NBN; ++bb)
+        for (int t = 0; t < 3; ++t) {
+            float* out = partials + ((size_t)wave * 27 + (row0 + r) * 3 + t) * MC * NC;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[(size_t)(ab * 16 + 4 * kq + i) * NC + bb * 16 + m] = acc[ab][bb][i];
+            for (int ab = 0; ab < NBM; ++ab)
+#pragma unroll
+                for (int bb = 0; bb < NBN; ++bb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) out[(size_t)(ab * 16 + 4 * kq + i) * NC + bb * 16 + m] = acc[r][t][ab][bb][i];
+        }
 }
 
 // dW[mi][ni][tap] (mi < MC, ni < NREAL) = sum over the waves' slots (FP64 sums in a fixed order). A
@@ -595,22 +651,34 @@ __global__ __launch_bounds__(64 * kReduceWaves) void wgrad_reduce_kernel(const f
 }
 
 // Per-block FP64 channel sums of a BF16 tensor with C channels over n voxels:
-// partials[block * C + c]. The block's threads cover 256 / C voxels per step.
+// partials[block * C + c]. A thread takes 8 channels of a voxel (16 bytes) at a time, the lanes of
+// the same channels meet by shuffles. (One channel a thread, 2-byte loads: 67 us for 33 MB, the 64^3
+// batch of 4; now 15, 2.2 TB/s.)
 template <int C>
 __global__ __launch_bounds__(256) void channel_sum_kernel(uint32_t n, const uint16_t* __restrict__ t, double* __restrict__ partials) {
-    static_assert(256 % C == 0, "channel count must divide 256");
-    __shared__ double lds[256];
-    constexpr uint32_t per = 256 / C;
-    const uint32_t c = threadIdx.x % C, vo = threadIdx.x / C;
-    double s = 0.0;
-    for (uint32_t v = blockIdx.x * per + vo; v < n; v += gridDim.x * per) s += (double)from_bf16(t[(size_t)v * C + c]);
-    lds[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x < C) {
-        double tot = 0.0;
-        for (uint32_t k = 0; k < per; ++k) tot += lds[k * C + threadIdx.x];
-        partials[(size_t)blockIdx.x * C + threadIdx.x] = tot;
+    static_assert(C % 8 == 0 && 64 % (C / 8) == 0, "whole groups of lanes per voxel");
+    constexpr uint32_t G = C / 8, per = 256 / G;
+    __shared__ double lds[4][C];
+    const uint32_t c8 = threadIdx.x % G, vo = threadIdx.x / G;
+    double s[8]{};
+#pragma unroll 4
+    for (uint32_t v = blockIdx.x * per + vo; v < n; v += gridDim.x * per) {
+        uint32_t u[4];
+        __builtin_memcpy(u, t + (size_t)v * C + 8 * c8, sizeof u);   // (a caller's tensor may be aligned to 2 bytes)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            s[2 * k] += (double)__uint_as_float(u[k] << 16);
+            s[2 * k + 1] += (double)__uint_as_float(u[k] & 0xffff0000u);
+        }
     }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+#pragma unroll
+        for (int m = (int)G; m < 64; m *= 2) s[k] += __shfl_xor(s[k], m, 64);
+        if ((threadIdx.x & 63u) < G) lds[threadIdx.x >> 6][8 * c8 + k] = s[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < C) partials[(size_t)blockIdx.x * C + threadIdx.x] = lds[0][threadIdx.x] + lds[1][threadIdx.x] + lds[2][threadIdx.x] + lds[3][threadIdx.x];
 }
 
 // out[c] = sum over `blocks` partial rows of c channels (fixed order; c divides 256): thread t adds

@@ -150,11 +150,12 @@ void conv_wgrad(int c1, int c2, int cout, const Dims& d, int batch, const uint16
     const uint64_t groups = (uint64_t)(d.nx / 16) * d.ny * d.nz * batch;
     const int nc = ((c1 + c2 + 15) / 16) * 16;
     const WgradPlan p = wgrad_plan(groups, 27, cout, nc);
-    const dim3 grid(p.blocks, 27);
     bool done = false;
 #define DS_WGRAD(A, B, C)                                                                                    \
     if (!done && c1 == A && c2 == B && cout == C) {                                                          \
-        wgrad_kernel<0, C, A, B><<<grid, 256, 0, s>>>(d, batch, dz, in1, in2, p.per_wave, slots);          \
+        constexpr int rows = C * ((A + B + 15) / 16 * 16) <= 512 ? 3 : 1;                                    \
+        const dim3 grid(p.blocks, 9 / rows);                                                                 \
+        wgrad_rows_kernel<rows, C, A, B><<<grid, 256, 0, s>>>(d, batch, dz, in1, in2, p.per_wave, slots);    \
         done = true;                                                                                         \
     }
     DS_WGRAD(2, 0, 16)
@@ -195,8 +196,8 @@ void tconv_wgrad(int cin, int cout, const Dims& dc, int batch, const uint16_t* i
     const uint64_t groups = (uint64_t)(dc.nx / 16) * dc.ny * dc.nz * batch;
     const WgradPlan p = wgrad_plan(groups, 8, cin, cout);
     const dim3 grid(p.blocks, 8);
-    if (cin == 64 && cout == 32) wgrad_kernel<1, 64, 32, 0><<<grid, 256, 0, s>>>(dc, batch, in, dout, nullptr, p.per_wave, slots);
-    else if (cin == 32 && cout == 16) wgrad_kernel<1, 32, 16, 0><<<grid, 256, 0, s>>>(dc, batch, in, dout, nullptr, p.per_wave, slots);
+    if (cin == 64 && cout == 32) wgrad_tconv_kernel<64, 32><<<grid, 256, 0, s>>>(dc, batch, in, dout, p.per_wave, slots);
+    else if (cin == 32 && cout == 16) wgrad_tconv_kernel<32, 16><<<grid, 256, 0, s>>>(dc, batch, in, dout, p.per_wave, slots);
     else throw Failure{DS_ERROR_UNSUPPORTED, "transposed convolution shape not in the network"};
     const uint32_t per = 8u * cin * cout;
     wgrad_reduce_kernel<<<blocks_for(per, 64), 64 * kReduceWaves, 0, s>>>(slots, p.waves, 8, cin, cout, cout, dw);
