@@ -98,11 +98,10 @@ enum { DS_PROJECTION_PCG = 0, DS_PROJECTION_RBGS = 1 };
  * per second at 128^3). The stopping test runs every second iteration, so iteration counts are
  * even except at an odd iteration cap. */
 /* DS_CG_MULTIGRID: CG preconditioned by an aggregation multigrid V-cycle instead of Jacobi (2 x 2 x 2
- * aggregates, Galerkin coarse operators built at context creation, two damped Jacobi sweeps before
- * and after each coarse correction, the coarsest level of at most 512 cells solved exactly). Same
- * stopping test on the true residual; a few tens of iterations where the Jacobi forms need about a
- * thousand (128^3 plume). One iteration is captured as a HIP graph on the context's stream. No
- * counterpart in the reference, which iterates red-black Gauss-Seidel (DS_PROJECTION_RBGS). */
+ * aggregates, Galerkin coarse operators built at context creation, two Jacobi sweeps with Chebyshev weights
+ * before and after each coarse correction, the coarsest level of at most 64 cells solved exactly).
+ * Same stopping test on the true residual; about ten iterations where the Jacobi forms need about a
+ * thousand (128^3 plume). No counterpart in the reference, which iterates red-black Gauss-Seidel (DS_PROJECTION_RBGS). */
 enum { DS_CG_SINGLE_REDUCTION = 0, DS_CG_TWO_REDUCTION = 1, DS_CG_SINGLE_REDUCTION_RESIDENT = 2, DS_CG_S_STEP = 3, DS_CG_MULTIGRID = 4 };
 
 /* Initial guess of the forward and adjoint pressure solves. */
