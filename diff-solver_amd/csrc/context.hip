@@ -456,13 +456,18 @@ ds_status ds_context_create(const ds_config* config, uint32_t mode, void* stream
             // the fused kernel reads one producer partial per thread: blocks <= kPcgThreads
             const uint64_t cap = std::min<uint64_t>(kPcgMaxBlocks, kPcgThreads);
             const uint64_t target = cfg.cg_variant == DS_CG_S_STEP ? kPcgTargetBlocksS2 : kPcgTargetBlocks;
-            while (zc < 64 && tiles * (uint64_t)g.nz > target * zc) zc *= 2;
-            while (tiles * (((uint64_t)g.nz + zc - 1) / zc) > cap) zc *= 2;
+            // A plane of more than `cap` tiles has no such zc. The multigrid form does without the tiling;
+            // the others are refused, here or (red-black projection) when a PCG solve is asked for.
+            const bool tiled = tiles <= cap;
+            if (!tiled && cfg.cg_variant != DS_CG_MULTIGRID && cfg.projection_solver != DS_PROJECTION_RBGS)
+                throw Failure{DS_ERROR_UNSUPPORTED, "grid too large for the PCG tiling"};
+            if (tiled) {
+                while (zc < 64 && tiles * (uint64_t)g.nz > target * zc) zc *= 2;
+                while (tiles * (((uint64_t)g.nz + zc - 1) / zc) > cap) zc *= 2;
+            }
             t.zc = zc;
-            const uint64_t G = tiles * (((uint64_t)g.nz + zc - 1) / zc);
+            const uint64_t G = tiled ? tiles * (((uint64_t)g.nz + zc - 1) / zc) : 0;
             c->pcg.blocks = (uint32_t)((G + 7) & ~7ull);
-            // the fused kernel gives each thread at most one producer partial
-            if (c->pcg.blocks > kPcgThreads) throw Failure{DS_ERROR_UNSUPPORTED, "grid too large for the PCG tiling"};
         }
         c->pcg.partials = device_alloc<double>(c, 2 * (size_t)kPartCount * kPcgMaxBlocks);   // two sets
         c->pcg.hist = device_alloc<double>(c, 2 * ((size_t)c->max_iterations + 4));

@@ -921,6 +921,7 @@ void pcg_resident_prepare(ds_context* c) {
 ds_solve_info pcg_solve_kind(ds_context* c, int kind, const float* const u[3], const float* const extra[3], float* xh,
                              float* xl, const float* x0h, const float* x0l, double tol, uint32_t max_it, bool correct, bool replay) {
     if (c->config.projection_solver == DS_PROJECTION_RBGS && kind != kRhsGiven) return rbgs_solve_kind(c, kind, u, extra, xh, xl);
+    if (c->pcg.blocks == 0) throw Failure{DS_ERROR_UNSUPPORTED, "grid too large for the PCG tiling"};
     RhsIn in{};
     for (int a = 0; a < 3; ++a) {
         in.u[a] = u ? u[a] : nullptr;

@@ -99,3 +99,21 @@ def random_fields(sc, seed=0, vel_scale=0.6):
 
 def plume_state(sc):
     return scenes.initial_state(sc), scenes.control(sc)
+
+
+def pressure_residual(code, x, b, periodic=(False, False, False)):
+    """b - A x in FP64 over the unknowns (code > 0), x and b cell fields (nz, ny, nx): A has the
+    diagonal `code` and -1 between neighbouring unknowns; periodic: per axis x, y, z."""
+    x = np.where(code > 0, np.asarray(x, dtype=np.float64), 0.0)
+    ax = code.astype(np.float64) * x
+    for axis, wraps in ((2, periodic[0]), (1, periodic[1]), (0, periodic[2])):
+        n = x.shape[axis]
+        lo, hi = [slice(None)] * 3, [slice(None)] * 3
+        lo[axis], hi[axis] = slice(0, n - 1), slice(1, n)
+        ax[tuple(lo)] -= x[tuple(hi)]
+        ax[tuple(hi)] -= x[tuple(lo)]
+        if wraps:
+            lo[axis], hi[axis] = slice(0, 1), slice(n - 1, n)
+            ax[tuple(lo)] -= x[tuple(hi)]
+            ax[tuple(hi)] -= x[tuple(lo)]
+    return np.where(code > 0, np.asarray(b, dtype=np.float64) - ax, 0.0)
