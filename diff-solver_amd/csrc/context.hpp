@@ -212,6 +212,7 @@ constexpr uint32_t kMgBottomCells = 4096;   // levels of at most this many cells
 // together, 1140 on the second and 342 on the third.
 constexpr uint32_t kMgBottomLds = 6144;
 constexpr int kMgBottomLevels = 5;
+enum MgBox : uint8_t { kMgBoxSmall, kMgBoxMedium, kMgBoxLarge, kMgBoxThinX, kMgBoxThinZ };
 struct MgBottom {
     uint32_t count;
     uint32_t off[kMgBottomLevels];  // first element of each level's vectors
@@ -222,6 +223,8 @@ struct MgBottom {
 struct MgWork {
     int levels = 0;
     MgLevel lv[kMgMaxLevels]{};
+    MgBox box[kMgMaxLevels]{};      // the kernels' boxes
+    uint32_t per = 0;               // bit a: axis a of the levels is periodic
     // per level: right-hand side (levels > 0), pre-smoothed iterate, result (levels > 0)
     float* vec[kMgMaxLevels][3]{};
     double* dense = nullptr;        // inverse of the coarsest operator, n x n (symmetric)

@@ -103,6 +103,16 @@ using BoxM = Box<16, 8, 4, 256>;
 using BoxS = Box<16, 4, 4, 192>;
 using BoxC = Box<16, 8, 8, 256>;
 using BoxD = Box<8, 8, 4, 192>;
+// Large grids of a few cells along x or z, level 0 and coarser. In a box of 32 x 8 x 8 the kernels load
+// and sweep 12 planes for one plane of cells, and 36 columns for one along x. Steps with it, with these
+// boxes, and with kernels of one thread per cell: 1024 x 1024 x 1 2257, 1490, 2135 us; 2 x 1024 x 1024
+// 6735, 2198, 2928; 3 x 1024 x 1024 7254, 3118, 4066; 6 x 1024 x 1024 8039, 4386, 6855; 512 x 512 x 2
+// 977, 789, 1442. (Thin along x: 4 x 32 x 8 3124, 8 x 16 x 8 3352, 4 x 64 x 4 3068 us at 2 x 1024 x 1024.)
+// Along y the cubic box does: 1024 x 2 x 1024 2350 against 2638 us.
+using BoxLX = Box<2, 64, 8, 448>;
+using BoxLZ = Box<32, 16, 2, 768>;
+using BoxCX = Box<2, 32, 8, 256>;
+using BoxCZ = Box<16, 16, 2, 448>;
 
 // Column (x, y) of a level, wrapped along the periodic axes: its offset in a plane, and whether it
 // lies in the grid and is the thread's to handle (the offset is 0 when not).
@@ -1059,28 +1069,59 @@ std::vector<double> dense_inverse(const HostLevel& L, const bool per[3]) {
     return out;
 }
 
+// Points of a level with halos of 2 that boxes of type B load and sweep.
+template <typename B>
+uint64_t box_points(const MgLevel& L) {
+    return (uint64_t)B::grid(L).count * (uint64_t)(B::template P<2> * B::template Z<2>);
+}
+
+// The box type of level l: by the number of cells, but a thin one on a large grid where it has less
+// than two thirds of the points (from 16 cells along x or 3 along z on it does not).
+MgBox choose_box(const MgLevel& L, int l) {
+    auto thin = [&]<typename N, typename X, typename Z>() {
+        const uint64_t x = box_points<X>(L), z = box_points<Z>(L);
+        if (3 * std::min(x, z) >= 2 * box_points<N>(L)) return kMgBoxLarge;
+        return x < z ? kMgBoxThinX : kMgBoxThinZ;
+    };
+    if (l > 0) return L.n < kMgCoarseLarge ? kMgBoxSmall : thin.template operator()<BoxC, BoxCX, BoxCZ>();
+    if (L.n < kMgMediumCells) return kMgBoxSmall;
+    if (L.n < kMgLargeCells) return kMgBoxMedium;
+    return thin.template operator()<BoxL, BoxLX, BoxLZ>();
+}
+
 }  // namespace
 
 void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
     MgWork& w = c->mg;
     const Geo& g = c->geo;
-    const bool per[3]{c->pressure_periodic[0], c->pressure_periodic[1], c->pressure_periodic[2]};
     require(code.size() >= (size_t)g.n, "multigrid: code shorter than the grid");
+    // The levels' axes: the grid's, those of one cell last. The cells lie in memory the same way, so a
+    // grid of 1 x ny x nz is one of ny x nz x 1, which the boxes fit better (1 x 1024 x 1024: 1490 us a
+    // step against 2189 with boxes thin along x).
+    int ext[3]{g.nx, g.ny, g.nz};
+    bool per[3]{c->pressure_periodic[0], c->pressure_periodic[1], c->pressure_periodic[2]};
+    for (int pass = 0; pass < 2; ++pass)
+        for (int a = 0; a < 2; ++a)
+            if (ext[a] == 1) {
+                std::swap(ext[a], ext[a + 1]);
+                std::swap(per[a], per[a + 1]);
+            }
+    w.per = (per[0] ? 1u : 0u) | (per[1] ? 2u : 0u) | (per[2] ? 4u : 0u);
     // level 0 as diagonal + couplings: A_ii = code_i, -1 between neighbouring unknowns (on an
     // extent-1 periodic axis a cell neighbours itself twice, as in the matrix-vector product)
     std::vector<HostLevel> levels(1);
     {
         HostLevel& f = levels[0];
-        f.nx = g.nx;
-        f.ny = g.ny;
-        f.nz = g.nz;
+        f.nx = ext[0];
+        f.ny = ext[1];
+        f.nz = ext[2];
         const size_t n = f.cells();
         f.diag.resize(n);
         for (auto& v : f.wp) v.assign(n, 0.0);
-        for (int z = 0; z < g.nz; ++z)
-            for (int y = 0; y < g.ny; ++y)
-                for (int x = 0; x < g.nx; ++x) {
-                    const size_t i = (size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * (size_t)z);
+        for (int z = 0; z < f.nz; ++z)
+            for (int y = 0; y < f.ny; ++y)
+                for (int x = 0; x < f.nx; ++x) {
+                    const size_t i = (size_t)x + (size_t)f.nx * ((size_t)y + (size_t)f.ny * (size_t)z);
                     f.diag[i] = (double)code[i];
                     if (!code[i]) continue;
                     for (int a = 0; a < 3; ++a) {
@@ -1157,6 +1198,7 @@ void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
     }
     require(off <= kMgBottomLds, "multigrid: the coarse levels do not fit one workgroup");
     bt.dense = w.dense;
+    for (int l = 0; l < w.levels; ++l) w.box[l] = choose_box(w.lv[l], l);
 }
 
 namespace {
@@ -1164,20 +1206,26 @@ namespace {
 Pair2 residuals(const ds_context* c) { return Pair2{{c->pcg.r, c->pcg.r_alt}}; }
 Pair2 directions(const ds_context* c) { return Pair2{{c->pcg.p[0], c->pcg.p[1]}}; }
 
-// Runs f with the box type of the context's level 0: enough boxes to fill the chip, the larger box
-// where there are.
+// Runs f with the box type of the context's level 0, or of its coarser level l.
 template <typename F>
 void with_box(const ds_context* c, F&& f) {
-    const uint32_t n = c->geo.n;
-    if (n >= kMgLargeCells) f.template operator()<BoxL>();
-    else if (n >= kMgMediumCells) f.template operator()<BoxM>();
-    else f.template operator()<BoxS>();
+    switch (c->mg.box[0]) {
+        case kMgBoxSmall: return f.template operator()<BoxS>();
+        case kMgBoxMedium: return f.template operator()<BoxM>();
+        case kMgBoxThinX: return f.template operator()<BoxLX>();
+        case kMgBoxThinZ: return f.template operator()<BoxLZ>();
+        default: return f.template operator()<BoxL>();
+    }
 }
 
 template <typename F>
-void with_coarse_box(const MgLevel& L, F&& f) {
-    if (L.n >= kMgCoarseLarge) f.template operator()<BoxC>();
-    else f.template operator()<BoxD>();
+void with_coarse_box(const ds_context* c, int l, F&& f) {
+    switch (c->mg.box[l]) {
+        case kMgBoxSmall: return f.template operator()<BoxD>();
+        case kMgBoxThinX: return f.template operator()<BoxCX>();
+        case kMgBoxThinZ: return f.template operator()<BoxCZ>();
+        default: return f.template operator()<BoxC>();
+    }
 }
 
 void launch_bottom(const MgBottom& B, const float* r, float* out, const double* partials, uint32_t blocks, PcgStatus* st,
@@ -1201,7 +1249,7 @@ void launch_cycle(ds_context* c, uint32_t k, bool advance, float* xh, float* xl,
     PcgWork& pw = c->pcg;
     hipStream_t s = c->stream;
     PcgStatus* st = pw.status;
-    const uint32_t per = pcg_periodic_bits(c);
+    const uint32_t per = w.per;
     const Pair2 r = residuals(c), p = directions(c);
     const bool direct = w.levels == 1;
     const MgLevel &L0 = w.lv[0], &L1 = w.lv[direct ? 0 : 1];
@@ -1212,14 +1260,14 @@ void launch_cycle(ds_context* c, uint32_t k, bool advance, float* xh, float* xl,
     });
     const int bf = w.bottom_first;
     for (int l = 1; l < bf; ++l)
-        with_coarse_box(w.lv[l], [&]<typename B>() {
+        with_coarse_box(c, l, [&]<typename B>() {
             mg_down_kernel<B><<<(B::grid(w.lv[l]).count + 7u) & ~7u, B::T, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l][1], w.vec[l + 1][0],
                                                                                  st);
         });
     launch_bottom(w.bottom, direct ? nullptr : w.vec[bf][0], direct ? nullptr : w.vec[bf][2], pw.partials, pw.blocks, st, tol2,
                   mode, after, s);
     for (int l = bf - 1; l >= 1; --l)
-        with_coarse_box(w.lv[l], [&]<typename B>() {
+        with_coarse_box(c, l, [&]<typename B>() {
             mg_up_kernel<B><<<(B::grid(w.lv[l]).count + 7u) & ~7u, B::T, 0, s>>>(w.lv[l], w.lv[l + 1], per, w.vec[l][0], w.vec[l][1], w.vec[l + 1][2],
                                                                                w.vec[l][2], st);
         });
@@ -1264,7 +1312,7 @@ void mg_set_iteration(ds_context* c, uint32_t k) {
 void mg_iteration(ds_context* c, uint32_t k, float* xh, float* xl, double tol2) {
     PcgWork& pw = c->pcg;
     with_box(c, [&]<typename B>() {
-        mg_direction_kernel<B><<<pw.blocks, B::T, 0, c->stream>>>(c->mg.lv[0], pcg_periodic_bits(c), c->mg.z, directions(c), pw.partials, pw.hist,
+        mg_direction_kernel<B><<<pw.blocks, B::T, 0, c->stream>>>(c->mg.lv[0], c->mg.per, c->mg.z, directions(c), pw.partials, pw.hist,
                                                                  pw.status, k);
     });
     launch_cycle(c, k, true, xh, xl, tol2, 0u);
