@@ -180,13 +180,20 @@ __device__ __forceinline__ float divide_small(float sum, float d) {
     return __builtin_amdgcn_div_fixupf(__fmaf_rn(__fmaf_rn(-d, q, sum), rd, q), d, sum);
 }
 
+// The axes of the boxes in terms of the grid's: those of one cell last. The cells lie in memory the same
+// way, so a grid of 1 x ny x nz is swept as ny x nz x 1 (the sum's order follows; colours are the same).
+struct BoxAxes {
+    int of[3];
+};
+
+// g: the grid with its axes in the boxes' order.
 // Wide: the thread's two cells in one load; x is not periodic then and nx >= 2 (a pair that has one
 // cell outside reads the pair next to it).
 template <typename B, bool Wide>
 __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __restrict__ bp, const uint8_t* __restrict__ diag,
                                                         const float* __restrict__ rhs, const float* __restrict__ p_in,
                                                         float* __restrict__ p_out, uint32_t ntx, uint32_t nty, uint32_t boxes, int ex, int ey,
-                                                        int ez, int iterations) {
+                                                        int ez, int iterations, BoxAxes axes) {
     constexpr int H = B::H, K = B::K, RY = B::RY, RZ = B::RZ, P = B::P, Pad = K + 2;
     __shared__ float s[2][RZ * P + 2 * Pad];
     const uint32_t b = xcd_block();
@@ -196,8 +203,8 @@ __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __r
     const bool active = j < RY;
     const int x = bx * ex - H + 2 * k - odd, y = by * ey - H + j, z0 = bz * ez - H;
     float out[2]{}, out_y = 0.0f;
-    const int iy = sweep_coord(*bp, 1, y, g.ny, out_y);
-    const int ix[2]{sweep_coord(*bp, 0, x, g.nx, out[0]), sweep_coord(*bp, 0, x + 1, g.nx, out[1])};
+    const int iy = sweep_coord(*bp, axes.of[1], y, g.ny, out_y);
+    const int ix[2]{sweep_coord(*bp, axes.of[0], x, g.nx, out[0]), sweep_coord(*bp, axes.of[0], x + 1, g.nx, out[1])};
     bool in[2];
     uint32_t at[2], keep[2];   // keep: 0 where there is nothing to update, or a neighbour is not loaded
 #pragma unroll
@@ -213,8 +220,8 @@ __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __r
     float p[2][RZ], r[2][RZ];
     uint32_t d[2][(RZ + 3) / 4]{};
     float out_z[2]{};
-    const bool wraps = sweep_coord(*bp, 2, -1, g.nz, out_z[0]) >= 0;
-    (void)sweep_coord(*bp, 2, g.nz, g.nz, out_z[1]);
+    const bool wraps = sweep_coord(*bp, axes.of[2], -1, g.nz, out_z[0]) >= 0;
+    (void)sweep_coord(*bp, axes.of[2], g.nz, g.nz, out_z[1]);
     int wz = wraps ? wrapi(z0, g.nz) : 0;
 #pragma unroll
     for (int z = 0; z < RZ; ++z) {
@@ -330,10 +337,17 @@ uint64_t box_count(const Geo& g) {
     return count(g.nx, B::X) * count(g.ny, B::Y) * count(g.nz, B::Z);
 }
 
-// One launch of rbgs_box_kernel; boxes of equal even extents that cover the grid.
+// Cells that the boxes of type B load, their halos among them.
 template <typename B>
-void launch_boxes(ds_context* c, const SBound* bp, const float* b, const float* p_in, float* p_out, uint32_t iterations) {
-    const Geo& g = c->geo;
+uint64_t box_points(const Geo& g) {
+    return box_count<B>(g) * (uint64_t)(2 * B::P * B::RZ);
+}
+
+// One launch of rbgs_box_kernel; boxes of equal even extents that cover the grid (g, its axes in the
+// boxes' order).
+template <typename B>
+void launch_boxes(ds_context* c, const Geo& g, const BoxAxes& axes, const SBound* bp, const float* b, const float* p_in, float* p_out,
+                  uint32_t iterations) {
     auto split = [](int n, int most, uint32_t& count) {
         count = ((uint32_t)n + (uint32_t)most - 1) / (uint32_t)most;
         return (int)((((uint32_t)n + count - 1) / count + 1u) & ~1u);
@@ -342,9 +356,9 @@ void launch_boxes(ds_context* c, const SBound* bp, const float* b, const float* 
     const int ex = split(g.nx, B::X, cx), ey = split(g.ny, B::Y, cy), ez = split(g.nz, B::Z, cz);
     const uint32_t boxes = cx * cy * cz, blocks = (boxes + 7u) & ~7u;
     auto launch = [&](auto kernel) {
-        kernel<<<blocks, B::T, 0, c->stream>>>(g, bp, c->rbgs_diag, b, p_in, p_out, cx, cy, boxes, ex, ey, ez, (int)iterations);
+        kernel<<<blocks, B::T, 0, c->stream>>>(g, bp, c->rbgs_diag, b, p_in, p_out, cx, cy, boxes, ex, ey, ez, (int)iterations, axes);
     };
-    if (!c->pressure_periodic[0] && g.nx >= 2) launch(rbgs_box_kernel<B, true>);
+    if (!c->pressure_periodic[axes.of[0]] && g.nx >= 2) launch(rbgs_box_kernel<B, true>);
     else launch(rbgs_box_kernel<B, false>);
 }
 
@@ -384,12 +398,21 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
         // boxes wherever the colouring holds: the launches of one colour remain for a periodic axis of
         // odd extent, where a sweep reads a neighbour that it writes itself
         if (coloured && iterations > 0) {
+            Geo gb = g;   // (cells and extents only are used)
+            BoxAxes axes{{0, 1, 2}};
+            int* const extents[3]{&gb.nx, &gb.ny, &gb.nz};
+            for (int pass = 0; pass < 2; ++pass)
+                for (int a = 0; a < 2; ++a)
+                    if (*extents[a] == 1) {
+                        std::swap(*extents[a], *extents[a + 1]);
+                        std::swap(axes.of[a], axes.of[a + 1]);
+                    }
             auto sweeps = [&]<typename B>() {
                 const uint32_t launches = (iterations + B::S - 1) / B::S;
                 float* from = launches % 2 ? xl : xh;   // both are zero; the last launch writes xh
                 for (uint32_t l = 0, done = 0; l < launches; ++l, done += B::S) {
                     float* to = from == xh ? xl : xh;
-                    launch_boxes<B>(c, bp, b, from, to, std::min<uint32_t>(B::S, iterations - done));
+                    launch_boxes<B>(c, gb, axes, bp, b, from, to, std::min<uint32_t>(B::S, iterations - done));
                     from = to;
                 }
             };
@@ -397,9 +420,22 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
             // are at most one for each of the 256 CUs: 64^3 (256 flat boxes, 64 deep ones), two steps of
             // 160 iterations, 1352 against 1929 us, 24^3 1245 against 1750; beyond that the halo
             // decides: 96 x 100 x 75 (798 flat boxes, 210 deep ones) 2788 against 2152 us.
+            // On a grid of a few cells along z or x Deep sweeps mostly cells outside it; a thin box is taken
+            // where it has less than two thirds of Deep's points (up to 2 cells along z, 8 along x). Steps of
+            // 80 iterations with Deep, with the thin box, and with a launch per colour: 1024 x 1024 x 1 1529,
+            // 1098, 2002 us; 512 x 512 x 2 604, 452, 1112; 2 x 1024 x 1024 6647, 2449, 2943 (4 x 64 x 8: 3481);
+            // 4 x 1024 x 1024 7056, 2484, 5168 (8 x 32 x 8: 4359); 6 x 1024 x 1024 7415, 4405, 7923. With axes of
+            // one cell last: 1 x 1024 x 1024 6051 -> 1101, 1024 x 1 x 1024 2876 -> 1094. Along y Deep does:
+            // 1024 x 2 x 1024 3046 against 3193.
             using Flat = SweepBox<2, 32, 16, 2>;
             using Deep = SweepBox<2, 32, 16, 8>;
-            if (box_count<Flat>(g) <= 256u) sweeps.template operator()<Flat>();
+            using Thin2 = SweepBox<2, 2, 64, 8>;
+            using Thin4 = SweepBox<2, 4, 64, 8>;
+            const uint64_t deep = box_points<Deep>(gb);
+            auto thin = [&]<typename B>() { return 3 * box_points<B>(gb) < 2 * deep; };
+            if (box_count<Flat>(gb) <= 256u || thin.template operator()<Flat>()) sweeps.template operator()<Flat>();
+            else if (gb.nx <= 2) sweeps.template operator()<Thin2>();
+            else if (thin.template operator()<Thin4>()) sweeps.template operator()<Thin4>();
             else sweeps.template operator()<Deep>();
             fill_zero(c, xl, g.n);
         } else for (uint32_t it = 0; it < iterations; ++it) {
