@@ -48,6 +48,54 @@ void fill_zero_d(ds_context* c, double* p, uint64_t count) {
 }
 
 namespace {
+// The contexts that exist, for release_idle_buffers (never destroyed: a context may outlive the
+// library's static objects).
+struct Contexts {
+    std::mutex lock;
+    std::vector<ds_context*> all;
+};
+Contexts& contexts() {
+    static Contexts* const c = new Contexts;
+    return *c;
+}
+}  // namespace
+
+void release_idle_buffers(ds_context* only) noexcept {
+    Contexts& known = contexts();
+    const std::lock_guard<std::mutex> hold(known.lock);
+    int device = 0;
+    const bool restore = hipGetDevice(&device) == hipSuccess;
+    for (ds_context* c : known.all) {
+        if (only && c != only) continue;
+        const std::vector<Buffers::Block> blocks = c->buffers.remove();
+        if (blocks.empty()) continue;
+        (void)hipSetDevice(c->device);
+        // not on the context's stream, which may be recording a graph: the buffers have no work pending
+        hipStream_t s = nullptr;
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess) {
+            for (const Buffers::Block& b : blocks) (void)hipFreeAsync(b.p, s);
+            (void)hipStreamSynchronize(s);
+            (void)hipStreamDestroy(s);
+        } else {
+            for (const Buffers::Block& b : blocks) (void)hipFree(b.p);
+        }
+        hipMemPool_t pool = nullptr;
+        if (hipDeviceGetDefaultMemPool(&pool, c->device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+    }
+    if (restore) (void)hipSetDevice(device);
+    (void)hipGetLastError();
+}
+
+void* device_malloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    release_idle_buffers(nullptr);
+    DS_HIP(hipMalloc(&p, bytes));
+    return p;
+}
+
+namespace {
 
 // model.cpp:17-28, evaluated in FP32 like the reference.
 bool contains(const ds_collider& col, float px, float py, float pz) {
@@ -522,6 +570,8 @@ ds_status ds_context_create(const ds_config* config, uint32_t mode, void* stream
             }
         }
         DS_HIP(hipStreamSynchronize(c->stream));   // model.cpp:181
+        const std::lock_guard<std::mutex> hold(contexts().lock);
+        contexts().all.push_back(c);
     });
     if (st != DS_OK) {
         ds_context_destroy(c);
@@ -533,6 +583,10 @@ ds_status ds_context_create(const ds_config* config, uint32_t mode, void* stream
 
 ds_status ds_context_destroy(ds_context* c) {
     if (!c) return DS_OK;
+    {
+        const std::lock_guard<std::mutex> hold(contexts().lock);
+        std::erase(contexts().all, c);
+    }
     ds_status st = DS_OK;
     if (c->stream && hipStreamSynchronize(c->stream) != hipSuccess) {
         set_error("ds_context_destroy: stream synchronisation failed");
@@ -600,8 +654,18 @@ ds_status ds_allocate(ds_context* c, size_t bytes, void** out) {
     }
     return guard([&] {
         *out = nullptr;
-        DS_HIP(hipMallocAsync(out, bytes ? bytes : 1, c->stream));   // cuda.cpp:39-43 (stream-ordered pool)
+        const size_t size = bytes ? bytes : 1;
+        if (hipMallocAsync(out, size, c->stream) == hipSuccess) return;   // cuda.cpp:39-43 (stream-ordered pool)
+        (void)hipGetLastError();
+        *out = nullptr;
+        release_idle_buffers(nullptr);
+        DS_HIP(hipMallocAsync(out, size, c->stream));
     });
+}
+
+ds_status ds_context_release_buffers(ds_context* c) {
+    release_idle_buffers(c);
+    return DS_OK;
 }
 
 ds_status ds_release(ds_context* c, void* p) {

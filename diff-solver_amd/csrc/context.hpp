@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdint>
 #include <exception>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -241,23 +242,37 @@ namespace ds {
 // the context between calls. Freed through the stream-ordered allocator they went back to the
 // operating system at every call's last synchronisation and were mapped again in the next call:
 // 39 + 4 ms of a 154 ms gradient (128^3, 32 steps). One stream per context, so a buffer that is
-// given back is taken again in stream order. Kept: what the last call used, at most 1/16 of the
-// card's memory, and only while a quarter of the card is free; all of it is freed when an
-// allocation fails and with the context.
+// given back is taken again in stream order; between calls the stream is drained, so an idle buffer
+// has no work pending.
+// Kept: what the last call used, at most 1/16 of the card's memory over the contexts of the process,
+// and nothing when a call ends with less than a quarter of the card free. Given back: with the
+// context, by ds_context_release_buffers, and when an allocation of the library fails
+// (release_idle_buffers).
 struct Buffers {
     struct Block {
         void* p;
         size_t bytes;
         uint64_t call;   // trajectory call that used it last
     };
+    std::mutex lock;           // of idle and busy: another thread may release the buffers between calls
     std::vector<Block> idle;
-    size_t idle_bytes = 0, limit = 0;
+    bool busy = false;         // a trajectory call runs: the idle buffers are its own
+    size_t limit = 0;
     uint64_t call = 0;
     void* take(size_t bytes, hipStream_t s);
     void give(void* p, size_t bytes, hipStream_t s) noexcept;
     // frees the idle buffers that the call before did not use (all: every one)
     void trim(bool all, hipStream_t s) noexcept;
+    // takes the idle buffers out, none during a trajectory call
+    std::vector<Block> remove() noexcept;
 };
+
+// Frees the idle trajectory buffers of context c, or of every context of the process (null), and
+// returns the memory to the device. Contexts inside a trajectory call keep theirs.
+void release_idle_buffers(ds_context* c) noexcept;
+
+// hipMalloc, tried again once the idle trajectory buffers are given back.
+void* device_malloc(size_t bytes);
 
 }  // namespace ds
 
@@ -361,8 +376,7 @@ namespace ds {
 
 template <typename T>
 T* device_alloc(ds_context* c, size_t count) {
-    void* p = nullptr;
-    DS_HIP(hipMalloc(&p, count * sizeof(T) > 0 ? count * sizeof(T) : 1));
+    void* p = device_malloc(count * sizeof(T) > 0 ? count * sizeof(T) : 1);
     c->allocations.push_back(p);
     return static_cast<T*>(p);
 }

@@ -3,8 +3,10 @@
 // xayah/solver.hpp through a thin adapter over the C-ABI views.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cmath>
 #include <functional>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -242,19 +244,27 @@ ds_solve_info vjp_step(ds_context* c, const ds_parameters* p, const ds_state* st
     return si;
 }
 
+namespace {
+std::atomic<size_t> g_idle_bytes{0};   // idle buffers of all contexts
+}
+
 void* Buffers::take(size_t bytes, hipStream_t s) {
-    for (size_t i = idle.size(); i-- > 0;)   // the one given back last: its lines may still be cached
-        if (idle[i].bytes == bytes) {
-            void* p = idle[i].p;
-            idle.erase(idle.begin() + (std::ptrdiff_t)i);
-            idle_bytes -= bytes;
-            return p;
-        }
+    {
+        const std::lock_guard<std::mutex> hold(lock);
+        for (size_t i = idle.size(); i-- > 0;)   // the one given back last: its lines may still be cached
+            if (idle[i].bytes == bytes) {
+                void* p = idle[i].p;
+                idle.erase(idle.begin() + (std::ptrdiff_t)i);
+                g_idle_bytes -= bytes;
+                return p;
+            }
+    }
     void* p = nullptr;
     if (hipMallocAsync(&p, bytes, s) == hipSuccess) return p;
     (void)hipGetLastError();
     trim(true, s);
     DS_HIP(hipStreamSynchronize(s));
+    release_idle_buffers(nullptr);
     DS_HIP(hipMallocAsync(&p, bytes, s));
     return p;
 }
@@ -264,28 +274,39 @@ void Buffers::give(void* p, size_t bytes, hipStream_t s) noexcept {
         size_t free_bytes = 0, total = 0;
         if (hipMemGetInfo(&free_bytes, &total) == hipSuccess) limit = total / 16;
     }
-    if (idle_bytes + bytes <= limit) {
+    if (g_idle_bytes.fetch_add(bytes) + bytes <= limit) {
         try {
+            const std::lock_guard<std::mutex> hold(lock);
             idle.push_back({p, bytes, call});
-            idle_bytes += bytes;
             return;
         } catch (...) {
         }
     }
+    g_idle_bytes -= bytes;
     (void)hipFreeAsync(p, s);
 }
 
 void Buffers::trim(bool all, hipStream_t s) noexcept {
+    const std::lock_guard<std::mutex> hold(lock);
     size_t kept = 0;
     for (const Block& b : idle) {
         if (!all && b.call == call) {
             idle[kept++] = b;
         } else {
             (void)hipFreeAsync(b.p, s);
-            idle_bytes -= b.bytes;
+            g_idle_bytes -= b.bytes;
         }
     }
     idle.resize(kept, Block{});
+}
+
+std::vector<Buffers::Block> Buffers::remove() noexcept {
+    std::vector<Block> out;
+    const std::lock_guard<std::mutex> hold(lock);
+    if (busy) return out;
+    out.swap(idle);
+    for (const Block& b : out) g_idle_bytes -= b.bytes;
+    return out;
 }
 
 namespace {
@@ -294,11 +315,18 @@ namespace {
 // less than a quarter of the card's memory is left.
 struct Trajectory {
     ds_context* c;
-    explicit Trajectory(ds_context* ctx) : c(ctx) { ++c->buffers.call; }
+    explicit Trajectory(ds_context* ctx) : c(ctx) {
+        const std::lock_guard<std::mutex> hold(c->buffers.lock);
+        c->buffers.busy = true;
+        ++c->buffers.call;
+    }
     ~Trajectory() {
+        (void)hipStreamSynchronize(c->stream);   // (drained, but for a call that failed)
         size_t free_bytes = 0, total = 0;
         const bool short_of = hipMemGetInfo(&free_bytes, &total) != hipSuccess || free_bytes < total / 4;
         c->buffers.trim(short_of, c->stream);
+        const std::lock_guard<std::mutex> hold(c->buffers.lock);
+        c->buffers.busy = false;
     }
     Trajectory(const Trajectory&) = delete;
     Trajectory& operator=(const Trajectory&) = delete;

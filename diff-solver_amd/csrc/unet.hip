@@ -260,8 +260,7 @@ namespace {
 
 template <typename T>
 T* unet_alloc(UNet* u, size_t count, bool activation = false) {
-    void* p = nullptr;
-    DS_HIP(hipMalloc(&p, count * sizeof(T) > 0 ? count * sizeof(T) : 1));
+    void* p = device_malloc(count * sizeof(T) > 0 ? count * sizeof(T) : 1);
     (activation ? u->activations : u->allocations).push_back(p);
     return static_cast<T*>(p);
 }

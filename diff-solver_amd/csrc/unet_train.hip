@@ -490,8 +490,7 @@ struct ds_unet_trainer {
     }
     template <typename T>
     T* alloc(size_t count_) {
-        void* p = nullptr;
-        DS_HIP(hipMalloc(&p, std::max<size_t>(count_ * sizeof(T), 1)));
+        void* p = ds::device_malloc(std::max<size_t>(count_ * sizeof(T), 1));
         allocations.push_back(p);
         return static_cast<T*>(p);
     }
@@ -598,8 +597,7 @@ struct Scratch {
     explicit Scratch(hipStream_t st) : s(st) {}
     template <typename T>
     T* get(size_t n) {
-        void* p = nullptr;
-        DS_HIP(hipMalloc(&p, std::max<size_t>(n * sizeof(T), 1)));
+        void* p = device_malloc(std::max<size_t>(n * sizeof(T), 1));
         ptrs.push_back(p);
         return static_cast<T*>(p);
     }

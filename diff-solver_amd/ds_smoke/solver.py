@@ -46,6 +46,7 @@ def load_library(path: str | None = None):
         "ds_context_create": (C.c_int32, [C.POINTER(abi.Config), C.c_uint32, P, C.POINTER(P)]),
         "ds_context_destroy": (C.c_int32, [P]),
         "ds_context_stream": (P, [P]),
+        "ds_context_release_buffers": (C.c_int32, [P]),
         "ds_context_domain_info": (C.c_int32, [P, C.POINTER(abi.DomainInfo)]),
         "ds_context_domain_masks": (C.c_int32, [P, P, P]),
         "ds_allocate": (C.c_int32, [P, C.c_size_t, C.POINTER(P)]),
@@ -154,6 +155,11 @@ def exported_symbols() -> list[str]:
     return sorted(n for n in dir(_LIB) if n.startswith("ds_"))
 
 
+def release_buffers():
+    """Give back the device buffers that every context keeps between trajectory calls (ds_context_release_buffers)."""
+    load_library().ds_context_release_buffers(None)
+
+
 def _ptr(t):
     return None if t is None else C.c_void_p(t.data_ptr())
 
@@ -202,10 +208,22 @@ class Context:
         except Exception:
             pass
 
+    def release_buffers(self):
+        """Give back the device buffers that this context keeps between trajectory calls."""
+        self._check(self.lib.ds_context_release_buffers(self.h), "ds_context_release_buffers")
+
     # ---- buffers
-    def _zeros(self, shape, dtype=None):
+    def _allocate(self, make):
+        """make() on this context's stream; when torch is out of memory, once more without the contexts' idle buffers."""
         with self.torch.cuda.stream(self.stream):
-            return self.torch.zeros(shape, dtype=dtype or self.torch.float32, device=self.device)
+            try:
+                return make()
+            except self.torch.cuda.OutOfMemoryError:
+                release_buffers()
+                return make()
+
+    def _zeros(self, shape, dtype=None):
+        return self._allocate(lambda: self.torch.zeros(shape, dtype=dtype or self.torch.float32, device=self.device))
 
     def zeros_cell(self):
         return self._zeros(cell_shape(self.n))
@@ -214,8 +232,8 @@ class Context:
         return tuple(self._zeros(face_shape(self.n, a)) for a in range(3))
 
     def to_device(self, a):
-        with self.torch.cuda.stream(self.stream):
-            return self.torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(self.device, non_blocking=False)
+        host = self.torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32))
+        return self._allocate(lambda: host.to(self.device, non_blocking=False))
 
     def synchronize(self):
         self.stream.synchronize()

@@ -265,6 +265,14 @@ uint64_t ds_config_face_count(const ds_config* config, uint32_t axis);
  * NULL (the context creates its own non-blocking stream) or a hipStream_t to run on. */
 ds_status ds_context_create(const ds_config* config, uint32_t mode, void* stream, ds_context** out);
 ds_status ds_context_destroy(ds_context* context);
+/* The trajectory calls (ds_simulate, ds_loss_gradient, ds_trajectory_*) keep their device buffers
+ * (checkpoints, step caches, tapes) in the context for the next call: what the last call used, at
+ * most 1/16 of the card's memory over the contexts of the process, and nothing when a call ends with
+ * less than a quarter of the card free. They are given back with the context, before an allocation of
+ * this library fails, and by this function: those of the context, or (NULL) of every context of the
+ * process. For programs that allocate by other means. Any thread may call it; a context inside a
+ * trajectory call keeps its buffers. No counterpart in the reference, which frees them in every call. */
+ds_status ds_context_release_buffers(ds_context* context);
 void* ds_context_stream(ds_context* context);
 ds_status ds_context_domain_info(ds_context* context, ds_domain_info* info);
 /* Copies the u8 solid mask and the u8 connectivity code (diagonal count, 0 = not an unknown)
