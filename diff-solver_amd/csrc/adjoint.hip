@@ -295,12 +295,10 @@ __global__ __launch_bounds__(256) void projection_vjp_face_kernel(Geo g, const V
         const int coord = A == 0 ? x : A == 1 ? y : z;
         const int n_a = dim_size(g, A);
         const bool per = vperiodic(b, A);
-        if (constrained_boundary<A>(g, b, coord) || (has_solids && adjacent_solid<A>(g, mask, x, y, z)) || (per && coord == n_a)) {
-            out.p[A][local] = 0.0f;
-            return;
-        }
-        float a = projected_face_adjoint<A>(g, in, x, y, z, local);
-        if (per && coord == 0) {
+        float a = 0.0f;
+        if (!(constrained_boundary<A>(g, b, coord) || (has_solids && adjacent_solid<A>(g, mask, x, y, z)) || (per && coord == n_a)))
+            a = projected_face_adjoint<A>(g, in, x, y, z, local);
+        if (per && coord == 0) {   // (also where a solid beyond this face, but not beyond its duplicate, constrains it)
             const int dx = A == 0 ? n_a : x, dy = A == 1 ? n_a : y, dz = A == 2 ? n_a : z;
             if (!(has_solids && adjacent_solid<A>(g, mask, dx, dy, dz)))
                 a += projected_face_adjoint<A>(g, in, dx, dy, dz, fidx(g, A, dx, dy, dz));
@@ -321,9 +319,9 @@ __global__ __launch_bounds__(256) void constrain_vjp_kernel(Geo g, const VBound*
         const int coord = A == 0 ? x : A == 1 ? y : z;
         const int n_a = dim_size(g, A);
         const bool per = vperiodic(b, A);
-        if (constrained_boundary<A>(g, b, coord) || (has_solids && adjacent_solid<A>(g, mask, x, y, z)) || (per && coord == n_a))
-            return;
-        float a = in.p[A][local];
+        float a = 0.0f;
+        if (!(constrained_boundary<A>(g, b, coord) || (has_solids && adjacent_solid<A>(g, mask, x, y, z)) || (per && coord == n_a)))
+            a = in.p[A][local];
         if (per && coord == 0) {
             const int dx = A == 0 ? n_a : x, dy = A == 1 ? n_a : y, dz = A == 2 ? n_a : z;
             if (!(has_solids && adjacent_solid<A>(g, mask, dx, dy, dz))) a += in.p[A][fidx(g, A, dx, dy, dz)];
