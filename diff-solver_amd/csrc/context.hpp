@@ -199,10 +199,9 @@ struct PcgWork {
 struct MgLevel {
     int nx, ny, nz;
     uint32_t n;
-    FastDiv dx, dy;                 // cell decode: divide by nx, ny
     const uint8_t* code;            // level 0
-    const float* diag;              // coarser levels
-    const float* idiag;             // 1 / diag on the unknowns, 0 elsewhere (coarser levels)
+    const float* diag;              // coarser levels above the bottom ones
+    const float* idiag;             // 1 / diag on the unknowns, 0 elsewhere (likewise)
     const float* wp[3];
 };
 constexpr int kMgMaxLevels = 32;
@@ -226,7 +225,8 @@ struct MgWork {
     MgLevel lv[kMgMaxLevels]{};
     MgBox box[kMgMaxLevels]{};      // the kernels' boxes
     uint32_t per = 0;               // bit a: axis a of the levels is periodic
-    // per level: right-hand side (levels > 0), pre-smoothed iterate, result (levels > 0)
+    // per level up to bottom_first: right-hand side (levels > 0), pre-smoothed iterate (not of the last),
+    // result (levels > 0)
     float* vec[kMgMaxLevels][3]{};
     double* dense = nullptr;        // inverse of the coarsest operator, n x n (symmetric)
     float* z = nullptr;             // the preconditioned residual

@@ -54,8 +54,13 @@ namespace {
 constexpr float kCheb[2]{0.564013325f, 1.477121796f};
 constexpr float kOver = 1.9f;   // scale of the prolonged coarse correction
 constexpr uint32_t kMgDotThreads = 512;
-constexpr uint32_t kMgLargeCells = 1u << 19, kMgMediumCells = 1u << 16;   // box of level 0 by its cells
-constexpr uint32_t kMgCoarseLarge = 1u << 17;                             // box of a coarser level
+// Boxes of level 0 and of a coarser level by its cells. The lines lie where the two sides are within 5 % of
+// each other (steps, us): large 545 and medium 502 at 64^3, 708 and 702 at 80 x 80 x 81, 720 and 740 at
+// 81 x 81 x 82, 735 and 757 at 90 x 70 x 110, 963 and 910 at 100^3, 1005 and 995 at 102^3; medium 420 and small 424
+// at 40^3, 426 and 432 at 41 x 40 x 40, 433 and 437 at 48^3; a coarser level's large and small at 65600 cells 731 and
+// 702, at 131072 844 and 818, at 175616 1105 and 1076.
+constexpr uint32_t kMgLargeCells = 1u << 19, kMgMediumCells = 1u << 16;
+constexpr uint32_t kMgCoarseLarge = 1u << 17;
 
 // 1 / d for a level-0 diagonal count (the hardware reciprocal: every use of a cell's value is the
 // same, so the smoother stays symmetric). Counts of 0 (not an unknown) give 1; the values they scale
@@ -1138,6 +1143,9 @@ void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
         levels.push_back(std::move(next));
     }
     w.levels = (int)levels.size();
+    // the levels one workgroup handles, from bottom_first on: they are laid out below
+    w.bottom_first = direct ? 1 : w.levels - 1;
+    while (!direct && w.bottom_first > 1 && levels[w.bottom_first - 1].cells() <= kMgBottomCells) --w.bottom_first;
     for (int l = 0; l < w.levels; ++l) {
         const HostLevel& H = levels[l];
         MgLevel& L = w.lv[l];
@@ -1145,13 +1153,11 @@ void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
         L.ny = H.ny;
         L.nz = H.nz;
         L.n = (uint32_t)H.cells();
-        L.dx = make_fastdiv((uint32_t)H.nx);
-        L.dy = make_fastdiv((uint32_t)H.ny);
         L.code = l == 0 ? c->code : nullptr;
         L.diag = nullptr;
         L.idiag = nullptr;
         for (int a = 0; a < 3; ++a) L.wp[a] = nullptr;
-        if (l > 0) {
+        if (l > 0 && l < w.bottom_first) {
             std::vector<float> buf(L.n);
             auto put = [&](const std::vector<double>& v) {
                 for (uint32_t i = 0; i < L.n; ++i) buf[i] = (float)v[i];
@@ -1164,21 +1170,22 @@ void mg_prepare(ds_context* c, const std::vector<uint8_t>& code) {
             for (uint32_t i = 0; i < L.n; ++i) inv[i] = H.diag[i] > 0.0 ? 1.0 / H.diag[i] : 0.0;
             L.idiag = put(inv);
             for (int a = 0; a < 3; ++a) L.wp[a] = put(H.wp[a]);
-            // right-hand side, pre-smoothed iterate, result
-            for (int k = 0; k < 3; ++k) w.vec[l][k] = device_alloc<float>(c, L.n);
-        } else if (!direct) {
-            w.vec[l][1] = device_alloc<float>(c, L.n);   // pre-smoothed iterate
         }
-        for (int k = 0; k < 3; ++k) fill_zero(c, w.vec[l][k], L.n);
+        if (!direct && l <= w.bottom_first) {
+            // right-hand side, pre-smoothed iterate, result
+            const bool used[3]{l > 0, l < w.bottom_first, l > 0};
+            for (int k = 0; k < 3; ++k)
+                if (used[k]) {
+                    w.vec[l][k] = device_alloc<float>(c, L.n);
+                    fill_zero(c, w.vec[l][k], L.n);
+                }
+        }
     }
     const std::vector<double> inv = dense_inverse(levels.back(), per);
     w.dense = device_alloc<double>(c, inv.size());
     DS_HIP(hipMemcpy(w.dense, inv.data(), inv.size() * sizeof(double), hipMemcpyHostToDevice));
     w.z = device_alloc<float>(c, g.n);
     fill_zero(c, w.z, g.n);
-    // the levels one workgroup handles
-    w.bottom_first = direct ? 1 : w.levels - 1;
-    while (!direct && w.bottom_first > 1 && w.lv[w.bottom_first - 1].n <= kMgBottomCells) --w.bottom_first;
     MgBottom& bt = w.bottom;
     uint32_t off = 0;
     for (int l = w.bottom_first; l < w.levels; ++l) {

@@ -535,9 +535,8 @@ __global__ __launch_bounds__(256) void wgrad_tconv_kernel(Dims d, int batch, con
 // m * NC + n] (NC = N channels rounded up to 16). A wave takes ROWS (3 or 1) rows of three taps along
 // x: they share the M fragments, and a row's three N fragments come from six voxels instead of
 // twelve. (A tap a wave was bound by its 2-byte loads and their addresses, eight for one matrix
-// instruction. 64^3 batch of 4, 16 -> 16 channels:
-// 314 us,
-// now 102; 16 + 16 -> 16: 379, now 125; 2 -> 16: 293, now 131; 32 -> 32 on the 32^3 level: 58, now 40.)
+// instruction. 64^3 batch of 4, 16 -> 16 channels: 314 us, now 102; 16 + 16 -> 16: 379, now 125; 2 -> 16:
+// 293, now 131; 32 -> 32 on the 32^3 level: 58, now 40.)
 // ROWS 3 while the accumulators fit beside four waves a SIMD (MC * NC <= 512: 72 registers), else 1.
 template <int ROWS, int MC, int C1, int C2>
 __global__ __launch_bounds__(256) void wgrad_rows_kernel(Dims d, int batch, const uint16_t* __restrict__ mt, const uint16_t* __restrict__ in1,

@@ -63,8 +63,8 @@ def scene_periodic(res=(12, 10, 8)):
 
 
 def scene_periodic_xy(res=(16, 12, 8)):
-    """Periodic in x and y with a power-of-two cell size (the velocity reverse gathers its fixed
-    start stencils there, and the periodic seams take the scatter path), fixed z faces."""
+    """Periodic in x and y with a power-of-two cell size (seams of the start and trace stencils on two
+    axes), fixed z faces."""
     h = 1.0 / 16.0
     sc = scenes.Scene(resolution=res, cell_size=h, time_step=0.5 * h, name="periodic_xy")
     sc.velocity_modes = (3, 3, 3, 3, 0, 2)
