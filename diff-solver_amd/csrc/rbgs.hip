@@ -296,10 +296,12 @@ __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __r
 // One launch of the reverse over the cells of colour `parity`: with Finish, the deferred second
 // half of the previous reverse sweep (that colour's rhs_bar += p_bar / diag, p_bar = 0); with
 // Gather, the first half of the next one (p_bar += sum over connected neighbours of p_bar / diag).
+// links: how often a cell is its own neighbour, twice per periodic axis of one cell. A sweep reads the
+// cell's old value that often, so its reverse leaves that share in p_bar instead of 0.
 template <bool Finish, bool Gather>
 __global__ __launch_bounds__(256) void rbgs_reverse_kernel(Geo g, const SBound* __restrict__ bp, const uint8_t* __restrict__ mask,
                                                            const uint8_t* __restrict__ diag, float* pbar, float* __restrict__ rbar,
-                                                           uint32_t parity) {
+                                                           uint32_t parity, uint32_t links) {
     int x, y, z;
     if (!colour_cell(g, blockIdx.x * blockDim.x + threadIdx.x, parity, x, y, z)) return;
     const uint32_t i = cidx(g, x, y, z);
@@ -307,8 +309,9 @@ __global__ __launch_bounds__(256) void rbgs_reverse_kernel(Geo g, const SBound* 
     if (Finish) {
         const uint32_t d = diag[i];
         if (d != 0u) {
-            rbar[i] += own / (float)d;
-            own = 0.0f;
+            own /= (float)d;
+            rbar[i] += own;
+            own = links ? own * (float)links : 0.0f;
         }
     }
     if (Gather && mask[i] == 0) {
@@ -321,7 +324,7 @@ __global__ __launch_bounds__(256) void rbgs_reverse_kernel(Geo g, const SBound* 
                 bool connected, fixed;
                 float fv;
                 rbgs_neighbour(g, *bp, mask, x, y, z, dim, dir, j, connected, fixed, fv);
-                if (connected) {
+                if (connected && j != i) {
                     const uint32_t dj = diag[j];
                     if (dj != 0u) s += pbar[j] / (float)dj;
                 }
@@ -445,10 +448,13 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
         check_launch("rbgs_sweep_kernel");
     } else if (iterations > 0) {
         // b holds p_bar; xh accumulates rhs_bar. Reverse order of the sweeps: colour 1, then 0, ...
-        rbgs_reverse_kernel<false, true><<<CB, kBlock, 0, c->stream>>>(g, c->d_pb, c->mask, c->rbgs_diag, b, xh, 0u);
+        const int extents[3]{g.nx, g.ny, g.nz};
+        uint32_t links = 0;
+        for (int a = 0; a < 3; ++a) links += c->pressure_periodic[a] && extents[a] == 1 ? 2u : 0u;
+        rbgs_reverse_kernel<false, true><<<CB, kBlock, 0, c->stream>>>(g, c->d_pb, c->mask, c->rbgs_diag, b, xh, 0u, links);
         for (uint32_t k = 1; k < 2 * iterations; ++k)
-            rbgs_reverse_kernel<true, true><<<CB, kBlock, 0, c->stream>>>(g, c->d_pb, c->mask, c->rbgs_diag, b, xh, k & 1u);
-        rbgs_reverse_kernel<true, false><<<CB, kBlock, 0, c->stream>>>(g, c->d_pb, c->mask, c->rbgs_diag, b, xh, 0u);
+            rbgs_reverse_kernel<true, true><<<CB, kBlock, 0, c->stream>>>(g, c->d_pb, c->mask, c->rbgs_diag, b, xh, k & 1u, links);
+        rbgs_reverse_kernel<true, false><<<CB, kBlock, 0, c->stream>>>(g, c->d_pb, c->mask, c->rbgs_diag, b, xh, 0u, links);
         check_launch("rbgs_reverse_kernel");
     }
     ds_solve_info si{};
