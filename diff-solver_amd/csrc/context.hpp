@@ -351,6 +351,7 @@ struct ds_context {
     // pressure boundary (device) for the red-black Gauss-Seidel mode, and its zeroed copy
     const ds::SBound* d_pb = nullptr;
     const ds::SBound* d_pb_zero = nullptr;
+    const ds::SBound* d_rbgs_pb = nullptr;   // DS_PROJECTION_RBGS: both with the axes in the boxes' order (rbgs.hip)
     ds::SBound pb_zero{};
     uint8_t* rbgs_diag = nullptr;     // RBGS diagonal per cell, 0 = not updated (DS_PROJECTION_RBGS)
 

@@ -180,20 +180,14 @@ __device__ __forceinline__ float divide_small(float sum, float d) {
     return __builtin_amdgcn_div_fixupf(__fmaf_rn(__fmaf_rn(-d, q, sum), rd, q), d, sum);
 }
 
-// The axes of the boxes in terms of the grid's: those of one cell last. The cells lie in memory the same
-// way, so a grid of 1 x ny x nz is swept as ny x nz x 1 (the sum's order follows; colours are the same).
-struct BoxAxes {
-    int of[3];
-};
-
-// g: the grid with its axes in the boxes' order.
+// g, bp: the grid and its boundary with the axes in the boxes' order (box_axes).
 // Wide: the thread's two cells in one load; x is not periodic then and nx >= 2 (a pair that has one
 // cell outside reads the pair next to it).
 template <typename B, bool Wide>
 __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __restrict__ bp, const uint8_t* __restrict__ diag,
                                                         const float* __restrict__ rhs, const float* __restrict__ p_in,
                                                         float* __restrict__ p_out, uint32_t ntx, uint32_t nty, uint32_t boxes, int ex, int ey,
-                                                        int ez, int iterations, BoxAxes axes) {
+                                                        int ez, int iterations) {
     constexpr int H = B::H, K = B::K, RY = B::RY, RZ = B::RZ, P = B::P, Pad = K + 2;
     __shared__ float s[2][RZ * P + 2 * Pad];
     const uint32_t b = xcd_block();
@@ -203,8 +197,8 @@ __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __r
     const bool active = j < RY;
     const int x = bx * ex - H + 2 * k - odd, y = by * ey - H + j, z0 = bz * ez - H;
     float out[2]{}, out_y = 0.0f;
-    const int iy = sweep_coord(*bp, axes.of[1], y, g.ny, out_y);
-    const int ix[2]{sweep_coord(*bp, axes.of[0], x, g.nx, out[0]), sweep_coord(*bp, axes.of[0], x + 1, g.nx, out[1])};
+    const int iy = sweep_coord(*bp, 1, y, g.ny, out_y);
+    const int ix[2]{sweep_coord(*bp, 0, x, g.nx, out[0]), sweep_coord(*bp, 0, x + 1, g.nx, out[1])};
     bool in[2];
     uint32_t at[2], keep[2];   // keep: 0 where there is nothing to update, or a neighbour is not loaded
 #pragma unroll
@@ -220,8 +214,8 @@ __global__ __launch_bounds__(B::T) void rbgs_box_kernel(Geo g, const SBound* __r
     float p[2][RZ], r[2][RZ];
     uint32_t d[2][(RZ + 3) / 4]{};
     float out_z[2]{};
-    const bool wraps = sweep_coord(*bp, axes.of[2], -1, g.nz, out_z[0]) >= 0;
-    (void)sweep_coord(*bp, axes.of[2], g.nz, g.nz, out_z[1]);
+    const bool wraps = sweep_coord(*bp, 2, -1, g.nz, out_z[0]) >= 0;
+    (void)sweep_coord(*bp, 2, g.nz, g.nz, out_z[1]);
     int wz = wraps ? wrapi(z0, g.nz) : 0;
 #pragma unroll
     for (int z = 0; z < RZ; ++z) {
@@ -346,10 +340,25 @@ uint64_t box_points(const Geo& g) {
     return box_count<B>(g) * (uint64_t)(2 * B::P * B::RZ);
 }
 
-// One launch of rbgs_box_kernel; boxes of equal even extents that cover the grid (g, its axes in the
-// boxes' order).
+// The grid with the axes in the order of the boxes: those of one cell last. The cells lie in memory the
+// same way, so a grid of 1 x ny x nz is swept as ny x nz x 1 (the sum's order follows; colours are the
+// same). of: the grid's axes.
+Geo box_axes(const Geo& g, int (&of)[3]) {
+    Geo b = g;   // (the boxes use its cells and extents only)
+    int* const extents[3]{&b.nx, &b.ny, &b.nz};
+    for (int a = 0; a < 3; ++a) of[a] = a;
+    for (int pass = 0; pass < 2; ++pass)
+        for (int a = 0; a < 2; ++a)
+            if (*extents[a] == 1) {
+                std::swap(*extents[a], *extents[a + 1]);
+                std::swap(of[a], of[a + 1]);
+            }
+    return b;
+}
+
+// One launch of rbgs_box_kernel; boxes of equal even extents that cover the grid.
 template <typename B>
-void launch_boxes(ds_context* c, const Geo& g, const BoxAxes& axes, const SBound* bp, const float* b, const float* p_in, float* p_out,
+void launch_boxes(ds_context* c, const Geo& g, bool periodic_x, const SBound* bp, const float* b, const float* p_in, float* p_out,
                   uint32_t iterations) {
     auto split = [](int n, int most, uint32_t& count) {
         count = ((uint32_t)n + (uint32_t)most - 1) / (uint32_t)most;
@@ -359,9 +368,9 @@ void launch_boxes(ds_context* c, const Geo& g, const BoxAxes& axes, const SBound
     const int ex = split(g.nx, B::X, cx), ey = split(g.ny, B::Y, cy), ez = split(g.nz, B::Z, cz);
     const uint32_t boxes = cx * cy * cz, blocks = (boxes + 7u) & ~7u;
     auto launch = [&](auto kernel) {
-        kernel<<<blocks, B::T, 0, c->stream>>>(g, bp, c->rbgs_diag, b, p_in, p_out, cx, cy, boxes, ex, ey, ez, (int)iterations, axes);
+        kernel<<<blocks, B::T, 0, c->stream>>>(g, bp, c->rbgs_diag, b, p_in, p_out, cx, cy, boxes, ex, ey, ez, (int)iterations);
     };
-    if (!c->pressure_periodic[axes.of[0]] && g.nx >= 2) launch(rbgs_box_kernel<B, true>);
+    if (!periodic_x && g.nx >= 2) launch(rbgs_box_kernel<B, true>);
     else launch(rbgs_box_kernel<B, false>);
 }
 
@@ -375,6 +384,18 @@ uint32_t colour_blocks(const Geo& g) {
 void rbgs_prepare(ds_context* c) {
     rbgs_diag_kernel<<<xcd_blocks_for(c->geo.n), kBlock, 0, c->stream>>>(c->geo, c->d_pb, c->mask, (uint32_t)c->anchor, c->rbgs_diag);
     check_launch("rbgs_diag_kernel");
+    // the pressure boundary and its zeroed form for the boxes
+    int of[3];
+    (void)box_axes(c->geo, of);
+    SBound host[2]{c->pb, c->pb_zero};
+    for (int a = 0; a < 3; ++a)
+        for (int f = 0; f < 2; ++f) {
+            host[0].modes[2 * a + f] = host[1].modes[2 * a + f] = c->pb.modes[2 * of[a] + f];
+            host[0].values[2 * a + f] = c->pb.values[2 * of[a] + f];
+        }
+    SBound* const bounds = device_alloc<SBound>(c, 2);
+    DS_HIP(hipMemcpy(bounds, host, sizeof host, hipMemcpyHostToDevice));
+    c->d_rbgs_pb = bounds;
 }
 
 // Forward (kind 1) or tangent (kind 3): p = RBGS(rhs of u) from 0, into xh (xl = 0). Adjoint
@@ -401,21 +422,15 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
         // boxes wherever the colouring holds: the launches of one colour remain for a periodic axis of
         // odd extent, where a sweep reads a neighbour that it writes itself
         if (coloured && iterations > 0) {
-            Geo gb = g;   // (cells and extents only are used)
-            BoxAxes axes{{0, 1, 2}};
-            int* const extents[3]{&gb.nx, &gb.ny, &gb.nz};
-            for (int pass = 0; pass < 2; ++pass)
-                for (int a = 0; a < 2; ++a)
-                    if (*extents[a] == 1) {
-                        std::swap(*extents[a], *extents[a + 1]);
-                        std::swap(axes.of[a], axes.of[a + 1]);
-                    }
+            int of[3];
+            const Geo gb = box_axes(g, of);
+            const SBound* const boxes_bp = kind == kRhsTangent ? c->d_rbgs_pb + 1 : c->d_rbgs_pb;
             auto sweeps = [&]<typename B>() {
                 const uint32_t launches = (iterations + B::S - 1) / B::S;
                 float* from = launches % 2 ? xl : xh;   // both are zero; the last launch writes xh
                 for (uint32_t l = 0, done = 0; l < launches; ++l, done += B::S) {
                     float* to = from == xh ? xl : xh;
-                    launch_boxes<B>(c, gb, axes, bp, b, from, to, std::min<uint32_t>(B::S, iterations - done));
+                    launch_boxes<B>(c, gb, c->pressure_periodic[of[0]], boxes_bp, b, from, to, std::min<uint32_t>(B::S, iterations - done));
                     from = to;
                 }
             };
@@ -430,6 +445,8 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
             // 4 x 1024 x 1024 7056, 2484, 5168 (8 x 32 x 8: 4359); 6 x 1024 x 1024 7415, 4405, 7923. With axes of
             // one cell last: 1 x 1024 x 1024 6051 -> 1101, 1024 x 1 x 1024 2876 -> 1094. Along y Deep does:
             // 1024 x 2 x 1024 3046 against 3193.
+            // Along x only beyond one deep box for each CU: 4 x 256 x 256 (512 of them) 663, 522; 7 x 128 x 256 (256)
+            // 503, 515; 8 x 128 x 128 (128) 483, 492.
             using Flat = SweepBox<2, 32, 16, 2>;
             using Deep = SweepBox<2, 32, 16, 8>;
             using Thin2 = SweepBox<2, 2, 64, 8>;
@@ -437,6 +454,7 @@ ds_solve_info rbgs_solve_kind(ds_context* c, int kind, const float* const u[3], 
             const uint64_t deep = box_points<Deep>(gb);
             auto thin = [&]<typename B>() { return 3 * box_points<B>(gb) < 2 * deep; };
             if (box_count<Flat>(gb) <= 256u || thin.template operator()<Flat>()) sweeps.template operator()<Flat>();
+            else if (box_count<Deep>(gb) <= 256u) sweeps.template operator()<Deep>();
             else if (gb.nx <= 2) sweeps.template operator()<Thin2>();
             else if (thin.template operator()<Thin4>()) sweeps.template operator()<Thin4>();
             else sweeps.template operator()<Deep>();

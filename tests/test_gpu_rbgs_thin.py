@@ -1,8 +1,8 @@
 """The red-black sweeps on grids that are thin along one axis (csrc/rbgs.hip, rbgs_solve_kind: more than
-256 flat boxes and less than two thirds of the deep box's points), with remainders, a collider, a
-fixed-value face and a periodic axis along and across the thin one. Against the oracle's FP64 sweeps:
-FP32 sums of seven terms and a division, contracted by the sweeps, 1e-6 per iteration at most. And the
-cost of the sweeps, which with the deep box followed the box and not the cells.
+256 flat boxes, along x more than 256 deep ones, and less than two thirds of the deep boxes' points), with
+remainders, a collider, a fixed-value face and a periodic axis along and across the thin one. Against the
+oracle's FP64 sweeps: FP32 sums of seven terms and a division, contracted by the sweeps, 1e-6 per
+iteration at most. And the cost of the sweeps, which with the deep box followed the box and not the cells.
 """
 import numpy as np
 import pytest
@@ -12,7 +12,7 @@ from helpers import collider, random_fields, rel
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(1, 300, 250), (2, 131, 190), (5, 66, 230), (4, 130, 90), (129, 1, 140), (131, 2, 130), (700, 301, 1), (702, 300, 2)]
+SIZES = [(1, 300, 250), (2, 181, 200), (5, 130, 266), (4, 261, 150), (8, 100, 90), (129, 1, 140), (131, 2, 130), (700, 301, 1), (702, 300, 2)]
 
 
 def _scene(res, periodic_axis=None):
