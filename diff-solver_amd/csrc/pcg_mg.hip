@@ -1081,7 +1081,7 @@ uint64_t box_points(const MgLevel& L) {
 }
 
 // The box type of level l: by the number of cells, but a thin one on a large grid where it has less
-// than two thirds of the points (from 16 cells along x or 3 along z on it does not).
+// than two thirds of the points (from 11 cells along x or 3 along z on it does not).
 MgBox choose_box(const MgLevel& L, int l) {
     auto thin = [&]<typename N, typename X, typename Z>() {
         const uint64_t x = box_points<X>(L), z = box_points<Z>(L);
